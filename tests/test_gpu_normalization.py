@@ -89,3 +89,30 @@ def test_no_foreground_and_overlap_rejected():
     buf = torch.zeros(41, 50, 3, dtype=torch.uint8, device="cuda")
     with pytest.raises(NscError):
         gpu.normalization(buf[:40], MEAN_T, STD_T, out=buf[1:])
+
+
+@pytest.mark.parametrize("w,h,pad,shift", [(2047, 1, 0, 0), (2048, 3, 0, 0), (2049, 2, 5, 0), (255, 9, 0, 1), (4100, 2, 4, 2),
+                                           (3, 700, 0, 3)])
+def test_chunk_edges_and_alignments(w, h, pad, shift):
+    """Work items of 2048 pixels and pieces of 256: rows that end inside, at and past them, as one long
+    row (pad 0) or row by row, from a base `shift` bytes past an aligned address."""
+    from nscale_amd import gpu
+    from nscale_amd.synth import synth_he
+    from tests._lib import o_normalize
+    bgr = synth_he(h, w, 11)
+    bgr[:, 0] = (60, 40, 20)  # dark pixels on every edge
+    bgr[:, -1] = (120, 60, 130)
+    ld = 3 * w + pad
+    flat = torch.zeros(h * ld + shift, dtype=torch.uint8, device="cuda")
+    view = flat[shift:].as_strided((h, w, 3), (ld, 3, 1))
+    view.copy_(torch.from_numpy(bgr).cuda())
+    outf = torch.full((h * ld + shift,), 7, dtype=torch.uint8, device="cuda")
+    out = outf[shift:].as_strided((h, w, 3), (ld, 3, 1))
+    print("normalization", w, h, pad, shift, flush=True)
+    gpu.normalization(view, MEAN_T, STD_T, out=out)
+    torch.cuda.synchronize()
+    _close(out.cpu().numpy(), o_normalize(bgr, MEAN_T, STD_T))
+    # nothing outside the image is written
+    rest = torch.ones_like(outf, dtype=torch.bool)
+    rest[shift:].as_strided((h, w, 3), (ld, 3, 1)).fill_(False)
+    assert bool((outf[rest] == 7).all())
