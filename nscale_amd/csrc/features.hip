@@ -11,7 +11,7 @@
 // gradient is taken at the nucleus's own pixels.  Then one wave each evaluates the intensity and the
 // gradient statistics from the histograms, four bins a lane.
 // A launch is bound by the latency of a workgroup's few dependent steps: 2601 nuclei of a 2048^2
-// tile: FEAT_US (210 us with a gradient plane, the histograms in memory and one thread per nucleus
+// tile: 28 us (210 us with a gradient plane, the histograms in memory and one thread per nucleus
 // running over 2 x 256 bins, which alone took 177 us).
 #include <cfloat>
 #include <cmath>
