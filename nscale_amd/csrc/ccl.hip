@@ -7,14 +7,23 @@
 //
 // Labelling is union-find with the smallest raster index as root (the reference's merge links
 // the larger root under the smaller, ConnComponents.cpp:34-43, so its labels are also the
-// smallest index of each component):
-//   1. ccl_local: 64x64 tiles in LDS, pixels start at the first pixel of their row run, runs
-//      of adjacent rows unite with atomicMin on local indices (local raster order = global
-//      raster order inside a tile), then each pixel stores the global index of its tile-local
-//      root;
-//   2. ccl_seams: pixels on tile seams unite with their cross-tile neighbours in global memory
-//      (atomicMin union, retry while the target stopped being a root);
-//   3. ccl_flatten: every pixel follows its chain to the root (a read-only walk).
+// smallest index of each component).  It works on runs, not pixels: a run is a maximal stretch of
+// left-joined pixels within one row of a 64 x 64 tile, and a row of a tile is two 64-bit words, the
+// foreground F and the run starts S.
+//   1. ccl_tile: one wave per tile, lane = row.  Bit operations on F and S give the joins to unite
+//      (a run's own joins need no union), the runs, numbered in raster order, unite in LDS with
+//      atomicMin on their numbers, and the tile leaves behind its F and S words, the number of the
+//      tile-local root of every run (two bytes), the places of the roots along its four edges, and for
+//      each tile-local root its entry in the forest P (the root's own global index) with what the
+//      caller needs of it: pixel count or flag;
+//   2. ccl_seams: two waves per tile unite the runs that meet across its left and its top edge, in P;
+//   3. ccl_roots (selections): each tile-local root finds its final root and hands its count or flag
+//      over;
+//   4. ccl_select writes the selected pixels, ccl_label the labels: both expand the words again.
+// P is indexed by pixel but only the entries of tile-local roots exist; no other per-pixel label is
+// stored on the way.  Bytes moved per pixel: about 0.4 for the words and roots, the image in and the
+// result out.  Labelling per pixel instead (labels in LDS, stored, seams from the stored labels, a
+// flattening pass, a consumer pass) moved 17 and was bound by instruction issue in its tile pass.
 // Pixel classes: FG_NEQ  -> foreground = value != key; neighbours join when both foreground
 //                FG_EQ   -> foreground = value != 0; neighbours join when values are equal
 //                FG_FEQ  -> foreground = cls != 0; neighbours join when float values are equal
@@ -27,7 +36,7 @@
 namespace nsc {
 namespace {
 
-constexpr int CT_W = 64, CT_H = 64, CT_N = CT_W * CT_H;
+constexpr int CT = 64;  // tile side: lanes of a wave, bits of a word
 enum { FG_NEQ = 0, FG_EQ = 1, FG_FEQ = 2 };
 
 struct Px {
@@ -35,7 +44,6 @@ struct Px {
     const float* fv;
     uint8_t key;
 };
-
 
 // find with intermediate pointer jumping (each visited node is re-pointed to its grandparent).
 // Parents are always smaller than children, and a non-root never becomes a root again, so
@@ -45,366 +53,808 @@ struct Px {
 // relaxed atomic accesses: other threads update the forest concurrently, so no access may be
 // kept in a register by the compiler
 __device__ __forceinline__ int ld_wg(const int* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-__device__ __forceinline__ void st_wg(int* a, int v) { __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
-__device__ __forceinline__ int lfind(int* L, int x) {
-    int p = ld_wg(&L[x]);
-    if (p == x) return x;
-    int q = ld_wg(&L[p]);
-    while (p != q) {
-        st_wg(&L[x], q);
-        x = p;
-        p = q;
-        q = ld_wg(&L[p]);
-    }
-    return p;
+// A run's node in LDS: its number's parent in the low half, the place of its first pixel in the tile
+// (row * 64 + column) in the high one.
+__device__ __forceinline__ int parent_of(const uint32_t* N, int x) {
+    return (int)(__hip_atomic_load(&N[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 0xFFFFu);
+}
+__device__ __forceinline__ uint32_t node_of(const uint32_t* N, int x) {
+    return __hip_atomic_load(&N[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-__device__ void lunite(int* L, int a, int b) {
+// Unites the sets of a and b.  Both walk to their roots together (each step's two reads in one round
+// trip), re-pointing what they pass to its grandparent, and stop as soon as they meet.
+__device__ __forceinline__ void lunite(uint32_t* N, int a, int b) {
     while (true) {
-        a = lfind(L, a);
-        b = lfind(L, b);
+        uint32_t na = node_of(N, a), nb = node_of(N, b);
+        int pa = (int)(na & 0xFFFFu), pb = (int)(nb & 0xFFFFu);
+        while (pa != a || pb != b) {
+            if (pa == pb) return;
+            const uint32_t qa = node_of(N, pa), qb = node_of(N, pb);
+            const int ga = (int)(qa & 0xFFFFu), gb = (int)(qb & 0xFFFFu);
+            if (ga != pa) __hip_atomic_store(&N[a], (na & 0xFFFF0000u) | ga, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (gb != pb) __hip_atomic_store(&N[b], (nb & 0xFFFF0000u) | gb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            a = pa;
+            na = qa;
+            pa = ga;
+            b = pb;
+            nb = qb;
+            pb = gb;
+        }
         if (a == b) return;
-        if (a > b) { int t = a; a = b; b = t; }
-        int old = atomicMin(&L[b], a);
+        if (a > b) {
+            const int t = a;
+            a = b;
+            b = t;
+            nb = na;
+        }
+        // the high halves are equal, so the minimum is that of the parents
+        const int old = (int)(atomicMin(&N[b], (nb & 0xFFFF0000u) | (uint32_t)a) & 0xFFFFu);
         if (old == b) return;
         b = old;
     }
+}
+
+// Orders LDS accesses between the lanes of one wave (they execute in program order).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // relaxed device-scope accesses: unions from every workgroup of the launch update the forest
 __device__ __forceinline__ int ld_rel(const int* a) { return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void st_rel(int* a, int v) { __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-__device__ __forceinline__ int gfind(int32_t* L, int x) {
-    int p = ld_rel(&L[x]);
-    if (p == x) return x;
-    int q = ld_rel(&L[p]);
-    while (p != q) {
-        st_rel(&L[x], q);
-        x = p;
-        p = q;
-        q = ld_rel(&L[p]);
-    }
-    return p;
-}
-
-// Union in global memory of two ancestors a, b of the pixels to join (the labels a seam pixel has
-// already read, usually tile-local roots that are still roots): both root checks are issued before
-// either is used, and a find runs only for an ancestor that stopped being a root.
-__device__ void gunite(int32_t* L, int a, int b) {
-    const int pa = ld_rel(&L[a]), pb = ld_rel(&L[b]);
-    if (pa != a) a = gfind(L, a);
-    if (pb != b) b = gfind(L, b);
+// The same union in global memory, of two tile-local roots.  What bounds the seams of a component that
+// spans the image is the chain of dependent round trips to the forest (about a microsecond each, past
+// the XCDs' own L2s), so both walks advance together and end where they meet.
+__device__ __forceinline__ void gunite(int32_t* L, int a, int b) {
+    int pa = ld_rel(&L[a]), pb = ld_rel(&L[b]);
     while (true) {
+        while (pa != a || pb != b) {
+            if (pa == pb) return;
+            const int ga = ld_rel(&L[pa]), gb = ld_rel(&L[pb]);
+            if (ga != pa) st_rel(&L[a], ga);
+            if (gb != pb) st_rel(&L[b], gb);
+            a = pa;
+            pa = ga;
+            b = pb;
+            pb = gb;
+        }
         if (a == b) return;
-        if (a > b) { int t = a; a = b; b = t; }
+        if (a > b) { const int t = a; a = b; b = t; }
         const int old = atomicMin(&L[b], a);
         if (old == b) return;
         b = old;
-        a = gfind(L, a);
-        b = gfind(L, b);
+        pa = ld_rel(&L[a]);
+        pb = ld_rel(&L[b]);
     }
 }
 
-// One 64 x 64 tile per workgroup; a row of the tile is one wave (lane = column), and thread t
-// handles rows t / 64, t / 64 + 4, ... .  Horizontal joins need no union: each pixel starts out
-// pointing at the first pixel of its run of left-joined pixels (from a ballot of the row).  A
-// vertical or diagonal join is united only where no join further left already connects the
-// same two runs:
-//   up (k, k-64):        skipped when k joins k-1, k-1 joins up, and k-64 joins k-65;
-//   up-left (k, k-65):   skipped when k joins up and k-64 joins k-65, or k joins k-1 and k-1
-//                        joins up;
-//   up-right (k, k-63):  skipped when k joins up and k-63 joins k-64, or k+1 joins k and k+1
-//                        joins up.
+// ---- the words of a tile -------------------------------------------------------------------
+struct RowWords {
+    uint64_t S, F;  // run starts, foreground
+};
+
+// What a labelling leaves per tile: the words of its 64 rows, the number of runs before each row, the
+// number of the tile-local root of every run, the places of the roots along the four edges (kNoRoot
+// for background), and, for the equal-value modes, the values of its first and last column (the seams
+// compare them).
+constexpr uint16_t kNoRoot = 0xFFFF;
+enum { E_LEFT = 0, E_RIGHT = 1, E_TOP = 2, E_BOTTOM = 3 };
+struct CclBufs {
+    RowWords* rows;
+    uint16_t *off, *roots;
+    uint16_t* edge_roots;  // [tile][4][64]
+    void* edge;            // uint8_t or float, [tile][2][64]
+    int cap;               // run slots of a tile
+};
+
+__device__ __forceinline__ int popc64(uint64_t v) { return (int)__popcll(v); }
+__device__ __forceinline__ uint64_t upto(int x) { return (2ull << x) - 1ull; }  // bits 0..x (x <= 63: 2 << 63 wraps to 0)
+// number, within its row, of the run that holds the foreground pixel at column x
+__device__ __forceinline__ int run_index(uint64_t S, int x) { return popc64(S & upto(x)) - 1; }
+// first column after the run that starts at a
+__device__ __forceinline__ int run_end(uint64_t S, uint64_t F, int a) {
+    const uint64_t stop = (S | ~F) & ~upto(a);
+    return stop ? __ffsll((long long)stop) - 1 : 64;
+}
+__device__ __forceinline__ uint64_t run_bits(int a, int end) { return (end < 64 ? 1ull << end : 0ull) - (1ull << a); }
+
+__device__ __forceinline__ uint64_t shfl_up64(uint64_t v) {  // from lane - 1; lane 0 receives 0
+    return (uint64_t)(uint32_t)dpp_from_left(0, (int)(uint32_t)v) |
+           (uint64_t)(uint32_t)dpp_from_left(0, (int)(uint32_t)(v >> 32)) << 32;
+}
+
+// 0x80 in every nonzero byte
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t x) { return (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u; }
+// The flags of eight bytes (as 0x80) as one byte: byte products with the bits' weights, summed
+__device__ __forceinline__ uint32_t gather_bits(uint32_t t0, uint32_t t1) {
+    return __builtin_amdgcn_udot4(t1, 0x80402010u, __builtin_amdgcn_udot4(t0, 0x08040201u, 0u, false), false) >> 7;
+}
+// four bits as four bytes of 0 / 255
+__device__ __forceinline__ uint32_t spread_bits(uint32_t b) { return ((b * 0x00204081u) & 0x01010101u) * 255u; }
+
+// 16 bytes of a row from column x of `cols` (any alignment; whole when `full`, else the bytes past the
+// row repeat its last one)
+__device__ __forceinline__ uint4 load16(const uint8_t* row, int x, int cols, bool full) {
+    uint4 v;
+    if (full) {
+        __builtin_memcpy(&v, row + x, 16);
+    } else {
+        uint32_t wd[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 16; ++j) wd[j >> 2] |= (uint32_t)row[min(x + j, cols - 1)] << (8 * (j & 3));
+        v = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+    }
+    return v;
+}
+
+// Bit x of lane y's result: pixel (x0 + x, y0 + y) lies in the image and differs from key.  A lane
+// loads four 16-byte pieces (a row is four lanes), turns each into 16 bits, and the rows come
+// together through LDS.
+__device__ __forceinline__ uint64_t tile_bits(const uint8_t* __restrict__ img, int w, int h, int x0, int y0, uint32_t key,
+                                              uint16_t* stage) {
+    const int lane = threadIdx.x & 63, r = lane >> 2, x = 16 * (lane & 3);
+    const int cols = min(CT, w - x0);
+    const bool full = cols == CT;
+    uint4 v[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        v[g] = load16(img + (size_t)min(y0 + 16 * g + r, h - 1) * w + x0, x, cols, full);
+    const uint32_t k4 = key * 0x01010101u;
+    const uint32_t inside = full ? 0xFFFFu : (x >= cols ? 0u : (uint32_t)((2u << min(cols - 1 - x, 15)) - 1u));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const uint32_t bits = gather_bits(nonzero_bytes(v[g].x ^ k4), nonzero_bytes(v[g].y ^ k4)) |
+                              gather_bits(nonzero_bytes(v[g].z ^ k4), nonzero_bytes(v[g].w ^ k4)) << 8;
+        stage[4 * (16 * g + r) + (lane & 3)] = (uint16_t)(y0 + 16 * g + r < h ? bits & inside : 0u);
+    }
+    wave_order();
+    const uint64_t m = *reinterpret_cast<const uint64_t*>(stage + 4 * lane);
+    wave_order();
+    return m;
+}
+
+// The joins of a row to unite with the row above.  A vertical or diagonal join is united only where no
+// join further left already connects the same two runs (F, jl: this row's foreground and left joins;
+// ju, jul, jur: joins with the pixel above, above left, above right; jlu: left joins of the row above):
+//   up:        skipped when the pixel joins its left one, that one joins up, and the pixels above join;
+//   up-left:   skipped when the pixel joins up and the pixels above join, or it joins its left one and
+//              that one joins up;
+//   up-right:  skipped when the pixel joins up and the pixels above join, or the pixel to its right
+//              joins it and joins up.
 // Every skipped join is implied by a path through joins that are united or skipped only by a rule
 // that looks further left, so the components are those of all joins.
-template <int MODE, int CONN>
-__global__ __launch_bounds__(256) void ccl_local(Px P, int32_t* __restrict__ L, int w, int h, int tiles_x,
-                                                 uint8_t* __restrict__ clear8) {
-    constexpr int PER = CT_N / 256;  // rows per thread
-    using V = typename std::conditional<MODE == FG_FEQ, float, uint32_t>::type;
-    __shared__ int ll[CT_N];
-    // pixel values the joins compare (equal-value modes)
-    __shared__ typename std::conditional<MODE == FG_FEQ, float, uint8_t>::type lv[MODE == FG_NEQ ? 1 : CT_N];
-    __shared__ unsigned long long jrow[CT_H];  // bit x of row y: pixel x joins pixel x - 1
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-    const int x0 = tx * CT_W, y0 = ty * CT_H;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // every load first, from clamped (always valid) addresses: a load per iteration with its use in
-    // the same iteration compiles to one memory round trip after another
-    uint8_t c[PER];
-    float f[PER];
-    const auto gimg = as_global(P.img);
-    const size_t gxc = (size_t)clampi(x0 + lane, 0, w - 1);
+struct JoinWords {
+    uint64_t up, ul, ur;
+};
+template <int CONN>
+__device__ __forceinline__ JoinWords joins_to_unite(uint64_t jl, uint64_t ju, uint64_t jul, uint64_t jur, uint64_t jlu) {
+    JoinWords J;
+    J.up = ju & ~(jl & (ju << 1) & jlu);
+    J.ul = CONN == 8 ? jul & ~((ju & jlu) | (jl & (ju << 1))) : 0ull;
+    J.ur = CONN == 8 ? jur & ~((ju & (jlu >> 1)) | ((jl >> 1) & (ju >> 1))) : 0ull;
+    return J;
+}
+
+// The words and joins of a tile where equal byte values join: the tile's bytes come to LDS, each lane
+// takes its row as 16 dwords (and the row above from the lane before it), and every comparison with a
+// neighbour is byte arithmetic on four pixels at a time.  (One ballot per row and comparison took 51 us
+// for a 4096 x 3071 mask, this EQ_US.)
+constexpr int kBytePitch = 17;  // dwords per staged row: the lanes' rows start in different banks
+template <int CONN>
+__device__ __forceinline__ void tile_words_eq(const uint8_t* __restrict__ img, int w, int h, int x0, int y0, RowWords& R,
+                                              JoinWords& J, uint8_t* edge, uint32_t* stage) {
+    const int lane = threadIdx.x & 63, r = lane >> 2, x = 16 * (lane & 3);
+    const int cols = min(CT, w - x0);
+    const bool full = cols == CT;
+    uint4 v[4];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const size_t i = (size_t)clampi(y0 + wv + 4 * j, 0, h - 1) * w + gxc;
-        c[j] = gimg[i];
-        if (MODE == FG_FEQ) f[j] = as_global(P.fv)[i];
+    for (int g = 0; g < 4; ++g) v[g] = load16(img + (size_t)min(y0 + 16 * g + r, h - 1) * w + x0, x, cols, full);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        uint32_t* q = stage + (16 * g + r) * kBytePitch + 4 * (lane & 3);
+        q[0] = v[g].x;
+        q[1] = v[g].y;
+        q[2] = v[g].z;
+        q[3] = v[g].w;
     }
-    auto val = [&](int j) -> V {
-        if constexpr (MODE == FG_FEQ) return f[j];
-        else return (V)c[j];
-    };
-    auto left_of = [&](V v) -> V { return from_left((V)0, v); };
-    unsigned fgbits = 0;  // bit j: row wv + 4 j of this column is foreground
+    wave_order();
+    uint32_t c[16], u[16];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int k = threadIdx.x + 256 * j, ly = wv + 4 * j;
-        const bool in = x0 + lane < w && y0 + ly < h;
-        const bool fg = in && (MODE == FG_NEQ ? c[j] != P.key : c[j] != 0);
-        fgbits |= (fg ? 1u : 0u) << j;
-        if (MODE == FG_EQ) lv[k] = c[j];
-        if (MODE == FG_FEQ) lv[k] = f[j];
-        // the left neighbour is lane - 1 of the same wave (lane 0 receives 0: no left join).  Every
-        // cross-lane read runs on all lanes (none of them under a condition): a lane that is
-        // switched off supplies nothing to its neighbour.
-        const bool fg_left = from_left(0, fg ? 1 : 0) != 0;
-        const V v_left = left_of(val(j));
-        bool jl = fg && fg_left;
-        if (MODE != FG_NEQ) jl = jl && val(j) == v_left;
-        const unsigned long long m = __ballot(jl);
-        // run start: the last position <= lane without a left join (bit 0 is never a join)
-        const unsigned long long upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-        const int start = 63 - __clzll((long long)(~m & upto));
-        ll[k] = fg ? ly * CT_W + start : -1;
-        if (lane == 0) jrow[ly] = m;
-    }
-    __syncthreads();
+    for (int j = 0; j < 16; ++j) c[j] = stage[lane * kBytePitch + j];
+    wave_order();
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int k = threadIdx.x + 256 * j, ly = wv + 4 * j;
-        if (ly == 0) continue;  // uniform over the wave
-        const bool fg = (fgbits >> j) & 1u;
-        const bool up = ll[k - CT_W] >= 0;
-        V vu = 0;
-        if (MODE != FG_NEQ) vu = (V)lv[k - CT_W];
-        const unsigned long long jr = jrow[ly], ju_row = jrow[ly - 1];
-        const bool jl = (jr >> lane) & 1ull;
-        const bool jl_up = (ju_row >> lane) & 1ull;  // k - 64 joins k - 65
-        bool ju = fg && up;
-        if (MODE != FG_NEQ) ju = ju && val(j) == vu;
-        const int ju_i = ju ? 1 : 0, up_i = up ? 1 : 0;
-        const bool ju_left = from_left(0, ju_i) != 0;
-        const bool do_up = ju && !(jl && ju_left && jl_up);
-        bool do_ul = false, do_ur = false;
+    for (int j = 0; j < 16; ++j) u[j] = (uint32_t)dpp_from_left(0, (int)c[j]);
+    uint64_t F = 0, nl = 0, nu = 0, nul = 0, nur = 0;  // foreground; pixels that differ from that neighbour
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) {
+        const int sh = 4 * j;
+        // the pixels' left, upper left and upper right neighbours: the words shifted by a byte
+        const uint32_t l0 = c[j] << 8 | (j ? c[j ? j - 1 : 0] >> 24 : 0u), l1 = c[j + 1] << 8 | c[j] >> 24;
+        F |= (uint64_t)gather_bits(nonzero_bytes(c[j]), nonzero_bytes(c[j + 1])) << sh;
+        nl |= (uint64_t)gather_bits(nonzero_bytes(c[j] ^ l0), nonzero_bytes(c[j + 1] ^ l1)) << sh;
+        nu |= (uint64_t)gather_bits(nonzero_bytes(c[j] ^ u[j]), nonzero_bytes(c[j + 1] ^ u[j + 1])) << sh;
         if (CONN == 8) {
-            const bool up_left = from_left(0, up_i) != 0, up_right = from_right(0, up_i) != 0;
-            const bool ju_right = from_right(0, ju_i) != 0;
-            const V vul = left_of(vu), vur = from_right((V)0, vu);
-            bool jul = fg && up_left, jur = fg && up_right;
-            if (MODE != FG_NEQ) {
-                jul = jul && val(j) == vul;
-                jur = jur && val(j) == vur;
-            }
-            const bool jl_upright = lane < 63 && ((ju_row >> (lane + 1)) & 1ull);  // k - 63 joins k - 64
-            const bool jl_right = lane < 63 && ((jr >> (lane + 1)) & 1ull);        // k + 1 joins k
-            do_ul = jul && !((ju && jl_up) || (jl && ju_left));
-            do_ur = jur && !((ju && jl_upright) || (jl_right && ju_right));
+            const uint32_t a0 = u[j] << 8 | (j ? u[j ? j - 1 : 0] >> 24 : 0u), a1 = u[j + 1] << 8 | u[j] >> 24;
+            const uint32_t b0 = u[j] >> 8 | u[j + 1] << 24, b1 = u[j + 1] >> 8 | (j < 14 ? u[j < 14 ? j + 2 : 15] << 24 : 0u);
+            nul |= (uint64_t)gather_bits(nonzero_bytes(c[j] ^ a0), nonzero_bytes(c[j + 1] ^ a1)) << sh;
+            nur |= (uint64_t)gather_bits(nonzero_bytes(c[j] ^ b0), nonzero_bytes(c[j + 1] ^ b1)) << sh;
         }
-        if (do_up) lunite(ll, k, k - CT_W);
-        if (do_ul) lunite(ll, k, k - CT_W - 1);
-        if (do_ur) lunite(ll, k, k - CT_W + 1);
+    }
+    if (!full) F &= (1ull << cols) - 1ull;
+    if (y0 + lane >= h) F = 0;
+    edge[lane] = (uint8_t)c[0];
+    edge[CT + lane] = (uint8_t)(c[15] >> 24);
+    const uint64_t Fu = shfl_up64(F);
+    const uint64_t jl = F & (F << 1) & ~nl;
+    R = RowWords{F & ~jl, F};
+    J = joins_to_unite<CONN>(jl, F & Fu & ~nu, F & (Fu << 1) & ~nul, F & (Fu >> 1) & ~nur, shfl_up64(jl));
+}
+
+// The same where equal floats join (NaN joins nothing): four waves of 16 rows each, lane = column; each
+// comparison of a row is one ballot, and row y's words go through LDS to lane y of the first wave.
+constexpr int kEqWords = 5;
+template <int CONN>
+__device__ __forceinline__ void tile_words_feq(const Px& P, int w, int h, int x0, int y0, RowWords& R, JoinWords& J,
+                                               float* edge, uint64_t (*words)[kEqWords]) {
+    const int lane = threadIdx.x & 63, r0 = 16 * (threadIdx.x >> 6);
+    const size_t gxc = (size_t)min(x0 + lane, w - 1);
+    const bool in_x = x0 + lane < w;
+    uint8_t c[17];
+    float f[17];
+    // every load first, from clamped (always valid) addresses; entry 0 is the row above the wave's
+#pragma unroll
+    for (int j = 0; j < 17; ++j) {
+        const size_t i = (size_t)min(max(y0 + r0 + j - 1, 0), h - 1) * w + gxc;
+        c[j] = as_global(P.img)[i];
+        f[j] = as_global(P.fv)[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const bool above = r0 > 0;  // row 0's neighbours above belong to another tile
+    uint64_t pF = __ballot(above && in_x && y0 + r0 - 1 < h && c[0] != 0);
+    float pl = from_left(0.0f, f[0]);
+    uint64_t pjl = __ballot(f[0] == pl) & pF & (pF << 1);
+#pragma unroll
+    for (int j = 1; j < 17; ++j) {
+        const int y = r0 + j - 1;
+        const float v = f[j], l = from_left(0.0f, v);
+        const uint64_t F = __ballot(in_x && y0 + y < h && c[j] != 0);
+        const uint64_t jl = __ballot(v == l) & F & (F << 1);
+        const uint64_t ju = __ballot(v == f[j - 1]) & F & pF;
+        uint64_t jul = 0, jur = 0;
+        if (CONN == 8) {
+            jul = __ballot(v == pl) & F & (pF << 1);
+            jur = __ballot(v == from_right(0.0f, f[j - 1])) & F & (pF >> 1);
+        }
+        const JoinWords q = joins_to_unite<CONN>(jl, ju, jul, jur, pjl);
+        const uint64_t word[kEqWords] = {F & ~jl, F, q.up, q.ul, q.ur};
+        if (lane < kEqWords) {
+            uint64_t v5 = word[0];
+#pragma unroll
+            for (int k = 1; k < kEqWords; ++k) v5 = lane == k ? word[k] : v5;
+            words[y][lane] = v5;
+        }
+        if (lane == 0) edge[y] = v;
+        if (lane == 63) edge[CT + y] = v;
+        pl = l;
+        pF = F;
+        pjl = jl;
     }
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int k = threadIdx.x + 256 * j, ly = wv + 4 * j;
-        const int gx = x0 + lane, gy = y0 + ly;
-        int r = ll[k];
-        int32_t out = -1;
-        if (r >= 0) {
-            r = lfind(ll, k);
-            out = (int32_t)((size_t)(y0 + r / CT_W) * w + (x0 + r % CT_W));
-            // clear8: entry cleared at every tile-local root (every final root is one), so a per-root
-            // table filled while flattening needs no image-sized fill
-            if (clear8 && r == k) clear8[out] = 0;
-        }
-        if (gx < w && gy < h) L[(size_t)gy * w + gx] = out;
-    }
+    R = RowWords{words[lane][0], words[lane][1]};
+    J = JoinWords{words[lane][2], words[lane][3], words[lane][4]};
 }
 
-// unions across tile seams: every pixel in a tile's first row, first column or last column
-// joins its "backward" neighbours (left, up, up-left, up-right) that lie in another tile.  Along a
-// seam, consecutive pixels usually link the same two tile-local components: a pixel skips a union
-// when the previous pixel of the seam joins, in the same direction, two pixels whose labels are the
-// ones it sees (the labels read are ancestors of those pixels, so the previous pixel's union joins
-// the same two sets).
-template <int MODE, int CONN>
-__global__ __launch_bounds__(256) void ccl_seams(Px P, int32_t* L, int w, int h, int tiles_x, int ntiles) {
-    constexpr int ND = CONN == 8 ? 4 : 2;
-    // with 4-connectivity a last-column pixel has no backward neighbour in another tile (left and
-    // up are in its own tile; the tile's top row covers the corner), so only 8 needs that column
-    const int per_tile = CONN == 8 ? CT_W + 2 * CT_H : CT_W + CT_H;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= ntiles * per_tile) return;
-    const int t = gid / per_tile, e = gid % per_tile;
-    const int tx = t % tiles_x, ty = t / tiles_x;
-    int lx, ly, sx, sy;  // position on the seam and the step to the previous seam pixel
-    if (e < CT_W) { lx = e; ly = 0; sx = -1; sy = 0; }
-    else if (e < CT_W + CT_H) { lx = 0; ly = e - CT_W; sx = 0; sy = -1; }
-    else { lx = CT_W - 1; ly = e - CT_W - CT_H; sx = 0; sy = -1; }
-    const bool has_prev = (sx ? lx : ly) > 0;
-    const int x = tx * CT_W + lx, y = ty * CT_H + ly;
-    if (x >= w || y >= h) return;
-    const int px = x + sx, py = y + sy;
-    const int dxs[4] = {-1, 0, -1, 1}, dys[4] = {0, -1, -1, -1};
-    // every label and value this pixel needs, loaded together from clamped (always valid)
-    // addresses; the checks below discard what lies outside the image or inside the tile
-    auto at = [&](int qx, int qy) { return (size_t)clampi(qy, 0, h - 1) * w + clampi(qx, 0, w - 1); };
-    const size_t i = (size_t)y * w + x, ip = at(px, py);
-    int lj[ND], ljp[ND];
-    size_t j[ND], jp[ND];
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-        j[d] = at(x + dxs[d], y + dys[d]);
-        jp[d] = at(px + dxs[d], py + dys[d]);
-    }
-    const int li = ld_wg(&L[i]), lp = ld_wg(&L[ip]);
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-        lj[d] = ld_wg(&L[j[d]]);
-        ljp[d] = ld_wg(&L[jp[d]]);
-    }
-    // the values the equal-value joins compare, loaded with the labels (inside the checks below
-    // each would be one more dependent round trip)
-    using V = typename std::conditional<MODE == FG_FEQ, float, uint8_t>::type;
-    V vi = 0, vp = 0, vj[ND], vjp[ND];
-    if (MODE != FG_NEQ) {
-        auto val = [&](size_t q) -> V {
-            if constexpr (MODE == FG_FEQ) return P.fv[q];
-            else return P.img[q];
-        };
-        vi = val(i);
-        vp = val(ip);
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-            vj[d] = val(j[d]);
-            vjp[d] = val(jp[d]);
-        }
-    }
-    if (li < 0) return;
-    auto cross = [&](int qx, int qy) { return (qx / CT_W != tx) || (qy / CT_H != ty); };
-    auto valid = [&](int qx, int qy) { return qx >= 0 && qy >= 0 && qx < w && qy < h && cross(qx, qy); };
-    const int lprev = has_prev ? lp : -1;
-    // Along a seam, consecutive pixels usually link the same two tile-local components: a pixel
-    // skips its union when the previous seam pixel joins, in the same direction, two pixels whose
-    // labels are the ones it sees (labels read are ancestors of those pixels, so the previous
-    // pixel's union joins the same two sets).
-#pragma unroll
-    for (int d = 0; d < ND; ++d) {
-        const int qx = x + dxs[d], qy = y + dys[d];
-        if (!valid(qx, qy) || lj[d] < 0 || (MODE != FG_NEQ && !(vi == vj[d]))) continue;
-        if (has_prev && lprev == li) {
-            const int rx = px + dxs[d], ry = py + dys[d];
-            if (valid(rx, ry) && ljp[d] == lj[d] && (MODE == FG_NEQ || vp == vjp[d])) continue;  // same union
-        }
-        gunite(L, li, lj[d]);  // labels are ancestors of their pixels
-    }
-}
+enum { SRC_NONE = 0, SRC_BYTES = 1, SRC_BORDER = 2 };
 
-// Four pixels per thread, i, i + S, i + 2S, i + 3S (S = threads in the grid): each of the four
-// loads is coalesced over the wave, and the four labels and the four first hops are each issued
-// together instead of one dependent round trip after another.
-// `zero_at_roots` / `zero8_at_roots` (optional): entry i cleared for every root i, so a per-root
-// table (areas, selection flags) needs no image-sized fill before it is filled in.
-// `flag_set` (optional): flag_set[root] = 1 for every component holding a pixel with
-// flag_src[i] != 0 (flag_src null: a pixel on the border of the fw x fh image); the entries must
-// have been cleared at the roots before (ccl_local's clear8)
-__global__ void ccl_flatten(int32_t* L, size_t n, int32_t bgval, int32_t* __restrict__ zero_at_roots,
-                            uint8_t* __restrict__ zero8_at_roots, const uint8_t* __restrict__ flag_src,
-                            uint8_t* flag_set, int fw, int fh) {
-    const size_t S = (size_t)gridDim.x * blockDim.x;
-    for (size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += 4 * S) {
-        int p[4], q[4];
-        bool sv[4] = {false, false, false, false};
+constexpr int ccl_cap(int mode) { return mode == FG_NEQ ? CT * CT / 2 : CT * CT; }  // most runs of a tile
+constexpr int ccl_tile_threads(int mode) { return mode == FG_FEQ ? 256 : 64; }
+
+// One tile per workgroup (its first wave, once the words are there).  Per tile-local root: P = its own
+// index; area (optional) = the pixels of its tile-local component; flag (optional) = whether that
+// holds a source pixel: a nonzero pixel of src (SRC_BYTES) or a pixel on the image border
+// (SRC_BORDER).  *zero (optional) is cleared for the passes that follow.
+template <int MODE, int CONN, int SRC>
+__global__ __launch_bounds__(ccl_tile_threads(MODE)) void ccl_tile(Px P, CclBufs B, int32_t* __restrict__ forest, int w, int h,
+                                                                   int tiles_x, int32_t* __restrict__ area,
+                                                                   uint8_t* __restrict__ flag,
+                                                                   const uint8_t* __restrict__ src, int* __restrict__ zero) {
+    // the runs' nodes (8 KB of LDS for binary masks: every tile of a 4096^2 image is resident at once)
+    __shared__ uint32_t node[ccl_cap(MODE)];
+    __shared__ union {
+        uint16_t bits[4 * CT];
+        uint32_t bytes[MODE == FG_EQ ? CT * kBytePitch : 1];
+        uint64_t words[MODE == FG_FEQ ? CT : 1][kEqWords];
+    } stage;
+    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
+    const int x0 = tx * CT, y0 = ty * CT, lane = threadIdx.x & 63;
+    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
+    RowWords R;
+    JoinWords J;
+    if constexpr (MODE == FG_NEQ) {
+        R.F = tile_bits(P.img, w, h, x0, y0, P.key, stage.bits);
+        const uint64_t jl = R.F & (R.F << 1), Fu = shfl_up64(R.F);
+        R.S = R.F & ~jl;
+        J = joins_to_unite<CONN>(jl, R.F & Fu, R.F & (Fu << 1), R.F & (Fu >> 1), Fu & (Fu << 1));
+    } else if constexpr (MODE == FG_EQ) {
+        tile_words_eq<CONN>(P.img, w, h, x0, y0, R, J, static_cast<uint8_t*>(B.edge) + (size_t)blockIdx.x * 2 * CT,
+                            stage.bytes);
+    } else {
+        tile_words_feq<CONN>(P, w, h, x0, y0, R, J, static_cast<float*>(B.edge) + (size_t)blockIdx.x * 2 * CT, stage.words);
+        if (threadIdx.x >= 64) return;
+        wave_order();  // the words have been read before their LDS holds bits
+    }
+    uint64_t T = 0;  // source pixels of the row
+    if constexpr (SRC == SRC_BYTES) T = tile_bits(src, w, h, x0, y0, 0, stage.bits);
+    if constexpr (SRC == SRC_BORDER) {
+        const int y = y0 + lane;
+        if (y == 0 || y == h - 1) T = ~0ull;
+        if (x0 == 0) T |= 1ull;
+        if (w - 1 - x0 < CT) T |= 1ull << (w - 1 - x0);
+    }
+    // the rows' first run numbers: exclusive scan of the run counts
+    const int nrun = popc64(R.S);
+    int off = nrun;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t i = i0 + j * S;
-            p[j] = i < n ? ld_wg(&L[i]) : -1;
-            if (flag_set && i < n) {
-                if (flag_src) {
-                    sv[j] = flag_src[i] != 0;
-                } else {
-                    const int x = (int)(i % fw), y = (int)(i / fw);
-                    sv[j] = x == 0 || y == 0 || x == fw - 1 || y == fh - 1;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int q = __shfl_up(off, o);
+        if (lane >= o) off += q;
+    }
+    off -= nrun;
+    B.rows[(size_t)blockIdx.x * CT + lane] = R;
+    B.off[(size_t)blockIdx.x * CT + lane] = (uint16_t)off;
+    const uint64_t Su = shfl_up64(R.S);
+    const int offu = dpp_from_left(0, off);
+    const int row = lane * CT, runs = __builtin_amdgcn_readlane(off + nrun, 63);
+    // A run starts out pointing at the run above of one of its joins, if it has any (a smaller number,
+    // so this is a forest without any atomics), and the forest is flattened: along a tall component
+    // one union per row at once would build a chain that every later find walks.  The joins that
+    // are left, where a run meets a second run above it, unite what is flat already.
+    {
+        int k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+            const int a = __ffsll((long long)m) - 1;
+            const uint64_t rb = run_bits(a, run_end(R.S, R.F, a)), up = J.up & rb, ul = J.ul & rb, ur = J.ur & rb;
+            const uint64_t f = up ? up : (ul ? ul : ur);
+            const int x = __ffsll((long long)f) - 1;
+            int par = k;
+            if (f) par = offu + run_index(Su, up ? x : (ul ? x - 1 : x + 1));
+            const uint64_t clr = ~(f & (0ull - f));
+            if (up) J.up &= clr;
+            else if (ul) J.ul &= clr;
+            else J.ur &= clr;
+            node[k] = (uint32_t)(row + a) << 16 | (uint32_t)par;
+        }
+    }
+    wave_order();
+    // every run at its root: pointer doubling, lane = run, four runs' reads in one round trip
+    auto flatten = [&]() {
+        for (;;) {
+            bool changed = false;
+            for (int k0 = 0; k0 < runs; k0 += 256) {
+                uint32_t v[4];
+                int q[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = node_of(node, min(k0 + 64 * j + lane, runs - 1));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) q[j] = parent_of(node, (int)(v[j] & 0xFFFFu));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int k = k0 + 64 * j + lane;
+                    if (k < runs && q[j] != (int)(v[j] & 0xFFFFu)) {
+                        node[k] = (v[j] & 0xFFFF0000u) | (uint32_t)q[j];
+                        changed = true;
+                    }
                 }
             }
+            wave_order();
+            if (!__any(changed)) break;
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) q[j] = p[j] >= 0 ? ld_wg(&L[p[j]]) : p[j];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t i = i0 + j * S;
-            if (i >= n) continue;
-            if (p[j] < 0) {
-                if (bgval != -1) L[i] = bgval;
-                continue;
-            }
-            // read-only walk: a path-jumping find here could re-point a pixel whose final root
-            // another thread has already written back to an intermediate ancestor.  Roots are final
-            // in this kernel and every value an entry takes is an ancestor, so cached loads are safe.
-            if (zero_at_roots && p[j] == (int)i) zero_at_roots[i] = 0;
-            if (zero8_at_roots && p[j] == (int)i) zero8_at_roots[i] = 0;
-            int r = p[j], nx = q[j];
-            while (nx != r) {
-                r = nx;
-                nx = ld_wg(&L[r]);
-            }
-            if (r != p[j]) L[i] = r;
-            if (sv[j]) flag_set[r] = 1;
+    };
+    flatten();
+    if (__any((J.up | J.ul | J.ur) != 0)) {
+        // one union per lane and turn, straight ones first
+        while (J.up | J.ul | J.ur) {
+            const uint64_t m = J.up ? J.up : (J.ul ? J.ul : J.ur);
+            const int x = __ffsll((long long)m) - 1, xu = J.up ? x : (J.ul ? x - 1 : x + 1);
+            const uint64_t clr = ~(m & (0ull - m));
+            if (J.up) J.up &= clr;
+            else if (J.ul) J.ul &= clr;
+            else J.ur &= clr;
+            lunite(node, off + run_index(R.S, x), offu + run_index(Su, xu));
         }
+        wave_order();
+        flatten();
+    }
+    uint16_t* const roots = B.roots + (size_t)blockIdx.x * B.cap;
+    uint16_t* const er = B.edge_roots + (size_t)blockIdx.x * 4 * CT;
+    for (int k = lane; k < runs; k += 64) roots[k] = (uint16_t)parent_of(node, k);
+    wave_order();
+    {
+        // edge pixels: left and right of the lane's row, top and bottom of the lane's column
+        auto root_place = [&](bool fg, int k) {
+            const int r = fg ? parent_of(node, k) : 0;
+            const uint32_t p = node[r] >> 16;
+            return fg ? (uint16_t)p : kNoRoot;
+        };
+        auto word_of = [](uint64_t v, int l) {
+            return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l) |
+                   (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32;
+        };
+        const uint64_t S0 = word_of(R.S, 0), F0 = word_of(R.F, 0), S3 = word_of(R.S, 63), F3 = word_of(R.F, 63);
+        const int off3 = __builtin_amdgcn_readlane(off, 63);
+        er[E_LEFT * CT + lane] = root_place(R.F & 1ull, off);
+        er[E_RIGHT * CT + lane] = root_place(R.F >> 63, off + nrun - 1);
+        er[E_TOP * CT + lane] = root_place((F0 >> lane) & 1ull, run_index(S0, lane));
+        er[E_BOTTOM * CT + lane] = root_place((F3 >> lane) & 1ull, off3 + run_index(S3, lane));
+    }
+    if (area || SRC != SRC_NONE) {
+        // the roots' places are not needed any more: count in bits 16..28, flag in bit 31
+        wave_order();
+        int k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k)
+            if (parent_of(node, k) == k) node[k] = (uint32_t)k;
+        wave_order();
+        k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+            const int a = __ffsll((long long)m) - 1, end = run_end(R.S, R.F, a), r = parent_of(node, k);
+            if (area) atomicAdd(&node[r], (uint32_t)(end - a) << 16);
+            if (SRC != SRC_NONE && (T & run_bits(a, end))) atomicOr(&node[r], 0x80000000u);
+        }
+        wave_order();
+    }
+    int k = off;
+    for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+        const uint32_t v = node_of(node, k);
+        if ((int)(v & 0xFFFFu) != k) continue;
+        const int g = (int)((size_t)(y0 + lane) * w + (x0 + __ffsll((long long)m) - 1));
+        forest[g] = g;
+        if (area) area[g] = (int)(v >> 16 & 0x1FFFu);
+        if (SRC != SRC_NONE) flag[g] = (uint8_t)(v >> 31);
     }
 }
 
-template <int MODE>
-int ccl_run(const Px& P, int32_t* L, int w, int h, int conn, int32_t bgval, hipStream_t s,
-            int32_t* zero_at_roots = nullptr, uint8_t* zero8_at_roots = nullptr, uint8_t* flag_set = nullptr,
-            const uint8_t* flag_src = nullptr) {
-    const int tiles_x = (int)cdiv(w, CT_W), tiles_y = (int)cdiv(h, CT_H);
-    const int nt = tiles_x * tiles_y;
-    const int nseam8 = nt * (CT_W + 2 * CT_H), nseam4 = nt * (CT_W + CT_H);
-    const size_t n = (size_t)w * h;
-    if (conn == 8) {
-        hipLaunchKernelGGL((ccl_local<MODE, 8>), dim3(nt), dim3(256), 0, s, P, L, w, h, tiles_x, flag_set);
-        hipLaunchKernelGGL((ccl_seams<MODE, 8>), dim3(cdiv(nseam8, 256)), dim3(256), 0, s, P, L, w, h, tiles_x, nt);
-    } else {
-        hipLaunchKernelGGL((ccl_local<MODE, 4>), dim3(nt), dim3(256), 0, s, P, L, w, h, tiles_x, flag_set);
-        hipLaunchKernelGGL((ccl_seams<MODE, 4>), dim3(cdiv(nseam4, 256)), dim3(256), 0, s, P, L, w, h, tiles_x, nt);
+// global index of the place r of tile (tx, ty)
+__device__ __forceinline__ int place_index(int tx, int ty, int r, int w) {
+    return (int)((size_t)(ty * CT + (r >> 6)) * w + (tx * CT + (r & 63)));
+}
+
+// Unions across tile edges: the tile's first wave takes the pixels of its first column with their left
+// neighbours (lane = row), the second its first row with the pixels above (lane = column).  A pixel
+// skips a union whose two tile-local roots an adjacent pixel unites by the same kind of join, or that
+// its own straight join makes: along an edge, consecutive pixels usually meet the same two components.
+template <int MODE, int CONN>
+__global__ __launch_bounds__(128) void ccl_seams(Px P, CclBufs B, int32_t* forest, int w, int h, int tiles_x) {
+    const int t = blockIdx.x, tx = t % tiles_x, ty = t / tiles_x, lane = threadIdx.x & 63;
+    using V = typename std::conditional<MODE == FG_FEQ, float, uint8_t>::type;
+    const bool vertical = threadIdx.x < 64;  // wave-uniform
+    if (vertical ? tx == 0 : ty == 0) return;
+    const uint16_t* er = B.edge_roots;
+    const int to = vertical ? t - 1 : t - tiles_x;  // the tile across the edge
+    const uint16_t rm = er[((size_t)t * 4 + (vertical ? E_LEFT : E_TOP)) * CT + lane];
+    const uint16_t ro = er[((size_t)to * 4 + (vertical ? E_RIGHT : E_BOTTOM)) * CT + lane];
+    // this pixel, the one opposite, that one's neighbours along the edge: foreground, tile-local root,
+    // value (equal-value modes)
+    const bool fm = rm != kNoRoot, fo = ro != kNoRoot;
+    const int gm = place_index(tx, ty, rm, w), go = vertical ? place_index(tx - 1, ty, ro, w) : place_index(tx, ty - 1, ro, w);
+    V vm = 0, vo = 0;
+    if (MODE != FG_NEQ) {
+        if (vertical) {
+            const V* e = static_cast<const V*>(B.edge);
+            vm = e[(size_t)t * 2 * CT + lane];
+            vo = e[(size_t)to * 2 * CT + CT + lane];
+        } else {
+            const size_t xc = (size_t)min(tx * CT + lane, w - 1);
+            const V* img;
+            if constexpr (MODE == FG_FEQ) img = P.fv;
+            else img = P.img;
+            vm = img[(size_t)ty * CT * w + xc];
+            vo = img[((size_t)ty * CT - 1) * w + xc];
+        }
     }
-    hipLaunchKernelGGL(ccl_flatten, dim3(std::min<unsigned>(cdiv(n, 1024), 65535u)), dim3(256), 0, s, L, n, bgval,
-                       zero_at_roots, zero8_at_roots, flag_src, flag_set, w, h);
+    const bool join = fm && fo && (MODE == FG_NEQ || vm == vo);
+    // neighbours along the edge
+    const bool pjoin = from_left(0, join ? 1 : 0) != 0, njoin = from_right(0, join ? 1 : 0) != 0;
+    const int pgm = from_left(-1, gm), ngm = from_right(-1, gm);
+    const int pgo = from_left(-1, go), ngo = from_right(-1, go);
+    if (join && !(pjoin && pgm == gm && pgo == go)) gunite(forest, gm, go);
+    if (CONN == 4) return;
+    bool fol = from_left(0, fo ? 1 : 0) != 0, for_ = from_right(0, fo ? 1 : 0) != 0;
+    int gol = pgo, gor = ngo;
+    V vol = 0, vor = 0;
+    if (MODE == FG_FEQ) {
+        vol = (V)from_left(0.0f, (float)vo);
+        vor = (V)from_right(0.0f, (float)vo);
+    } else if (MODE == FG_EQ) {
+        vol = (V)from_left(0, (int)vo);
+        vor = (V)from_right(0, (int)vo);
+    }
+    // the two pixels beyond the ends of the row above belong to the tiles beside it (a column's ends
+    // have no such pixel here: the first row's wave takes those joins)
+    const int side = lane == 0 ? -1 : 1, tn = t - tiles_x + side;
+    if (!vertical && ((lane == 0 && tx > 0) || (lane == 63 && tx + 1 < tiles_x))) {
+        const uint16_t r = er[((size_t)tn * 4 + E_BOTTOM) * CT + (side < 0 ? CT - 1 : 0)];
+        const bool f = r != kNoRoot;
+        const int g = place_index(tx + side, ty - 1, r, w);
+        V v = 0;
+        if (MODE != FG_NEQ) {
+            const V* img;
+            if constexpr (MODE == FG_FEQ) img = P.fv;
+            else img = P.img;
+            v = img[((size_t)ty * CT - 1) * w + (size_t)(tx * CT + (side < 0 ? -1 : CT))];
+        }
+        if (side < 0) { fol = f; gol = g; vol = v; }
+        else { for_ = f; gor = g; vor = v; }
+    }
+    const bool jl = fm && fol && (MODE == FG_NEQ || vm == vol), jr = fm && for_ && (MODE == FG_NEQ || vm == vor);
+    if (jl && !(join && gol == go) && !(pjoin && pgm == gm)) gunite(forest, gm, gol);
+    if (jr && !(join && gor == go) && !(njoin && ngm == gm)) gunite(forest, gm, gor);
+}
+
+// the final root of a tile-local root.  A read-only walk: a path-jumping find here could re-point an
+// entry whose final root another thread has already stored to an intermediate ancestor.  Roots are
+// final once the seams are done and every value an entry takes is an ancestor, so cached loads are safe.
+__device__ __forceinline__ int final_root(const int32_t* forest, int g) {
+    int r = g, nx = ld_wg(&forest[g]);
+    while (nx != r) {
+        r = nx;
+        nx = ld_wg(&forest[r]);
+    }
+    return r;
+}
+
+// Every tile-local root that is not final hands its count or flag to the final root and points at it.
+__global__ __launch_bounds__(256) void ccl_roots(CclBufs B, int32_t* forest, int w, int tiles_x, int ntiles, int32_t* area,
+                                                 uint8_t* flag) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (t >= ntiles) return;
+    const uint64_t S = B.rows[(size_t)t * CT + lane].S;
+    int k = B.off[(size_t)t * CT + lane];
+    const uint16_t* roots = B.roots + (size_t)t * B.cap;
+    for (uint64_t m = S; m; m &= m - 1, ++k) {
+        if (roots[k] != k) continue;
+        const int g = place_index(t % tiles_x, t / tiles_x, lane * CT + __ffsll((long long)m) - 1, w);
+        const int r = final_root(forest, g);
+        if (r == g) continue;
+        forest[g] = r;
+        if (area) atomicAdd(&area[r], area[g]);
+        if (flag && flag[g]) flag[r] = 1;
+    }
+}
+
+// What a selection writes per pixel, sel = the pixel's component is selected (by its area in [lo, hi),
+// or by its flag):
+//   OUT_MASK     255 where sel                           (bwareaopen2)
+//   OUT_UNSEL    255 where foreground and not sel         (plateaus without a greater neighbour)
+//   OUT_HOLES    0 where sel, else 255                    (imfillHoles: passable and reached from the border)
+//   OUT_KEEP     a where sel, else 0                      (bwselect)
+//   OUT_BINREC   a where nonzero, else 255 where sel      (imreconstructBinary: a = marker)
+//   OUT_FILL     a | (255 - a at the seeds b, else 255 where sel)   (imfill)
+enum { OUT_MASK = 0, OUT_UNSEL, OUT_HOLES, OUT_KEEP, OUT_BINREC, OUT_FILL };
+
+template <int OUT>
+__device__ __forceinline__ uint32_t select_word(uint32_t sel, uint32_t a, uint32_t b) {
+    if (OUT == OUT_HOLES) return ~sel;
+    if (OUT == OUT_KEEP) return a & sel;
+    if (OUT == OUT_BINREC) return a | (sel & ~((nonzero_bytes(a) >> 7) * 255u));
+    if (OUT == OUT_FILL) {
+        const uint32_t sd = (nonzero_bytes(b) >> 7) * 255u;
+        return a | (sd & ~a) | (sel & ~sd);
+    }
+    return sel;
+}
+
+// One tile per wave: the selected tile-local roots become bits in LDS, the selected runs bits of the
+// rows' words (lane = row), the words bytes (a lane writes four 16-byte pieces, a row is four lanes).
+// *count (optional) = number of selected components, counted at their final roots; one atomic per
+// workgroup, and the grid is at most kSelectBlocks (atomics on one address cost about 10 ns each: one
+// per tile of a 4096^2 image took 40 us).
+constexpr int kSelectBlocks = 512;
+template <int OUT>
+__global__ __launch_bounds__(256) void ccl_select(CclBufs B, const int32_t* __restrict__ forest, int w, int h, int tiles_x,
+                                                  int ntiles, const int32_t* __restrict__ area, int lo, int hi,
+                                                  const uint8_t* __restrict__ flag, const uint8_t* a, const uint8_t* b,
+                                                  uint8_t* out, int* count) {
+    __shared__ uint32_t keep_s[4][CT * CT / 32];
+    __shared__ uint64_t words_s[4][CT];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    uint32_t* const keep = keep_s[wv];
+    uint64_t* const words = words_s[wv];
+    int n = 0;
+    for (int t = blockIdx.x * 4 + wv; t < ntiles; t += 4 * gridDim.x) {
+        const int tx = t % tiles_x, ty = t / tiles_x;
+        const RowWords R = B.rows[(size_t)t * CT + lane];
+        const int off = B.off[(size_t)t * CT + lane];
+        const uint16_t* roots = B.roots + (size_t)t * B.cap;
+        keep[lane] = 0;
+        keep[64 + lane] = 0;
+        wave_order();
+        int k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+            if (roots[k] != k) continue;
+            const int g = place_index(tx, ty, lane * CT + __ffsll((long long)m) - 1, w), r = forest[g];  // final: ccl_roots has run
+            bool s;
+            if (OUT == OUT_MASK) {
+                const int ar = area[r];
+                s = ar >= lo && ar < hi;
+                n += (s && r == g) ? 1 : 0;
+            } else {
+                s = flag[r] != 0;
+            }
+            if (s) atomicOr(&keep[k >> 5], 1u << (k & 31));
+        }
+        wave_order();
+        uint64_t sel = 0;
+        k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+            const int x = __ffsll((long long)m) - 1, r = roots[k];
+            if ((keep[r >> 5] >> (r & 31)) & 1u) sel |= run_bits(x, run_end(R.S, R.F, x));
+        }
+        words[lane] = OUT == OUT_UNSEL ? R.F & ~sel : sel;
+        wave_order();
+        const int x0 = tx * CT, y0 = ty * CT, cols = min(CT, w - x0), x = 16 * (lane & 3);
+        const bool full = cols == CT;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int y = 16 * g + (lane >> 2);
+            if (y0 + y >= h || x >= cols) continue;
+            const size_t row = (size_t)(y0 + y) * w + x0;
+            uint4 va = make_uint4(0, 0, 0, 0), vb = va;
+            if (OUT >= OUT_KEEP) va = load16(a + row, x, cols, full);
+            if (OUT == OUT_FILL) vb = load16(b + row, x, cols, full);
+            const uint32_t bits = (uint32_t)(words[y] >> x);
+            const uint4 v = make_uint4(select_word<OUT>(spread_bits(bits & 15u), va.x, vb.x),
+                                       select_word<OUT>(spread_bits(bits >> 4 & 15u), va.y, vb.y),
+                                       select_word<OUT>(spread_bits(bits >> 8 & 15u), va.z, vb.z),
+                                       select_word<OUT>(spread_bits(bits >> 12 & 15u), va.w, vb.w));
+            if (full) {
+                __builtin_memcpy(out + row + x, &v, 16);
+            } else {
+                const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+                for (int j = 0; j < min(16, cols - x); ++j) out[row + x + j] = (uint8_t)(wd[j >> 2] >> (8 * (j & 3)));
+            }
+        }
+        wave_order();
+    }
+    if (count) block_count_add(n, count);  // `count` is the same for every thread
+}
+
+// Labels of a tile: the final root of each tile-local root, then of each run, in LDS; then lane = column
+// and a row a step.  forest may be the label image itself: a root's entry is overwritten with its
+// final root, which any walk may meet instead of the entry it replaces, and no other entry is read.
+__global__ __launch_bounds__(256) void ccl_label(CclBufs B, int32_t* forest, int32_t* L, int w, int h, int tiles_x,
+                                                 int32_t bgval) {
+    __shared__ int lab[CT * CT];  // by run number
+    __shared__ RowWords words[CT];
+    __shared__ int offs[CT];
+    const int t = blockIdx.x, tx = t % tiles_x, ty = t / tiles_x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const RowWords R = B.rows[(size_t)t * CT + lane];
+    const int off = B.off[(size_t)t * CT + lane];
+    const uint16_t* roots = B.roots + (size_t)t * B.cap;
+    if (wv == 0) {
+        words[lane] = R;
+        offs[lane] = off;
+    }
+    // the four waves take a row's runs in turn
+    {
+        int k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+            if (((k - off) & 3) != wv) continue;
+            if (roots[k] == k) lab[k] = final_root(forest, place_index(tx, ty, lane * CT + __ffsll((long long)m) - 1, w));
+        }
+    }
+    __syncthreads();
+    {
+        int k = off;
+        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+            if (((k - off) & 3) != wv) continue;
+            const int r = roots[k];
+            if (r != k) lab[k] = lab[r];
+        }
+    }
+    __syncthreads();
+    const int x = tx * CT + lane;
+    if (x >= w) return;
+#pragma unroll 4
+    for (int y = wv; y < CT; y += 4) {
+        if (ty * CT + y >= h) break;
+        const RowWords W = words[y];
+        const bool fg = (W.F >> lane) & 1ull;
+        const int v = lab[fg ? offs[y] + run_index(W.S, lane) : 0];
+        L[(size_t)(ty * CT + y) * w + x] = fg ? v : bgval;
+    }
+}
+
+struct CclGrid {
+    int tiles_x, nt;
+};
+CclGrid ccl_grid(int w, int h) {
+    const int tx = (int)cdiv(w, CT);
+    return CclGrid{tx, tx * (int)cdiv(h, CT)};
+}
+
+// scratch of a labelling: run slots for the most runs a tile can hold (every second pixel of a row, or
+// every pixel where equal values join)
+CclBufs ccl_carve(Carver& c, int nt, int mode) {
+    CclBufs B;
+    B.cap = ccl_cap(mode);
+    B.rows = c.take<RowWords>((size_t)nt * CT);
+    B.off = c.take<uint16_t>((size_t)nt * CT);
+    B.roots = c.take<uint16_t>((size_t)nt * B.cap);
+    B.edge_roots = c.take<uint16_t>((size_t)nt * 4 * CT);
+    B.edge = mode == FG_NEQ ? nullptr : c.take<uint8_t>((size_t)nt * 2 * CT * (mode == FG_FEQ ? sizeof(float) : 1));
+    return B;
+}
+
+struct CclWork {  // a labelling in progress
+    Scratch sc;
+    CclBufs B;
+    CclGrid g;
+};
+
+// the tile and seam passes; flag / src: see ccl_tile
+template <int MODE, int CONN, int SRC>
+int ccl_forest_t(const Px& P, CclWork& W, int32_t* forest, int w, int h, int32_t* area, uint8_t* flag, const uint8_t* src,
+                 int* zero, hipStream_t s) {
+    W.g = ccl_grid(w, h);
+    Carver m(nullptr);
+    (void)ccl_carve(m, W.g.nt, MODE);
+    NSC_CHECK(W.sc.alloc(m.size(), s));
+    Carver c(W.sc.p);
+    W.B = ccl_carve(c, W.g.nt, MODE);
+    hipLaunchKernelGGL((ccl_tile<MODE, CONN, SRC>), dim3(W.g.nt), dim3(ccl_tile_threads(MODE)), 0, s, P, W.B, forest, w, h, W.g.tiles_x, area,
+                       flag, src, zero);
+    hipLaunchKernelGGL((ccl_seams<MODE, CONN>), dim3(W.g.nt), dim3(128), 0, s, P, W.B, forest, w, h, W.g.tiles_x);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
 }
 
-// ------------------------------------------------------------------------------------------
-// operators on top of the labels
-// ------------------------------------------------------------------------------------------
-// Component areas with one atomic per run of equal labels in each wave's 64 consecutive pixels
-// (coalesced loads; the background component of a fill would otherwise take one atomic per pixel
-// on a single address).  A lane starts a run when its label differs from the previous lane's;
-// the run ends where the next one starts.
-__global__ void k_area(const int32_t* __restrict__ L, int32_t* __restrict__ area, size_t n) {
-    const int lane = threadIdx.x & 63;
-    const size_t wave = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const size_t nwave = ((size_t)gridDim.x * blockDim.x) >> 6;
-    for (size_t base = wave * 64; base < n; base += nwave * 64) {
-        const size_t i = base + lane;
-        const int r = i < n ? L[i] : -2;
-        const int prev = __shfl_up(r, 1);
-        const bool head = (lane == 0 || prev != r) && r != -2;
-        const unsigned long long heads = __ballot(head);
-        if (head && r >= 0) {
-            // next run start after this lane (or the end of the window / of the image)
-            const unsigned long long later = lane == 63 ? 0ull : (heads >> (lane + 1));
-            int end = later ? lane + 1 + __ffsll((long long)later) - 1 : 64;
-            const size_t lim = n - base;  // valid lanes in this window
-            if ((size_t)end > lim) end = (int)lim;
-            atomicAdd(&area[r], end - lane);
-        }
+template <int MODE>
+int ccl_labels(const Px& P, int32_t* L, int w, int h, int conn, int32_t bgval, hipStream_t s) {
+    CclWork W;
+    if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_NONE>(P, W, L, w, h, nullptr, nullptr, nullptr, nullptr, s)));
+    else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_NONE>(P, W, L, w, h, nullptr, nullptr, nullptr, nullptr, s)));
+    hipLaunchKernelGGL(ccl_label, dim3(W.g.nt), dim3(256), 0, s, W.B, L, L, w, h, W.g.tiles_x, bgval);
+    NSC_HIP(hipGetLastError());
+    return NSC_OK;
+}
+
+// component selection by a flag: sources = nonzero pixels of src, or the image border when src is null
+template <int MODE, int OUT>
+int ccl_select_flag(const Px& P, const uint8_t* src, const uint8_t* a, const uint8_t* b, uint8_t* out, int w, int h, int conn,
+                    int32_t* forest, uint8_t* flag, hipStream_t s) {
+    CclWork W;
+    if (src) {
+        if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_BYTES>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
+        else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_BYTES>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
+    } else {
+        if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_BORDER>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
+        else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_BORDER>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
     }
+    hipLaunchKernelGGL(ccl_roots, dim3(cdiv(W.g.nt, 4)), dim3(256), 0, s, W.B, forest, w, W.g.tiles_x, W.g.nt,
+                       (int32_t*)nullptr, flag);
+    hipLaunchKernelGGL((ccl_select<OUT>), dim3(cdiv(W.g.nt, 4)), dim3(256), 0, s, W.B, forest, w, h, W.g.tiles_x, W.g.nt,
+                       (const int32_t*)nullptr, 0, 0, flag, a, b, out, (int*)nullptr);
+    NSC_HIP(hipGetLastError());
+    return NSC_OK;
+}
+
+template <int MODE>
+int ccl_select_area(const Px& P, uint8_t* out, int w, int h, int lo, int hi, int conn, int* dcount, int32_t* forest,
+                    int32_t* area, hipStream_t s) {
+    CclWork W;
+    if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_NONE>(P, W, forest, w, h, area, nullptr, nullptr, dcount, s)));
+    else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_NONE>(P, W, forest, w, h, area, nullptr, nullptr, dcount, s)));
+    hipLaunchKernelGGL(ccl_roots, dim3(cdiv(W.g.nt, 4)), dim3(256), 0, s, W.B, forest, w, W.g.tiles_x, W.g.nt, area,
+                       (uint8_t*)nullptr);
+    const unsigned nb = dcount ? std::min<unsigned>(cdiv(W.g.nt, 4), kSelectBlocks) : cdiv(W.g.nt, 4);
+    hipLaunchKernelGGL((ccl_select<OUT_MASK>), dim3(nb), dim3(256), 0, s, W.B, forest, w, h, W.g.tiles_x, W.g.nt, area, lo, hi,
+                       (const uint8_t*)nullptr, (const uint8_t*)nullptr, (const uint8_t*)nullptr, out, dcount);
+    NSC_HIP(hipGetLastError());
+    return NSC_OK;
 }
 
 // The per-pixel label consumers below take four pixels per thread and iteration, i, i + S, i + 2S,
@@ -413,116 +863,6 @@ __global__ void k_area(const int32_t* __restrict__ L, int32_t* __restrict__ area
 #define NSC_FOR4(n)                                                                                  \
     for (size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, S = (size_t)gridDim.x * blockDim.x; \
          i0 < (n); i0 += 4 * S)
-
-// bwareaopen2 flatten output: 255 where lo <= area(root) < hi; count kept roots
-__global__ void k_area_select(const int32_t* __restrict__ L, const int32_t* __restrict__ area, uint8_t* __restrict__ out,
-                              size_t n, int lo, int hi, int* count) {
-    int local = 0;
-    NSC_FOR4(n) {
-        int r[4], a[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = i0 + j * S < n ? L[i0 + j * S] : -1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) a[j] = r[j] >= 0 ? area[r[j]] : 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t i = i0 + j * S;
-            if (i >= n) continue;
-            const bool keep = r[j] >= 0 && a[j] >= lo && a[j] < hi;
-            out[i] = keep ? 255 : 0;
-            local += (keep && (size_t)r[j] == i) ? 1 : 0;
-        }
-    }
-    if (count) block_count_add(local, count);  // `count` is the same for every thread
-}
-
-// imreconstructBinary output: marker where marker != 0, else 255 where the mask component holds a
-// source, else 0.  imfill additionally ORs with the image (mode 1) using mask = 255 - img.
-__global__ void k_binrecon_out(const int32_t* __restrict__ L, const uint8_t* __restrict__ flag,
-                               const uint8_t* __restrict__ marker, uint8_t* __restrict__ out, size_t n) {
-    NSC_FOR4(n) {
-        int r[4];
-        uint8_t m[4], f[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t i = i0 + j * S;
-            r[j] = i < n ? L[i] : -1;
-            m[j] = i < n ? marker[i] : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = r[j] >= 0 ? flag[r[j]] : 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (i0 + j * S < n) out[i0 + j * S] = m[j] ? m[j] : (f[j] ? 255 : 0);
-    }
-}
-
-// imfill(img, seeds): img | rec, rec = (255-img) at seeds inside passable (img != 255), 255 at other
-// reached pixels, 0 elsewhere
-__global__ void k_imfill_out(const int32_t* __restrict__ L, const uint8_t* __restrict__ flag, const uint8_t* __restrict__ img,
-                             const uint8_t* __restrict__ seeds, uint8_t* __restrict__ out, size_t n) {
-    NSC_FOR4(n) {
-        int r[4];
-        uint8_t v[4], sd[4], f[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t i = i0 + j * S;
-            r[j] = i < n ? L[i] : -1;
-            v[j] = i < n ? img[i] : 0;
-            sd[j] = i < n ? seeds[i] : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = r[j] >= 0 ? flag[r[j]] : 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint8_t rec = sd[j] ? (uint8_t)(255 - v[j]) : (f[j] ? 255 : 0);
-            if (i0 + j * S < n) out[i0 + j * S] = v[j] | rec;
-        }
-    }
-}
-
-// imfillHoles(binary): 255 unless the pixel is passable (!= 255) and its component touches the border
-__global__ void k_fillholes_out(const int32_t* __restrict__ L, const uint8_t* __restrict__ flag, uint8_t* __restrict__ out,
-                                size_t n) {
-    NSC_FOR4(n) {
-        int r[4];
-        uint8_t f[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = i0 + j * S < n ? L[i0 + j * S] : -1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = r[j] >= 0 ? flag[r[j]] : 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (i0 + j * S < n) out[i0 + j * S] = f[j] ? 0 : 255;
-    }
-}
-
-// bwselect: bw where the component holds a seed pixel
-__global__ void k_bwselect_out(const int32_t* __restrict__ L, const uint8_t* __restrict__ flag, const uint8_t* __restrict__ bw,
-                               uint8_t* __restrict__ out, size_t n) {
-    NSC_FOR4(n) {
-        int r[4];
-        uint8_t b[4], f[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const size_t i = i0 + j * S;
-            r[j] = i < n ? L[i] : -1;
-            b[j] = i < n ? bw[i] : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = r[j] >= 0 ? flag[r[j]] : 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (i0 + j * S < n) out[i0 + j * S] = f[j] ? b[j] : 0;
-    }
-}
-
-__global__ void k_and_nonzero(const uint8_t* a, const uint8_t* b, uint8_t* out, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const uint8_t av = a[i], bv = b[i];  // both loads unconditional (no branch around the second)
-        out[i] = (av != 0 && bv != 0) ? 255 : 0;
-    }
-}
 
 // ---- canonical relabel: rank of each root in raster order ----
 // A workgroup of 1024 threads covers SCAN_B = 4096 consecutive pixels, four per thread (contiguous,
@@ -768,65 +1108,38 @@ __global__ void k_fill_i32(int32_t* p, int32_t v, size_t n) {
 }  // namespace
 
 // ------------------------------------------------------------------------------------------
-int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, bool equal_values, int32_t bgval,
-           hipStream_t s) {
-    Px P{img, nullptr, 0};
-    if (equal_values) return ccl_run<FG_EQ>(P, labels, w, h, conn, bgval, s);
-    return ccl_run<FG_NEQ>(P, labels, w, h, conn, bgval, s);
+// binary: every nonzero pixel has the same value, so equal-value joins are joins of foreground
+int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, int32_t bgval, bool binary, hipStream_t s) {
+    const Px P{img, nullptr, 0};
+    return binary ? ccl_labels<FG_NEQ>(P, labels, w, h, conn, bgval, s) : ccl_labels<FG_EQ>(P, labels, w, h, conn, bgval, s);
 }
 
 int ccl_neq(const uint8_t* img, uint8_t key, int32_t* labels, int w, int h, int conn, hipStream_t s) {
-    Px P{img, nullptr, key};
-    return ccl_run<FG_NEQ>(P, labels, w, h, conn, -1, s);
+    return ccl_labels<FG_NEQ>(Px{img, nullptr, key}, labels, w, h, conn, -1, s);
 }
 
-int ccl_mask(const uint8_t* fg, const float* vals, int32_t* labels, int w, int h, int conn, hipStream_t s) {
-    Px P{fg, vals, 0};
-    return ccl_run<FG_FEQ>(P, labels, w, h, conn, -1, s);
+// 255 where the connected set of equal `vals` among the pixels with fg != 0 holds no pixel with
+// src != 0, else 0
+int ccl_plateaus_without(const uint8_t* fg, const float* vals, const uint8_t* src, uint8_t* out, int w, int h, int conn,
+                         int32_t* forest, uint8_t* flag, hipStream_t s) {
+    return ccl_select_flag<FG_FEQ, OUT_UNSEL>(Px{fg, vals, 0}, src, nullptr, nullptr, out, w, h, conn, forest, flag, s);
 }
 
-// ccl_mask whose flatten also clears flags[root] for every root (a per-root flag table then
-// needs no image-sized fill)
-int ccl_mask_clear_root_flags(const uint8_t* fg, const float* vals, int32_t* labels, int w, int h, int conn,
-                              uint8_t* flags, hipStream_t s) {
-    Px P{fg, vals, 0};
-    return ccl_run<FG_FEQ>(P, labels, w, h, conn, -1, s, nullptr, flags);
-}
-
-int bwareaopen_impl(const uint8_t* img, uint8_t* out, int w, int h, int lo, int hi, int conn, int* dcount,
+int bwareaopen_impl(const uint8_t* img, uint8_t* out, int w, int h, int lo, int hi, int conn, int* dcount, bool binary,
                     int32_t* labels, int32_t* area, hipStream_t s) {
-    const size_t n = (size_t)w * h;
-    // equal-value labelling whose flatten clears the roots' area entries (the only ones read)
-    NSC_CHECK(ccl_run<FG_EQ>(Px{img, nullptr, 0}, labels, w, h, conn, -1, s, area));
-    hipLaunchKernelGGL(k_area, grid1(n), dim3(256), 0, s, labels, area, n);
-    if (dcount) NSC_HIP(hipMemsetAsync(dcount, 0, sizeof(int), s));
-    hipLaunchKernelGGL(k_area_select, grid_counted(n), dim3(256), 0, s, labels, area, out, n, lo, hi, dcount);
-    NSC_HIP(hipGetLastError());
-    return NSC_OK;
-}
-
-// component selection: passable = (img != key), sources = src != 0 (or the border when src null)
-static int select_components(const uint8_t* img, uint8_t key, const uint8_t* src, int32_t* labels, uint8_t* flag,
-                             int w, int h, int conn, hipStream_t s) {
-    // labelling that clears the roots' flags (the only entries read or set) in its tile pass and
-    // sets them while flattening: flag[root] = 1 for components holding a source
-    return ccl_run<FG_NEQ>(Px{img, nullptr, key}, labels, w, h, conn, -1, s, nullptr, nullptr, flag, src);
+    const Px P{img, nullptr, 0};
+    return binary ? ccl_select_area<FG_NEQ>(P, out, w, h, lo, hi, conn, dcount, labels, area, s)
+                  : ccl_select_area<FG_EQ>(P, out, w, h, lo, hi, conn, dcount, labels, area, s);
 }
 
 int fill_holes_impl(const uint8_t* img, uint8_t* out, int w, int h, int conn, int32_t* labels, uint8_t* flag,
                     hipStream_t s) {
-    NSC_CHECK(select_components(img, 255, nullptr, labels, flag, w, h, conn, s));
-    hipLaunchKernelGGL(k_fillholes_out, grid1((size_t)w * h), dim3(256), 0, s, labels, flag, out, (size_t)w * h);
-    NSC_HIP(hipGetLastError());
-    return NSC_OK;
+    return ccl_select_flag<FG_NEQ, OUT_HOLES>(Px{img, nullptr, 255}, nullptr, nullptr, nullptr, out, w, h, conn, labels, flag, s);
 }
 
 int bwselect_impl(const uint8_t* bw, const uint8_t* seeds, uint8_t* out, int w, int h, int conn, int32_t* labels,
                   uint8_t* flag, hipStream_t s) {
-    NSC_CHECK(select_components(bw, 0, seeds, labels, flag, w, h, conn, s));
-    hipLaunchKernelGGL(k_bwselect_out, grid1((size_t)w * h), dim3(256), 0, s, labels, flag, bw, out, (size_t)w * h);
-    NSC_HIP(hipGetLastError());
-    return NSC_OK;
+    return ccl_select_flag<FG_NEQ, OUT_KEEP>(Px{bw, nullptr, 0}, seeds, bw, nullptr, out, w, h, conn, labels, flag, s);
 }
 
 int relabel_impl(int32_t* labels, int w, int h, int32_t bgval, int* dcount, int32_t* rank, hipStream_t s) {
@@ -907,7 +1220,7 @@ int nsc_cc_label_u8(const uint8_t* img, int32_t* labels, int w, int h, int32_t b
     NSC_ARG(img && labels && w > 0 && h > 0 && valid_conn(conn), "cc_label_u8");
     NSC_LABEL_SIZE(w, h);
     NSC_CHECK(ensure_init());
-    return ccl_u8(img, labels, w, h, conn, true, bgval, as_stream(stream));
+    return ccl_u8(img, labels, w, h, conn, bgval, false, as_stream(stream));
 }
 
 int nsc_bwlabel2_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, void* stream) {
@@ -943,7 +1256,7 @@ int nsc_bwareaopen2_u8(const uint8_t* img, uint8_t* out, int w, int h, int minSi
     int32_t* labels = sc.as<int32_t>();
     int32_t* area = labels + n;
     int* dcount = reinterpret_cast<int*>(area + n);
-    NSC_CHECK(bwareaopen_impl(img, out, w, h, minSize, maxSize, conn, dcount, labels, area, s));
+    NSC_CHECK(bwareaopen_impl(img, out, w, h, minSize, maxSize, conn, dcount, false, labels, area, s));
     if (count) {
         NSC_HIP(hipMemcpyAsync(count, dcount, sizeof(int), hipMemcpyDeviceToHost, s));
         NSC_HIP(stream_sync(s));
@@ -959,15 +1272,11 @@ int nsc_imreconstruct_binary_u8(const uint8_t* marker, const uint8_t* mask, uint
     hipStream_t s = as_stream(stream);
     const size_t n = (size_t)w * h;
     Scratch sc;
-    NSC_CHECK(sc.alloc(sizeof(int32_t) * n + 2 * n, s));
+    NSC_CHECK(sc.alloc(sizeof(int32_t) * n + n, s));
     int32_t* labels = sc.as<int32_t>();
-    uint8_t* flag = reinterpret_cast<uint8_t*>(labels + n);
-    uint8_t* src = flag + n;
-    hipLaunchKernelGGL(k_and_nonzero, grid1(n), dim3(256), 0, s, marker, mask, src, n);
-    NSC_CHECK(select_components(mask, 0, src, labels, flag, w, h, conn, s));
-    hipLaunchKernelGGL(k_binrecon_out, grid1(n), dim3(256), 0, s, labels, flag, marker, out, n);
-    NSC_HIP(hipGetLastError());
-    return NSC_OK;
+    // a component is reached where the marker is nonzero on one of its (mask) pixels
+    return ccl_select_flag<FG_NEQ, OUT_BINREC>(Px{mask, nullptr, 0}, marker, marker, nullptr, out, w, h, conn, labels,
+                                               reinterpret_cast<uint8_t*>(labels + n), s);
 }
 
 int nsc_imfill_u8(const uint8_t* img, const uint8_t* seeds, uint8_t* out, int w, int h, int conn, void* stream) {
@@ -979,11 +1288,8 @@ int nsc_imfill_u8(const uint8_t* img, const uint8_t* seeds, uint8_t* out, int w,
     Scratch sc;
     NSC_CHECK(sc.alloc(sizeof(int32_t) * n + n, s));
     int32_t* labels = sc.as<int32_t>();
-    uint8_t* flag = reinterpret_cast<uint8_t*>(labels + n);
-    NSC_CHECK(select_components(img, 255, seeds, labels, flag, w, h, conn, s));
-    hipLaunchKernelGGL(k_imfill_out, grid1(n), dim3(256), 0, s, labels, flag, img, seeds, out, n);
-    NSC_HIP(hipGetLastError());
-    return NSC_OK;
+    return ccl_select_flag<FG_NEQ, OUT_FILL>(Px{img, nullptr, 255}, seeds, img, seeds, out, w, h, conn, labels,
+                                             reinterpret_cast<uint8_t*>(labels + n), s);
 }
 
 int nsc_imfill_holes_u8(const uint8_t* img, uint8_t* out, int w, int h, int conn, void* stream) {

@@ -18,7 +18,7 @@ int morph_impl(const uint8_t* in, uint8_t* out, int w, int h, const uint8_t* ker
                hipStream_t s);
 int morph_open_impl(const uint8_t* in, uint8_t* out, uint8_t* tmp, int w, int h, const uint8_t* kernel, int k,
                     hipStream_t s);
-int bwareaopen_impl(const uint8_t* img, uint8_t* out, int w, int h, int lo, int hi, int conn, int* dcount,
+int bwareaopen_impl(const uint8_t* img, uint8_t* out, int w, int h, int lo, int hi, int conn, int* dcount, bool binary,
                     int32_t* labels, int32_t* area, hipStream_t s);
 int fill_holes_impl(const uint8_t* img, uint8_t* out, int w, int h, int conn, int32_t* labels, uint8_t* flag,
                     hipStream_t s);
@@ -30,7 +30,7 @@ int local_max_impl(const float* img, uint8_t* out, int w, int h, int conn, bool 
 size_t local_max_scratch(int w, int h);
 size_t ws2_scratch(int w, int h);
 int ws2_from_labels(const uint8_t* bgr, const int32_t* labels, int32_t* out, int w, int h, void* scratch, hipStream_t s);
-int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, bool equal_values, int32_t bgval, hipStream_t s);
+int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, int32_t bgval, bool binary, hipStream_t s);
 int relabel_impl(int32_t* labels, int w, int h, int32_t bgval, int* dcount, int32_t* rank, hipStream_t s);
 int root_count_impl(const int32_t* labels, int w, int h, int* dcount, hipStream_t s);
 int bbox_impl(const int32_t* canon, int w, int h, int n, int32_t* out5, int32_t* area, hipStream_t s);
@@ -427,7 +427,7 @@ int stage_s1(Chain& C, const uint8_t* bgr, int w, int h, const nsc_seg_params& p
     NSC_CHECK(fill_holes_impl(W.t1, W.fill1, w, h, p.fillHolesConnectivity, W.L, W.tmp8, s));
     NSC_CHECK(C.save(7, W.fill1, n));
     C.mark(7);
-    NSC_CHECK(bwareaopen_impl(W.fill1, W.bw1_t, w, h, p.minSize, p.maxSize, 8, &W.counts[1], W.L, W.area, s));
+    NSC_CHECK(bwareaopen_impl(W.fill1, W.bw1_t, w, h, p.minSize, p.maxSize, 8, &W.counts[1], true, W.L, W.area, s));
     NSC_CHECK(C.save(8, W.bw1_t, n));
     NSC_CHECK(C.save(9, W.t2, n));
     C.mark(8);
@@ -444,11 +444,12 @@ int stage_s1(Chain& C, const uint8_t* bgr, int w, int h, const nsc_seg_params& p
 }
 
 // plSeparateNuclei (HistologicalEntities.cpp:308-449) on seg_open: seg_nonoverlap in W.nonov.
-int stage_a4(Chain& C, const uint8_t* bgr, const uint8_t* seg_open, int w, int h, int minSizePl, int wsConn) {
+// binary: seg_open holds 0 and 255 only (the chain's own), else any values (a caller's mask).
+int stage_a4(Chain& C, const uint8_t* bgr, const uint8_t* seg_open, bool binary, int w, int h, int minSizePl, int wsConn) {
     Workspace& W = C.W;
     hipStream_t s = C.s;
     const size_t n = (size_t)w * h;
-    NSC_CHECK(bwareaopen_impl(seg_open, W.seg_big_t, w, h, minSizePl, INT_MAX, 8, nullptr, W.L, W.area, s));
+    NSC_CHECK(bwareaopen_impl(seg_open, W.seg_big_t, w, h, minSizePl, INT_MAX, 8, nullptr, binary, W.L, W.area, s));
     NSC_CHECK(C.save(14, W.seg_big_t, n));
     C.mark(14);
     NSC_CHECK(morph_impl(W.seg_big_t, W.seg_big, w, h, kCross3, 3, 0, false, s));  // HE.cpp:330
@@ -467,7 +468,7 @@ int stage_a4(Chain& C, const uint8_t* bgr, const uint8_t* seg_open, int w, int h
     C.mark(18);
     // watershed2(nuclei, distance2, watershedConnectivity)  HE.cpp:414
     NSC_CHECK(local_max_impl(W.d2, W.tmp8, w, h, wsConn, true, W.big, s));
-    NSC_CHECK(ccl_u8(W.tmp8, W.L, w, h, wsConn, true, -1, s));
+    NSC_CHECK(ccl_u8(W.tmp8, W.L, w, h, wsConn, -1, true, s));
     NSC_CHECK(ws2_from_labels(W.nuclei, W.L, W.wm, w, h, W.big, s));
     NSC_CHECK(C.save(20, W.wm, 4 * n));
     hipLaunchKernelGGL(k_nonoverlap, grid1(n), dim3(256), 0, s, W.seg_big, W.wm, W.nonov, n);
@@ -553,16 +554,16 @@ int segment_body(const uint8_t* bgr_in, int w, int h, const nsc_seg_params& p, i
     NSC_CHECK(morph_open_impl(W.seg_nohole, W.seg_open, W.tmp8, w, h, kCross3, 3, s));  // HE.cpp:498-499
     NSC_CHECK(C.save(13, W.seg_open, n));
     C.mark(13);
-    st = stage_a4(C, bgr, W.seg_open, w, h, p.minSizePl, p.watershedConnectivity);
+    st = stage_a4(C, bgr, W.seg_open, true, w, h, p.minSizePl, p.watershedConnectivity);
     if (st != NSC_SEG_CONTINUE) return st;
 
-    NSC_CHECK(bwareaopen_impl(W.nonov, W.seg, w, h, p.minSizeSeg, p.maxSizeSeg, 4, &W.counts[2], W.L, W.area, s));  // :548
+    NSC_CHECK(bwareaopen_impl(W.nonov, W.seg, w, h, p.minSizeSeg, p.maxSizeSeg, 4, &W.counts[2], true, W.L, W.area, s));  // :548
     NSC_CHECK(C.save(23, W.seg, n));
     C.mark(23);
     NSC_CHECK(fill_holes_impl(W.seg, W.fin, w, h, p.fillHolesConnectivity, W.L, W.tmp8, s));  // :573
     NSC_CHECK(C.save(24, W.fin, n));
     C.mark(24);
-    NSC_CHECK(ccl_u8(W.fin, labels, w, h, 8, true, -1, s));  // bwlabel2(final, 8) :585
+    NSC_CHECK(ccl_u8(W.fin, labels, w, h, 8, -1, true, s));  // bwlabel2(final, 8) :585
     NSC_CHECK(C.save(25, labels, 4 * n));
     // number of nuclei = number of roots (rank scratch in W.area)
     const bool canonical = io && io->canonical;
@@ -701,7 +702,7 @@ int nsc_pl_separate_nuclei(const uint8_t* bgr, size_t bgr_step, const uint8_t* s
             in = bgr_c.as<uint8_t>();
         }
         NSC_HIP(hipMemcpy2DAsync(W.seg_open, (size_t)w, seg_open, open_step, (size_t)w, h, hipMemcpyDeviceToDevice, s));
-        const int st = stage_a4(C, in, W.seg_open, w, h, minSizePl, watershedConnectivity);
+        const int st = stage_a4(C, in, W.seg_open, false, w, h, minSizePl, watershedConnectivity);
         if (st != NSC_SEG_CONTINUE) return st;
         NSC_HIP(hipMemcpy2DAsync(seg_nonoverlap, out_step, W.nonov, (size_t)w, (size_t)w, h, hipMemcpyDeviceToDevice, s));
         NSC_HIP(stream_sync(s));

@@ -284,13 +284,6 @@ __device__ __forceinline__ R from_right(R old, R v) {
 }
 
 // ---- internal entry points shared between translation units ------------------------------
-// connected-component labelling with min-index roots; pred: 0 = nonzero, 1 = equal u8 values,
-// 2 = equal float values restricted to fg != 0 (fg given separately)
-struct CCL;
-int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, bool equal_values, int32_t bgval,
-           hipStream_t s);
-int ccl_mask(const uint8_t* fg, const float* vals, int32_t* labels, int w, int h, int conn, hipStream_t s);
-
 template <typename T>
 int recon_impl(const T* marker, const T* mask, T* out, int w, int h, int conn, hipStream_t s);
 template <typename T>

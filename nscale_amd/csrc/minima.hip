@@ -17,9 +17,8 @@
 
 namespace nsc {
 
-int ccl_mask(const uint8_t* fg, const float* vals, int32_t* labels, int w, int h, int conn, hipStream_t s);
-int ccl_mask_clear_root_flags(const uint8_t* fg, const float* vals, int32_t* labels, int w, int h, int conn,
-                              uint8_t* flags, hipStream_t s);
+int ccl_plateaus_without(const uint8_t* fg, const float* vals, const uint8_t* src, uint8_t* out, int w, int h, int conn,
+                         int32_t* forest, uint8_t* flag, hipStream_t s);
 
 namespace {
 
@@ -69,23 +68,6 @@ __global__ void k_lmax_cand(const float* __restrict__ c, const float* __restrict
         const bool cd = !(mk < rc);
         cand[i] = cd ? 1 : 0;
         greater[i] = (cd && g) ? 1 : 0;
-    }
-}
-
-__global__ void k_flag_from(const int32_t* __restrict__ L, const uint8_t* __restrict__ src, uint8_t* flag, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        if (src[i]) {
-            const int r = L[i];
-            if (r >= 0) flag[r] = 1;
-        }
-    }
-}
-
-__global__ void k_lmax_out(const int32_t* __restrict__ L, const uint8_t* __restrict__ flag, uint8_t* __restrict__ out,
-                           size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int r = L[i];
-        out[i] = (r >= 0 && !flag[r]) ? 255 : 0;
     }
 }
 
@@ -154,11 +136,8 @@ int local_max_impl(const float* img, uint8_t* out, int w, int h, int conn, bool 
         hipLaunchKernelGGL((k_lmax_cand<8>), grid1(n), dim3(256), 0, s, c, marker, rec, cand, greater, w, h);
     else
         hipLaunchKernelGGL((k_lmax_cand<4>), grid1(n), dim3(256), 0, s, c, marker, rec, cand, greater, w, h);
-    NSC_CHECK(ccl_mask_clear_root_flags(cand, c, L, w, h, conn, flag, s));  // flag[] is read at roots only
-    hipLaunchKernelGGL(k_flag_from, grid1(n), dim3(256), 0, s, L, greater, flag, n);
-    hipLaunchKernelGGL(k_lmax_out, grid1(n), dim3(256), 0, s, L, flag, out, n);
     NSC_HIP(hipGetLastError());
-    return NSC_OK;
+    return ccl_plateaus_without(cand, c, greater, out, w, h, conn, L, flag, s);
 }
 
 }  // namespace nsc

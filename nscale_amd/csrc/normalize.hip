@@ -58,8 +58,11 @@ struct NormParams {
 // coefficients, d_fg - d_bg = (97 R - 852 G + 621 B - 4169) / 1000 exactly; the float coefficients
 // and the float roundings of values below 300 move it by less than 1e-4, so wherever that integer
 // is not zero its sign decides, and only exact ties (75 of the 2^24 colours) take the float path.
+__device__ __forceinline__ int norm_num(uint32_t b, uint32_t g, uint32_t r) {
+    return 97 * (int)r - 852 * (int)g + 621 * (int)b - 4169;
+}
 __device__ __forceinline__ bool norm_fg(const NormDisc& D, uint32_t b, uint32_t g, uint32_t r) {
-    const int num = 97 * (int)r - 852 * (int)g + 621 * (int)b - 4169;
+    const int num = norm_num(b, g, r);
     if (num != 0) return num > 0;
     float d[2];
 #pragma unroll
@@ -244,10 +247,13 @@ __device__ __forceinline__ uint32_t norm_px(const uint32_t wd[3], int k) {
            0xFFFFFFu;
 }
 
-// one selected pixel into the thread's sums
-__device__ __forceinline__ void stats_add(const NormConsts& C, const double2* lg, uint32_t px, double acc[7]) {
+// one listed pixel (foreground, or one of the discriminant's ties) into the thread's sums
+__device__ __forceinline__ void stats_add(const NormConsts& C, const NormDisc& D, const double2* lg, uint32_t px,
+                                          double acc[7]) {
+    const uint32_t b = px & 255u, g = px >> 8 & 255u, r = px >> 16;
+    if (!norm_fg(D, b, g, r)) return;  // a tie that the float path decides against
     float lab[3];
-    norm_lab(C, lg, px & 255u, px >> 8 & 255u, px >> 16, lab);
+    norm_lab(C, lg, b, g, r, lab);
     if (!((lab[0] * lab[1]) * lab[2] > 0.0f)) return;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -270,8 +276,6 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_stats(NormImage I, NormCo
     constexpr int kWaves = kNormThreads / 64, kPer = kNormChunk / kStatsPiece;
     __shared__ double2 lg[kLogTabN];
     __shared__ uint32_t lists[kWaves][64 + kStatsPiece];
-    load_log_tab(lg);
-    __syncthreads();
     const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
     uint32_t* const list = lists[wv];
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
@@ -291,12 +295,14 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_stats(NormImage I, NormCo
     uint32_t wd[3], nx[3];
     long long pc = (long long)blockIdx.x * kWaves + wv;
     int mine = load(pc, wd);
+    load_log_tab(lg);
+    __syncthreads();
     for (; pc < pieces; pc += step) {
         const int nmine = load(pc + step, nx);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const uint32_t px = norm_px(wd, k);
-            const bool take = k < mine && norm_fg(D, px & 255u, px >> 8 & 255u, px >> 16);
+            const bool take = k < mine && norm_num(px & 255u, px >> 8 & 255u, px >> 16) >= 0;
             const unsigned long long m = __ballot(take);
             if (take) list[held + __popcll(m & ((1ull << ln) - 1ull))] = px;
             held += __popcll(m);
@@ -304,14 +310,14 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_stats(NormImage I, NormCo
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         while (held >= 64) {
             held -= 64;
-            stats_add(C, lg, list[held + ln], acc);
+            stats_add(C, D, lg, list[held + ln], acc);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         mine = nmine;
 #pragma unroll
         for (int k = 0; k < 3; ++k) wd[k] = nx[k];
     }
-    if (ln < held) stats_add(C, lg, list[ln], acc);
+    if (ln < held) stats_add(C, D, lg, list[ln], acc);
     __shared__ double red[kNormThreads / 64][8];
 #pragma unroll
     for (int c = 0; c < 7; ++c) {
@@ -372,8 +378,9 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_finish(const double* __re
 // A chunk's bytes pass through LDS: each thread takes its four pixels as words, settles the
 // background pixels that norm_bg_fast decides and lists the others; the list is then worked
 // through densely, and the chunk leaves as words again.
-// 4096^2 H&E tile: 79 us (185 us with the full transform, by series, on every pixel).
-__global__ __launch_bounds__(kNormThreads) void k_norm_apply(NormImage I, NormConsts C, NormDisc D, NormBg G,
+// 4096^2 H&E tile: 81 us (185 us with the full transform, by series, on every pixel).
+// Six waves per SIMD: three workgroups of a CU work while another waits at its barrier.
+__global__ __launch_bounds__(kNormThreads, 6) void k_norm_apply(NormImage I, NormConsts C, NormDisc D, NormBg G,
                                                              const double* __restrict__ part, int nblocks,
                                                              NormParams target, uint8_t* out, size_t out_ld) {
     __shared__ NormTabs T;
@@ -383,6 +390,16 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_apply(NormImage I, NormCo
     __shared__ double red[kNormThreads / 64][8], tot[8];
     __shared__ NormParams sP;
     static_assert(kNormChunk <= 1 << 15, "list entries hold a pixel and a flag");
+    // an item's words and the number of pixels the thread has of it; the first item's are on their way
+    // while the tables and the totals are made
+    auto load = [&](long long it, uint32_t wd[3]) {
+        size_t off;
+        const int mine = min(max(norm_item(I, it, I.ld, &off) - 4 * (int)threadIdx.x, 0), 4);
+        norm_load4(I.bgr + off + 12 * (size_t)threadIdx.x, mine, wd);
+        return mine;
+    };
+    uint32_t wd[3];
+    int mine = load(blockIdx.x, wd);  // the grid has at most one workgroup per item
     load_log_tab(T.lg);
     for (int i = threadIdx.x; i < kExpTabN; i += kNormThreads) T.ex[i] = kExpTab[i];
     if (threadIdx.x < 2) count[threadIdx.x] = 0;
@@ -398,12 +415,8 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_apply(NormImage I, NormCo
     uint8_t* const by = reinterpret_cast<uint8_t*>(buf);
     int turn = 0;
     for (long long it = blockIdx.x; it < I.items; it += gridDim.x, turn ^= 1) {
-        size_t off, ooff;
-        const int n = norm_item(I, it, I.ld, &off);
-        (void)norm_item(I, it, out_ld, &ooff);
-        const int mine = min(max(n - 4 * (int)threadIdx.x, 0), 4);
-        uint32_t wd[3], px[4];
-        norm_load4(I.bgr + off + 12 * (size_t)threadIdx.x, mine, wd);
+        if (it != (long long)blockIdx.x) mine = load(it, wd);
+        uint32_t px[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             px[k] = norm_px(wd, k);
@@ -446,6 +459,8 @@ __global__ __launch_bounds__(kNormThreads) void k_norm_apply(NormImage I, NormCo
             p[2] = o[2];
         }
         __syncthreads();
+        size_t ooff;
+        (void)norm_item(I, it, out_ld, &ooff);
         uint8_t* q = out + ooff + 12 * (size_t)threadIdx.x;
         if (mine == 4 && (reinterpret_cast<uintptr_t>(q) & 3) == 0) {
             uint32_t* qw = reinterpret_cast<uint32_t*>(q);

@@ -257,7 +257,7 @@ using namespace nsc;
 namespace nsc {
 int local_max_impl(const float* img, uint8_t* out, int w, int h, int conn, bool minima, void* scratch, hipStream_t s);
 size_t local_max_scratch(int w, int h);
-int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, bool equal_values, int32_t bgval, hipStream_t s);
+int ccl_u8(const uint8_t* img, int32_t* labels, int w, int h, int conn, int32_t bgval, bool binary, hipStream_t s);
 }  // namespace nsc
 
 extern "C" {
@@ -298,7 +298,7 @@ int nsc_watershed2(const uint8_t* bgr, const float* img, int32_t* out, int w, in
     uint8_t* minima = b.as<uint8_t>();
     int32_t* labels = reinterpret_cast<int32_t*>(minima + n + (16 - n % 16) % 16);
     NSC_CHECK(local_max_impl(img, minima, w, h, conn, true, a.p, s));  // localMinima (MO.cpp:3730)
-    NSC_CHECK(ccl_u8(minima, labels, w, h, conn, true, -1, s));       // bwlabel2 (MO.cpp:3737)
+    NSC_CHECK(ccl_u8(minima, labels, w, h, conn, -1, true, s));       // bwlabel2 (MO.cpp:3737)
     return ws2_from_labels(bgr, labels, out, w, h, a.p, s);
 }
 
