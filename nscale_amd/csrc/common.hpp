@@ -52,9 +52,9 @@ int ensure_init();
 // Scratch comes from the calling thread's arena when one is active (a chain call activates its
 // workspace's arena: a device buffer allocated once, handed out as a stack -- scopes nest, so
 // frees arrive in reverse order, and a buffer freed out of order is reclaimed when everything
-// above it is gone), else from the device's default memory pool (hipMallocAsync, release
-// threshold raised at init).  Either way the memory is stream-ordered: reuse by a later
-// operator on the same stream is safe without synchronisation.
+// above it is gone), else from the thread's call cache (below), else from the device's default memory
+// pool (hipMallocAsync, release threshold raised at init).  Either way the memory is stream-ordered:
+// reuse by a later operator on the same stream is safe without synchronisation.
 struct Arena {
     uint8_t* base = nullptr;
     size_t cap = 0, top = 0;
@@ -87,10 +87,18 @@ struct ArenaScope {
     ~ArenaScope() { thread_arena() = prev; }
 };
 
+// Call cache: operator calls outside a chain take their scratch from blocks that the calling thread
+// keeps (capi.cpp).  The pool's free and allocation cost 12-37 us a pair while one size repeats, and
+// 360 us when sizes alternate (hipMallocAsync 200, hipFreeAsync 160; five pairs are one labelling
+// call's), more than most operators' kernels.  take returns nullptr where the cache does not serve: the
+// pool does then.
+void* call_cache_take(size_t bytes, hipStream_t s);
+void call_cache_give(void* p);
+
 struct Scratch {
     void* p = nullptr;
     hipStream_t s = nullptr;
-    bool from_arena = false;
+    bool from_arena = false, from_cache = false;
     Scratch() = default;
     Scratch(const Scratch&) = delete;
     Scratch& operator=(const Scratch&) = delete;
@@ -105,6 +113,10 @@ struct Scratch {
                 return NSC_OK;
             }
         }
+        if ((p = call_cache_take(bytes, stream)) != nullptr) {
+            from_cache = true;
+            return NSC_OK;
+        }
         hipError_t e = hipMallocAsync(&p, bytes, stream);
         if (e != hipSuccess) {
             p = nullptr;
@@ -118,12 +130,14 @@ struct Scratch {
             if (from_arena) {
                 Arena* a = thread_arena();
                 if (!a || !a->give(p)) { /* arena gone: nothing to return */ }
+            } else if (from_cache) {
+                call_cache_give(p);
             } else {
                 (void)hipFreeAsync(p, s);
             }
         }
         p = nullptr;
-        from_arena = false;
+        from_arena = from_cache = false;
     }
     template <typename T>
     T* as() const { return static_cast<T*>(p); }
