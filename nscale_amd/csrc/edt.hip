@@ -7,13 +7,21 @@
 // precise transform evaluates (sqr_tab[|q-p|] + f[p]); rows without any zero in any column give
 // sqrtf(0 + 1e15f) as OpenCV's "infinite" column value does.
 //
-// Column pass (segmented for parallelism): per 64-row column segment, first/last zero; per column,
-// carry of the nearest zero above/below each segment; per segment, the final vertical distance g
-// (uint16, 0xFFFF = no zero in the column) from a 64-bit mask of the segment's zero rows.
-// Row pass: one workgroup per row, g staged in LDS; each pixel searches outward while dx^2 is
-// below its best squared distance (work ~ distance value).  A pixel whose search would exceed
-// SEARCH_CAP columns flags its row; flagged rows are recomputed with the exact integer
-// lower-envelope algorithm (one thread per row, O(w)).
+// 1. k_edt_masks: the zero pixels of every column as 64-bit words, one per 64 rows.
+// 2. k_edt_tiles: 64 x 64 pixels per workgroup, with 32 columns more on either side.  A thread turns
+//    its column's words (its own and the two next to it) into the vertical distances g of its 64
+//    rows, capped at 63, in LDS; then each pair of pixels looks outward, both sides and both pixels in
+//    one packed 16-bit operation, while dx^2 is below its best squared distance (four pairs per thread
+//    at once: with one, a turn is a round trip to LDS and 512^2 took 40 us).  A result of at most
+//    32^2 is exact: every candidate it has not seen is larger (dx > 32, or g > 32 where the cap or the
+//    missing words hide it).  Pixels further away flag their row.
+// 3. k_edt_rows: flagged rows (the others' workgroups leave at once).  g of the whole row from the
+//    words; each flagged pixel searches outward over the row; a search that would exceed SEARCH_CAP
+//    columns has the row recomputed with the exact integer lower-envelope algorithm.
+// The masks are 1/8 byte per pixel, so nothing but the image and the result moves: 4096^2 nuclei mask
+// 44 us.  (With the vertical distances as a 16-bit plane, segments' carries, one pixel per lane
+// and 32-bit squares in the search, six launches: 190 us, of which the search 78, bound by its
+// instructions.)
 #include "common.hpp"
 
 namespace nsc {
@@ -22,90 +30,119 @@ namespace {
 constexpr int SEG = 64;
 constexpr uint16_t NONE = 0xFFFF;
 constexpr int SEARCH_CAP = 1024;
+constexpr int E_COLS = 64, E_HALO = 32, E_WIDE = E_COLS + 2 * E_HALO, E_THREADS = 256;
+constexpr int E_CAP = 63;  // largest g of the tile pass
 
-__global__ void k_zero_i32(int* p, int n) {
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-}
-
-// first / last zero row inside each segment of each column (-1 = none)
-__global__ void k_seg_zeros(const uint8_t* __restrict__ img, int w, int h, int nseg, int16_t* __restrict__ fz,
-                            int16_t* __restrict__ lz) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int sg = blockIdx.y;
+// zero pixels of 64 rows of a column, bit = row; the flags of the segment's rows are cleared for the
+// passes that follow
+__global__ __launch_bounds__(64) void k_edt_masks(const uint8_t* __restrict__ img, int w, int h, uint64_t* __restrict__ zm,
+                                                  int* __restrict__ rowflag) {
+    const int sg = blockIdx.y, y0 = sg * SEG, n = min(h, y0 + SEG) - y0;
+    if (blockIdx.x == 0 && (int)threadIdx.x < n) rowflag[y0 + threadIdx.x] = 0;
+    const int x = blockIdx.x * 64 + threadIdx.x;
     if (x >= w) return;
-    const int y0 = sg * SEG, n = min(h, y0 + SEG) - y0;
     // 64 loads in flight (rows past the image read the last row and are masked off), a bit per zero row
     uint32_t v[SEG];
 #pragma unroll
     for (int j = 0; j < SEG; ++j) v[j] = img[(size_t)min(y0 + j, h - 1) * w + x];
-    unsigned long long zm = 0;
+    uint32_t lo = 0, hi = 0;
 #pragma unroll
-    for (int j = 0; j < SEG; ++j) zm |= (unsigned long long)(v[j] == 0 && j < n) << j;
-    fz[(size_t)sg * w + x] = (int16_t)(zm ? __ffsll((long long)zm) - 1 : -1);
-    lz[(size_t)sg * w + x] = (int16_t)(zm ? 63 - __clzll((long long)zm) : -1);
+    for (int j = 0; j < 32; ++j) lo |= (v[j] == 0 ? 1u : 0u) << j;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) hi |= (v[32 + j] == 0 ? 1u : 0u) << j;
+    uint64_t m = (uint64_t)lo | (uint64_t)hi << 32;
+    if (n < SEG) m &= (1ull << n) - 1ull;
+    zm[(size_t)sg * w + x] = m;
 }
 
-// per column: row of the nearest zero strictly before / after each segment (-1 / INT_MAX-ish)
-__global__ void k_seg_carry(const int16_t* __restrict__ fz, const int16_t* __restrict__ lz, int w, int nseg,
-                            int32_t* __restrict__ above, int32_t* __restrict__ below) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= w) return;
-    // sixteen segments' entries loaded at a time (clamped indices), then scanned
-    constexpr int CH = 16;
-    int last = -1;
-    for (int s0 = 0; s0 < nseg; s0 += CH) {
-        int l[CH];
-#pragma unroll
-        for (int j = 0; j < CH; ++j) l[j] = lz[(size_t)min(s0 + j, nseg - 1) * w + x];
-#pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const int s = s0 + j;
-            if (s >= nseg) break;
-            above[(size_t)s * w + x] = last;
-            if (l[j] >= 0) last = s * SEG + l[j];
-        }
-    }
-    int first = -1;
-    for (int s1 = nseg - 1; s1 >= 0; s1 -= CH) {
-        int f[CH];
-#pragma unroll
-        for (int j = 0; j < CH; ++j) f[j] = fz[(size_t)max(s1 - j, 0) * w + x];
-#pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const int s = s1 - j;
-            if (s < 0) break;
-            below[(size_t)s * w + x] = first;
-            if (f[j] >= 0) first = s * SEG + f[j];
-        }
-    }
-}
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u16x2 pk(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
 
-__global__ void k_col_dist(const uint8_t* __restrict__ img, int w, int h, const int32_t* __restrict__ above,
-                           const int32_t* __restrict__ below, uint16_t* __restrict__ g) {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int sg = blockIdx.y;
-    if (x >= w) return;
-    const int y0 = sg * SEG, n = min(h, y0 + SEG) - y0;
-    // the segment's column at once: 64 loads in flight (rows past the image read the last row and
-    // are masked off), then a bit per zero row; each row's nearest zero above / below inside the
-    // segment is the highest set bit at or below it / the lowest at or above it
-    uint32_t v[SEG];
+__global__ __launch_bounds__(E_THREADS) void k_edt_tiles(const uint64_t* __restrict__ zm, int w, int h, int nseg,
+                                                      float* __restrict__ out, int* __restrict__ rowflag) {
+    __shared__ uint16_t G[SEG][E_WIDE];
+    const int sg = blockIdx.y, y0 = sg * SEG, x0 = blockIdx.x * E_COLS;
+    if (threadIdx.x < E_WIDE) {
+        const int x = x0 - E_HALO + (int)threadIdx.x;
+        // all three words from clamped (always valid) addresses; what lies outside the image holds no zero
+        const size_t xc = (size_t)clampi(x, 0, w - 1);
+        const uint64_t a = zm[(size_t)max(sg - 1, 0) * w + xc], m = zm[(size_t)sg * w + xc],
+                       b = zm[(size_t)min(sg + 1, nseg - 1) * w + xc];
+        const bool in = x >= 0 && x < w;
+        const uint64_t up = in && sg > 0 ? a : 0ull, own = in ? m : 0ull, dn = in && sg + 1 < nseg ? b : 0ull;
+        // distance of the row before the first to its nearest zero above it, of the row after the last below
+        uint32_t d = up ? (uint32_t)min((int)__clzll((long long)up), E_CAP) : (uint32_t)E_CAP;
+        uint32_t g[SEG];
 #pragma unroll
-    for (int j = 0; j < SEG; ++j) v[j] = img[(size_t)min(y0 + j, h - 1) * w + x];
-    unsigned long long zm = 0;
+        for (int j = 0; j < SEG; ++j) {
+            d = ((uint32_t)(own >> (j & 32)) >> (j & 31) & 1u) ? 0u : min(d + 1u, (uint32_t)E_CAP);
+            g[j] = d;
+        }
+        d = dn ? (uint32_t)min((int)__ffsll((long long)dn) - 1, E_CAP) : (uint32_t)E_CAP;
 #pragma unroll
-    for (int j = 0; j < SEG; ++j) zm |= (unsigned long long)(v[j] == 0 && j < n) << j;
-    const int up = above[(size_t)sg * w + x];  // row of the nearest zero above the segment (-1: none)
-    const int dn = below[(size_t)sg * w + x];  // row of the nearest zero below it (-1: none)
+        for (int j = SEG - 1; j >= 0; --j) {
+            d = min(d + 1u, g[j]);  // g[j] is 0 at a zero
+            G[j][threadIdx.x] = (uint16_t)d;
+        }
+    }
+    __syncthreads();
+    constexpr int NP = E_COLS / 2, STEP = E_THREADS / NP, K = 4;  // pairs per row, rows per step
+    const int c = 2 * ((int)threadIdx.x % NP), x = x0 + c;
+    for (int yb = (int)threadIdx.x / NP; yb < SEG; yb += K * STEP) {
+        if (y0 + yb - (int)threadIdx.x / NP >= h) break;  // the same for the whole workgroup
+        uint32_t lc[K], rc[K];
+        u16x2 best[K];
+        auto pair_at = [&](int k, int o) {
+            return *reinterpret_cast<const uint32_t*>(&G[yb + k * STEP][E_HALO + c + o]);  // 4-byte aligned
+        };
 #pragma unroll
-    for (int j = 0; j < SEG; ++j) {
-        if (j >= n) break;
-        const unsigned long long le = zm & (j == SEG - 1 ? ~0ull : ((2ull << j) - 1)), ge = zm >> j;
-        const int zu = le ? y0 + 63 - __clzll((long long)le) : up;
-        const int zd = ge ? y0 + j + __ffsll((long long)ge) - 1 : dn;
-        const int y = y0 + j;
-        const uint32_t du = zu >= 0 ? (uint32_t)(y - zu) : NONE, dd = zd >= 0 ? (uint32_t)(zd - y) : NONE;
-        g[(size_t)y * w + x] = (uint16_t)min(du, dd);
+        for (int k = 0; k < K; ++k) {
+            lc[k] = rc[k] = pair_at(k, 0);
+            best[k] = pk(lc[k]) * pk(lc[k]);
+        }
+        // two steps a turn: an odd one straddles the words of its even neighbours
+        for (int dx = 1; dx < E_HALO; dx += 2) {
+            u16x2 worst = best[0];
+#pragma unroll
+            for (int k = 1; k < K; ++k) worst = __builtin_elementwise_max(worst, best[k]);
+            const uint32_t b = __builtin_bit_cast(uint32_t, worst);
+            if (!__any((int)max(b & 0xFFFFu, b >> 16) > dx * dx)) break;
+            uint32_t ln[K], rn[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                ln[k] = pair_at(k, -dx - 1);
+                rn[k] = pair_at(k, dx + 1);
+            }
+            const unsigned short s1 = (unsigned short)(dx * dx), s2 = (unsigned short)((dx + 1) * (dx + 1));
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const u16x2 m1 = __builtin_elementwise_min(pk(lc[k] << 16 | ln[k] >> 16), pk(rc[k] >> 16 | rn[k] << 16));
+                const u16x2 m2 = __builtin_elementwise_min(pk(ln[k]), pk(rn[k]));
+                best[k] = __builtin_elementwise_min(best[k], m1 * m1 + u16x2{s1, s1});
+                best[k] = __builtin_elementwise_min(best[k], m2 * m2 + u16x2{s2, s2});
+                lc[k] = ln[k];
+                rc[k] = rn[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int y = y0 + yb + k * STEP;
+            if (y >= h || x >= w) continue;
+            const uint32_t b = __builtin_bit_cast(uint32_t, best[k]), d0 = b & 0xFFFFu, d1 = b >> 16;
+            float* const o = out + (size_t)y * w + x;
+            // the squared distance is an integer below 2^24: one exact float whatever dx and g it came from
+            const float f0 = d0 <= E_HALO * E_HALO ? sqrtf((float)d0) : -1.0f;
+            const float f1 = d1 <= E_HALO * E_HALO ? sqrtf((float)d1) : -1.0f;
+            bool far = f0 < 0.0f;
+            if (x + 1 < w) {
+                const float2 f = make_float2(f0, f1);
+                __builtin_memcpy(o, &f, 8);
+                far = far || f1 < 0.0f;
+            } else {
+                o[0] = f0;
+            }
+            if (far) rowflag[y] = 1;
+        }
     }
 }
 
@@ -114,17 +151,37 @@ __device__ __forceinline__ float edt_value(long long dx2, long long g) {
     return sqrtf((float)dx2 + fg);
 }
 
-__global__ __launch_bounds__(256) void k_row_search(const uint16_t* __restrict__ g, int w, int h, float* __restrict__ out,
-                                                    int* __restrict__ fallback_rows, int* __restrict__ nfallback) {
-    extern __shared__ uint16_t grow[];
+__global__ __launch_bounds__(256) void k_edt_rows(const uint64_t* __restrict__ zm, int w, int h, int nseg,
+                                                  float* __restrict__ out, const int* __restrict__ rowflag) {
+    extern __shared__ uint16_t lds[];
     const int y = blockIdx.x;
-    const uint16_t* gr = g + (size_t)y * w;
-    for (int x = threadIdx.x; x < w; x += blockDim.x) grow[x] = gr[x];
-    __syncthreads();
-    __shared__ int need;
+    if (!rowflag[y]) return;
+    uint16_t* const grow = lds;  // vertical distances of the row (NONE: no zero in the column)
+    const int sg = y / SEG, j = y % SEG;
+    for (int x = threadIdx.x; x < w; x += blockDim.x) {
+        const uint64_t m = zm[(size_t)sg * w + x], le = m & ((2ull << j) - 1ull), ge = m >> j;
+        uint32_t du = NONE, dd = NONE;
+        if (le) du = (uint32_t)(j - 63 + (int)__clzll((long long)le));
+        else
+            for (int s = sg - 1; s >= 0; --s)
+                if (const uint64_t q = zm[(size_t)s * w + x]) {
+                    du = (uint32_t)(y - (s * SEG + 63 - (int)__clzll((long long)q)));
+                    break;
+                }
+        if (ge) dd = (uint32_t)__ffsll((long long)ge) - 1u;
+        else
+            for (int s = sg + 1; s < nseg; ++s)
+                if (const uint64_t q = zm[(size_t)s * w + x]) {
+                    dd = (uint32_t)(s * SEG + (int)__ffsll((long long)q) - 1 - y);
+                    break;
+                }
+        grow[x] = (uint16_t)min(du, dd);
+    }
+    __shared__ int need, kk;
     if (threadIdx.x == 0) need = 0;
     __syncthreads();
     for (int x = threadIdx.x; x < w; x += blockDim.x) {
+        if (!(out[(size_t)y * w + x] < 0.0f)) continue;
         // squared distances in 32 bits, exactly: g <= 65534 so g^2 < 2^32 and UINT_MAX marks "no
         // zero"; a candidate dx^2 + v^2 is compared as v^2 < best - dx^2 (dx^2 < best), which can
         // neither overflow nor underflow, and a winner is below the old best
@@ -147,7 +204,7 @@ __global__ __launch_bounds__(256) void k_row_search(const uint16_t* __restrict__
                     if (v != NONE && v * v < best - dx2) { best = dx2 + v * v; bdx = dx; bg = v; }
                 }
             }
-            if (dx == SEARCH_CAP + 1) need = 1;  // search cut short: exact envelope later
+            if (dx == SEARCH_CAP + 1) need = 1;  // search cut short: exact envelope below
         }
         float o;
         if (best == UINT_MAX) o = sqrtf(1e15f);
@@ -155,25 +212,16 @@ __global__ __launch_bounds__(256) void k_row_search(const uint16_t* __restrict__
         out[(size_t)y * w + x] = o;
     }
     __syncthreads();
-    if (threadIdx.x == 0 && need) fallback_rows[atomicAdd(nfallback, 1)] = y;
-}
-
-// exact lower envelope of the parabolas (x - p)^2 + g(p)^2 over the columns with a zero
-// (Felzenszwalb-Huttenlocher with exact integer intersection tests); one workgroup per flagged
-// row, the apex stack in LDS, built by one lane and evaluated by all
-__global__ __launch_bounds__(256) void k_row_envelope(const uint16_t* __restrict__ g, int w, int h, float* __restrict__ out,
-                                                      const int* __restrict__ rows, const int* __restrict__ nrows) {
-    extern __shared__ int v[];
-    __shared__ int kk;
-    if ((int)blockIdx.x >= min(*nrows, h)) return;
-    const int y = rows[blockIdx.x];
-    if (y < 0 || y >= h) return;
-    const uint16_t* gr = g + (size_t)y * w;
-    auto f = [&](int p) { return (long long)gr[p] * gr[p]; };
+    if (!need) return;
+    // exact lower envelope of the parabolas (x - p)^2 + g(p)^2 over the columns with a zero
+    // (Felzenszwalb-Huttenlocher with exact integer intersection tests), the apex stack in LDS (a column
+    // fits 16 bits), built by one lane and evaluated by all
+    uint16_t* const v = lds + w;
+    auto f = [&](int p) { return (long long)grow[p] * grow[p]; };
     if (threadIdx.x == 0) {
         int k = -1;
         for (int q = 0; q < w; ++q) {
-            if (gr[q] == NONE) continue;
+            if (grow[q] == NONE) continue;
             while (k >= 1) {
                 const int p = v[k], r = v[k - 1];
                 // drop p when the (r, q) intersection is not right of the (r, p) intersection
@@ -182,7 +230,7 @@ __global__ __launch_bounds__(256) void k_row_envelope(const uint16_t* __restrict
                 if (nq * (long long)(p - r) <= np * (long long)(q - r)) --k;
                 else break;
             }
-            v[++k] = q;
+            v[++k] = (uint16_t)q;
         }
         kk = k;
     }
@@ -201,7 +249,7 @@ __global__ __launch_bounds__(256) void k_row_envelope(const uint16_t* __restrict
             else hi = mid;
         }
         const int p = v[lo];
-        out[(size_t)y * w + x] = edt_value((long long)(x - p) * (x - p), gr[p]);
+        out[(size_t)y * w + x] = edt_value((long long)(x - p) * (x - p), grow[p]);
     }
 }
 
@@ -218,40 +266,21 @@ int edt_impl(const uint8_t* img, float* out, int w, int h, hipStream_t s) {
         return NSC_ERR_LIMIT;
     }
     const int nseg = (int)cdiv(h, SEG);
-    const size_t n = (size_t)w * h;
-    auto carve = [&](Carver& c, int32_t*& above, int32_t*& below, int*& rows, int*& nrows, uint16_t*& g, int16_t*& fz,
-                     int16_t*& lz) {
-        above = c.take<int32_t>((size_t)nseg * w);
-        below = c.take<int32_t>((size_t)nseg * w);
-        rows = c.take<int>(h);
-        nrows = c.take<int>(1);
-        g = c.take<uint16_t>(n);
-        fz = c.take<int16_t>((size_t)nseg * w);
-        lz = c.take<int16_t>((size_t)nseg * w);
-    };
-    int32_t *above, *below;
-    int *rows, *nrows;
-    uint16_t* g;
-    int16_t *fz, *lz;
     Carver measure(nullptr);
-    carve(measure, above, below, rows, nrows, g, fz, lz);
+    measure.take<uint64_t>((size_t)nseg * w);
+    measure.take<int>(h);
     Scratch sc;
     NSC_CHECK(sc.alloc(measure.size(), s));
     Carver cut(sc.p);
-    carve(cut, above, below, rows, nrows, g, fz, lz);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, nrows, 1);
-    dim3 gb(cdiv(w, 64), nseg);
-    hipLaunchKernelGGL(k_seg_zeros, gb, dim3(64), 0, s, img, w, h, nseg, fz, lz);
-    hipLaunchKernelGGL(k_seg_carry, dim3(cdiv(w, 64)), dim3(64), 0, s, fz, lz, w, nseg, above, below);
-    hipLaunchKernelGGL(k_col_dist, gb, dim3(64), 0, s, img, w, h, above, below, g);
-    const size_t lds = sizeof(uint16_t) * w;
-    hipLaunchKernelGGL(k_row_search, dim3(h), dim3(256), lds, s, g, w, h, out, rows, nrows);
-    // rows whose search was cut short (distances beyond SEARCH_CAP): exact envelope; the launch
-    // is unconditional and its blocks beyond the flagged count exit at once (no host sync)
-    const size_t lds2 = sizeof(int) * w;
-    if (lds2 > 64 * 1024) NSC_HIP(hipFuncSetAttribute((const void*)k_row_envelope,
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2));
-    hipLaunchKernelGGL(k_row_envelope, dim3(h), dim3(256), lds2, s, g, w, h, out, rows, nrows);
+    uint64_t* zm = cut.take<uint64_t>((size_t)nseg * w);
+    int* rowflag = cut.take<int>(h);
+    hipLaunchKernelGGL(k_edt_masks, dim3(cdiv(w, 64), nseg), dim3(64), 0, s, img, w, h, zm, rowflag);
+    hipLaunchKernelGGL(k_edt_tiles, dim3(cdiv(w, E_COLS), nseg), dim3(E_THREADS), 0, s, zm, w, h, nseg, out, rowflag);
+    // the launch is unconditional and the workgroups of unflagged rows leave at once (no host sync)
+    const size_t lds = 2 * sizeof(uint16_t) * (size_t)w;
+    if (lds > 64 * 1024)
+        NSC_HIP(hipFuncSetAttribute((const void*)k_edt_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_edt_rows, dim3(h), dim3(256), lds, s, zm, w, h, nseg, out, rowflag);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
 }
