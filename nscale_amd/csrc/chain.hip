@@ -25,7 +25,6 @@ int fill_holes_impl(const uint8_t* img, uint8_t* out, int w, int h, int conn, in
 int bwselect_impl(const uint8_t* bw, const uint8_t* seeds, uint8_t* out, int w, int h, int conn, int32_t* labels,
                   uint8_t* flag, hipStream_t s);
 int edt_impl(const uint8_t* img, float* out, int w, int h, hipStream_t s);
-int imhmin_impl(const float* img, float* out, int w, int h, float hval, int conn, float* s1, float* s2, hipStream_t s);
 int local_max_impl(const float* img, uint8_t* out, int w, int h, int conn, bool minima, void* scratch, hipStream_t s);
 size_t local_max_scratch(int w, int h);
 size_t ws2_scratch(int w, int h);
@@ -147,31 +146,26 @@ __global__ void k_norbc(uint8_t* __restrict__ seg, const uint8_t* __restrict__ r
     }
 }
 
-// dist -> distance (HE.cpp:366-374) -> imhmin operands mask = -distance, marker = mask - 1
-// (MO.cpp:3355-3356); nuclei = img masked by seg_big (HE.cpp:407)
+// nuclei = img masked by seg_big (HE.cpp:407); distance = -dist inside, -FLT_MAX outside (HE.cpp:366-374),
+// for the stage dump only
 __global__ void k_dist_prep(const float* __restrict__ dist, const uint8_t* __restrict__ seg_big,
                             const uint8_t* __restrict__ bgr, size_t n, float* __restrict__ distance,
-                            float* __restrict__ hmask, float* __restrict__ hmarker, uint8_t* __restrict__ nuclei) {
+                            uint8_t* __restrict__ nuclei) {
     // every load unconditional, then selects (a load under the mask's condition compiles to a
     // branch around it, and the loads of a pixel then wait for one another)
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         const uint8_t sb = seg_big[i];
-        const float dv = dist[i];
         const uint8_t c0 = bgr[3 * i], c1 = bgr[3 * i + 1], c2 = bgr[3 * i + 2];
         const bool f = sb != 0;
-        const float d = f ? -dv : -FLT_MAX;
-        if (distance) distance[i] = d;
-        const float m = -d;
-        hmask[i] = m;
-        hmarker[i] = m - 1.0f;
+        if (distance) distance[i] = f ? -dist[i] : -FLT_MAX;
         nuclei[3 * i] = f ? c0 : 0;
         nuclei[3 * i + 1] = f ? c1 : 0;
         nuclei[3 * i + 2] = f ? c2 : 0;
     }
 }
 
-__global__ void k_negate_f(float* a, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) a[i] = -a[i];
+__global__ void k_negate_f(const float* __restrict__ a, float* __restrict__ out, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) out[i] = -a[i];
 }
 
 // seg_nonoverlap = seg_big where watermask >= 0  (HE.cpp:423-424)
@@ -197,7 +191,7 @@ struct Workspace {
         *seg_nohole, *seg_open, *seg_big_t, *seg_big, *nonov, *seg, *fin, *tmp8, *nuclei;
     // 32-bit planes
     int32_t *L, *area, *wm;
-    float *dist, *distance, *hmask, *hmarker, *d2;
+    float *dist, *distance, *d2;
     void* big;  // shared by local minima and the watershed (max of their scratch)
     int* counts;  // [0] background, [1] compcount S1, [2] compcount final-area, [3] ncomp
     Arena arena;  // operator scratch during a chain call (separate allocation)
@@ -212,7 +206,7 @@ static size_t big_scratch(int w, int h) { return al256(std::max(local_max_scratc
 
 size_t workspace_bytes(int mw, int mh) {
     const size_t n = (size_t)mw * mh;
-    return 23 * al256(n) + al256(3 * n) + 8 * al256(4 * n) + big_scratch(mw, mh) + 256;
+    return 23 * al256(n) + al256(3 * n) + 6 * al256(4 * n) + big_scratch(mw, mh) + 256;
 }
 
 size_t workspace_arena_bytes(int mw, int mh) { return kArenaPerPx * (size_t)mw * mh + ((size_t)64 << 20); }
@@ -245,8 +239,6 @@ static int ws_alloc(Workspace& W, int mw, int mh) {
     W.wm = reinterpret_cast<int32_t*>(p); p += i32;
     W.dist = reinterpret_cast<float*>(p); p += i32;
     W.distance = reinterpret_cast<float*>(p); p += i32;
-    W.hmask = reinterpret_cast<float*>(p); p += i32;
-    W.hmarker = reinterpret_cast<float*>(p); p += i32;
     W.d2 = reinterpret_cast<float*>(p); p += i32;
     W.big = p; p += big;
     W.counts = reinterpret_cast<int*>(p);
@@ -458,16 +450,20 @@ int stage_a4(Chain& C, const uint8_t* bgr, const uint8_t* seg_open, bool binary,
     NSC_CHECK(edt_impl(W.seg_big, W.dist, w, h, s));  // HE.cpp:359
     NSC_CHECK(C.save(16, W.dist, 4 * n));
     hipLaunchKernelGGL(k_dist_prep, grid1(n), dim3(256), 0, s, W.dist, W.seg_big, bgr, n, C.want(17) ? W.distance : nullptr,
-                       W.hmask, W.hmarker, W.nuclei);
+                       W.nuclei);
     NSC_CHECK(C.save(17, W.distance, 4 * n));
     C.mark(16);
-    NSC_CHECK(recon_impl<float>(W.hmarker, W.hmask, W.d2, w, h, 8, s));  // imhmin(distance, 1, 8) HE.cpp:384
-    hipLaunchKernelGGL(k_negate_f, grid1(n), dim3(256), 0, s, W.d2, n);
-    NSC_CHECK(C.save(18, W.d2, 4 * n));
+    // distance2 = imhmin(distance, 1, 8) (HE.cpp:384), kept negated: -distance is dist, with FLT_MAX in
+    // the background, where dist is 0; distance2's minima are the maxima of its negation
+    NSC_CHECK(recon_hdome_impl(W.dist, W.d2, w, h, 8, 1.0f, false, true, s));
+    if (C.want(18)) {
+        hipLaunchKernelGGL(k_negate_f, grid1(n), dim3(256), 0, s, W.d2, W.distance, n);
+        NSC_CHECK(C.save(18, W.distance, 4 * n));
+    }
     NSC_CHECK(C.save(19, W.nuclei, 3 * n));
     C.mark(18);
     // watershed2(nuclei, distance2, watershedConnectivity)  HE.cpp:414
-    NSC_CHECK(local_max_impl(W.d2, W.tmp8, w, h, wsConn, true, W.big, s));
+    NSC_CHECK(local_max_impl(W.d2, W.tmp8, w, h, wsConn, false, W.big, s));
     NSC_CHECK(ccl_u8(W.tmp8, W.L, w, h, wsConn, -1, true, s));
     NSC_CHECK(ws2_from_labels(W.nuclei, W.L, W.wm, w, h, W.big, s));
     NSC_CHECK(C.save(20, W.wm, 4 * n));

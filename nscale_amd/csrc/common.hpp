@@ -302,5 +302,10 @@ template <typename T>
 int recon_impl(const T* marker, const T* mask, T* out, int w, int h, int conn, hipStream_t s);
 template <typename T>
 int recon_batched_impl(const nsc_recon_desc* d, int n, hipStream_t s);
+// reconstruction of m - depth under m for m = img, -img (negate; the result is negated too) or img with
+// FLT_MAX at its zeros (zero_max), without planes for m and m - depth
+int recon_hdome_impl(const float* img, float* out, int w, int h, int conn, float depth, bool negate, bool zero_max,
+                     hipStream_t s);
+int recon_hmin_batched_impl(const nsc_recon_desc* d, int n, float depth, hipStream_t s);
 
 }  // namespace nsc

@@ -26,6 +26,7 @@
 //    the GPU keeps working during the round trip.
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
 #include <climits>
 #include <cstdlib>
 #include <cstring>
@@ -103,7 +104,20 @@ struct RImg {
     T* out;
     int w, h, tiles_x, tiles_y, conn, base;
     int rgx, rgy;  // region grid (G x G windows per region) of the launch; base counts regions
+    // derived form (HDome windows): one image in place of marker and mask, see HDome
+    uint32_t in_flip, out_flip;
+    float depth;
+    int zero_max;
 };
+
+// Reconstruction of m - depth under m, where m is made of one float image as it is loaded: the image
+// with its sign flipped (in_flip), or with FLT_MAX in place of its zeros (zero_max); the result is
+// stored with its sign flipped by out_flip.  This is imhmin and the first step of the local extrema
+// without the planes of m, of m - depth and of the unflipped result (20 bytes per pixel and two passes
+// over them).
+__device__ __forceinline__ float flip_sign(float v, uint32_t flip) {
+    return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) ^ flip);
+}
 
 template <typename T>
 struct RShared {
@@ -276,7 +290,7 @@ __device__ __forceinline__ auto col_sum(const R (&v)[TH]) {
 }
 
 // one tile of one image: load window, sweep to stability, write owned pixels, mark neighbours
-template <typename T, int CONN>
+template <typename T, int CONN, bool HD = false>
 __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass, RShared<T>& sh, int* __restrict__ next_list,
                                            int* __restrict__ next_count, unsigned* __restrict__ stamp,
                                            unsigned long long* dirty = nullptr) {
@@ -304,7 +318,7 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
     // every lane loads from a clamped (always valid) address so that the 128 loads of the window
     // issue back to back; pixels outside the image are replaced by the frame value afterwards
     const auto gmask = as_global(mask);
-    const auto gsrc = as_global(pass == 0 ? marker : (const T*)out);
+    const auto gsrc = as_global(pass == 0 ? (HD ? mask : marker) : (const T*)out);
     const size_t gxc = (size_t)clampi(gx, 0, w - 1);
     // 16 rows at a time: all 32 loads of a chunk are issued before any of them is used (the
     // scheduling fences stop the compiler from sinking loads to their uses)
@@ -323,6 +337,11 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
             const int y = c + j, gy = ty * OH - 1 + y;
             const bool inb = col_in && gy >= 0 && gy < h;
             const uint32_t keep = inb ? ~0u : 0u;
+            if constexpr (HD) {
+                const bool z = im.zero_max && m_ld[j] == 0.0f;
+                m_ld[j] = z ? FLT_MAX : flip_sign(m_ld[j], im.in_flip);
+                s_ld[j] = pass == 0 ? m_ld[j] - im.depth : flip_sign(s_ld[j], im.out_flip);
+            }
             const R mk = keep_bits(m_ld[j], keep);
             const R val = keep_bits(smin(s_ld[j], m_ld[j]), keep);
             const bool frozen = col_frozen || y == 0 || y == TH - 1 || !inb;
@@ -374,7 +393,10 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
 #pragma unroll
         for (int y = 1; y < TH - 1; ++y) {
             const int gy = ty * OH - 1 + y;
-            if (gy < h) gcol[(size_t)gy * w] = (T)v[y];
+            if (gy < h) {
+                if constexpr (HD) gcol[(size_t)gy * w] = flip_sign(v[y], im.out_flip);
+                else gcol[(size_t)gy * w] = (T)v[y];
+            }
         }
     }
     // ---- owned-border changes -> mark neighbours ----
@@ -406,7 +428,7 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
 // Pass 0 runs every tile of every image; pass k > 0 runs the tiles listed by pass k - 1.  Blocks
 // stride over their work; a batch's images are found through tile_img (global tile -> image).
 // CONN 0 = per-image connectivity.
-template <typename T, int CONN>
+template <typename T, int CONN, bool HD = false>
 __device__ __forceinline__ void recon_tiles_body(RShared<T>& sh, const RImg<T>* __restrict__ imgs, const RImg<T>& one,
                                                  const int* __restrict__ tile_img, int ntiles, const int* __restrict__ list,
                                                  const int* __restrict__ list_count, int* __restrict__ next_list,
@@ -420,22 +442,22 @@ __device__ __forceinline__ void recon_tiles_body(RShared<T>& sh, const RImg<T>* 
         const RImg<T> im = imgs ? imgs[tile_img[g]] : one;
         const int local = g - im.base;
         if (CONN == 8 || (CONN == 0 && im.conn == 8))
-            recon_tile<T, 8>(im, local, pass, sh, next_list, next_count, stamp, dirty);
+            recon_tile<T, 8, HD>(im, local, pass, sh, next_list, next_count, stamp, dirty);
         else
-            recon_tile<T, 4>(im, local, pass, sh, next_list, next_count, stamp, dirty);
+            recon_tile<T, 4, HD>(im, local, pass, sh, next_list, next_count, stamp, dirty);
         __syncthreads();  // the shared window is reused by the next tile
     }
 }
 
-template <typename T, int CONN>
+template <typename T, int CONN, bool HD>
 __global__ __launch_bounds__(64, RECON_WAVES) void recon_tiles(const RImg<T>* __restrict__ imgs, RImg<T> one, const int* __restrict__ tile_img,
                                                   int ntiles, const int* __restrict__ list, const int* __restrict__ list_count,
                                                   int* __restrict__ next_list, int* __restrict__ next_count,
                                                   int* __restrict__ clear_count, unsigned* __restrict__ stamp, int pass,
                                                   unsigned long long* __restrict__ dirty) {
     __shared__ RShared<T> sh;
-    recon_tiles_body<T, CONN>(sh, imgs, one, tile_img, ntiles, list, list_count, next_list, next_count, clear_count, stamp,
-                              pass, dirty);
+    recon_tiles_body<T, CONN, HD>(sh, imgs, one, tile_img, ntiles, list, list_count, next_list, next_count, clear_count,
+                                  stamp, pass, dirty);
 }
 
 // ---- the residual wavefront as a device-side work queue ----------------------------------------
@@ -786,8 +808,8 @@ static void launch_pass(int grid, hipStream_t s, const RImg<T>* imgs_dev, const 
                         const int* lst, const int* cnt, int* nl, int* nc, int* clr, unsigned* stamp, int pass,
                         unsigned long long* dirty = nullptr) {
     if (G == 1)
-        hipLaunchKernelGGL((recon_tiles<T, CONN>), dim3(grid), dim3(64), 0, s, imgs_dev, one, tile_img, nt, lst, cnt, nl, nc,
-                           clr, stamp, pass, dirty);
+        hipLaunchKernelGGL((recon_tiles<T, CONN, false>), dim3(grid), dim3(64), 0, s, imgs_dev, one, tile_img, nt, lst, cnt,
+                           nl, nc, clr, stamp, pass, dirty);
     else
         hipLaunchKernelGGL((recon_regions<T, CONN, G>), dim3(grid), dim3(64 * G * G), 0, s, imgs_dev, one, tile_img, nt, lst,
                            cnt, nl, nc, clr, stamp, pass);
@@ -799,6 +821,22 @@ static void launch_conn(int conn, int grid, hipStream_t s, const RImg<T>* imgs_d
     if (conn == 8) launch_pass<T, 8, G>(grid, s, imgs_dev, one, tile_img, nt, lst, cnt, nl, nc, clr, stamp, pass);
     else if (conn == 4) launch_pass<T, 4, G>(grid, s, imgs_dev, one, tile_img, nt, lst, cnt, nl, nc, clr, stamp, pass);
     else launch_pass<T, 0, G>(grid, s, imgs_dev, one, tile_img, nt, lst, cnt, nl, nc, clr, stamp, pass);
+}
+
+// the derived form's pass (one-window regions)
+static void launch_hdome(int conn, int grid, hipStream_t s, const RImg<float>* imgs_dev, const RImg<float>& one,
+                         const int* tile_img, int nt, const int* lst, const int* cnt, int* nl, int* nc, int* clr,
+                         unsigned* stamp, int pass) {
+    unsigned long long* const none = nullptr;
+    if (conn == 8)
+        hipLaunchKernelGGL((recon_tiles<float, 8, true>), dim3(grid), dim3(64), 0, s, imgs_dev, one, tile_img, nt, lst, cnt,
+                           nl, nc, clr, stamp, pass, none);
+    else if (conn == 4)
+        hipLaunchKernelGGL((recon_tiles<float, 4, true>), dim3(grid), dim3(64), 0, s, imgs_dev, one, tile_img, nt, lst, cnt,
+                           nl, nc, clr, stamp, pass, none);
+    else
+        hipLaunchKernelGGL((recon_tiles<float, 0, true>), dim3(grid), dim3(64), 0, s, imgs_dev, one, tile_img, nt, lst, cnt,
+                           nl, nc, clr, stamp, pass, none);
 }
 
 // largest region side the workgroup's LDS holds for the element type
@@ -902,7 +940,7 @@ static bool drain_enabled() {
     return d < 0 ? drain_env() : d != 0;
 }
 
-template <typename T>
+template <typename T, bool HD = false>
 static int recon_passes(const RImg<T>* imgs_dev, const RImg<T>& one, const int* tile_img, int nt, long long pixels, int conn,
                         int G, const ReconBufs& B, hipStream_t s) {
     const long long max_pass = pass_limit(pixels);
@@ -913,6 +951,10 @@ static int recon_passes(const RImg<T>* imgs_dev, const RImg<T>& one, const int* 
         // a serving thread's later passes run on at most 1024 workgroups that loop over the list:
         // beside the other slots' kernels, a pass's idle workgroups only wait for CUs
         const int grid = pass == 0 || !thread_serving() ? grid0 : std::min(grid0, 1024);
+        if constexpr (HD) {
+            launch_hdome(conn, grid, s, imgs_dev, one, tile_img, nt, lst, cnt, nl, nc, clr, stamp, pass);
+            return;
+        }
         switch (G) {
             case 2: launch_conn<T, 2>(conn, grid, s, imgs_dev, one, tile_img, nt, lst, cnt, nl, nc, clr, stamp, pass); break;
             case 3: launch_conn<T, (max_region<T>() >= 3 ? 3 : 2)>(conn, grid, s, imgs_dev, one, tile_img, nt, lst, cnt, nl,
@@ -1042,22 +1084,38 @@ static void set_regions(RImg<T>& r, int G) {
 
 template <typename T>
 int recon_impl(const T* marker, const T* mask, T* out, int w, int h, int conn, hipStream_t s) {
-    RImg<T> one{marker, mask, out, w, h, (int)cdiv(w, OW), (int)cdiv(h, OH), conn, 0, 0, 0};
+    RImg<T> one{marker, mask, out, w, h, (int)cdiv(w, OW), (int)cdiv(h, OH), conn, 0, 0, 0, 0, 0, 0.0f, 0};
     const int G = region_side<T>();
     set_regions(one, G);
     return recon_run_scratch<T>(nullptr, one, nullptr, one.rgx * one.rgy, (long long)w * h, conn, G, s);
 }
 
+// The derived form of one image (see HDome above flip_sign): out = the reconstruction, its sign
+// flipped when `negate`.
+int recon_hdome_impl(const float* img, float* out, int w, int h, int conn, float depth, bool negate, bool zero_max,
+                     hipStream_t s) {
+    const uint32_t flip = negate ? 0x80000000u : 0u;
+    RImg<float> one{nullptr, img, out, w, h, (int)cdiv(w, OW), (int)cdiv(h, OH), conn, 0, 0, 0, flip, flip, depth, zero_max};
+    set_regions(one, 1);
+    const int nt = one.rgx * one.rgy;
+    Scratch sc;
+    NSC_CHECK(sc.alloc(recon_scratch_bytes(nt), s));
+    const ReconBufs B = recon_carve(sc.p, nt);
+    recon_clear(B, s);
+    return recon_passes<float, true>(nullptr, one, nullptr, nt, (long long)w * h, conn, 1, B, s);
+}
+
 // A batch of images in one launch per pass: the image table and the tile -> image map live in
-// stream-ordered scratch.  conn: 4 or 8 for the whole batch, 0 = per image.
-template <typename T>
-int recon_batched_impl(const nsc_recon_desc* d, int n, hipStream_t s) {
+// stream-ordered scratch.  conn: 4 or 8 for the whole batch, 0 = per image.  HD: the derived form of
+// every image (mask = the image, no marker) with `depth`, signs flipped both ways (imhmin).
+template <typename T, bool HD>
+static int recon_batched_run(const nsc_recon_desc* d, int n, float depth, hipStream_t s) {
     std::vector<RImg<T>> imgs(n);
     long long nt = 0, pixels = 0;
     int conn_all = d[0].conn;
-    const int G = region_side<T>();
+    const int G = HD ? 1 : region_side<T>();
     for (int i = 0; i < n; ++i) {
-        NSC_ARG(d[i].marker && d[i].mask && d[i].out && d[i].w > 0 && d[i].h > 0 && (d[i].conn == 4 || d[i].conn == 8),
+        NSC_ARG((HD || d[i].marker) && d[i].mask && d[i].out && d[i].w > 0 && d[i].h > 0 && (d[i].conn == 4 || d[i].conn == 8),
                 "imreconstruct batched: descriptor");
         RImg<T>& r = imgs[i];
         r.marker = static_cast<const T*>(d[i].marker);
@@ -1069,6 +1127,9 @@ int recon_batched_impl(const nsc_recon_desc* d, int n, hipStream_t s) {
         r.tiles_y = (int)cdiv(r.h, OH);
         r.conn = d[i].conn;
         r.base = (int)nt;
+        r.in_flip = r.out_flip = HD ? 0x80000000u : 0u;
+        r.depth = depth;
+        r.zero_max = 0;
         set_regions(r, G);
         nt += (long long)r.rgx * r.rgy;
         pixels += (long long)r.w * r.h;
@@ -1085,10 +1146,27 @@ int recon_batched_impl(const nsc_recon_desc* d, int n, hipStream_t s) {
     int* tile_dev = reinterpret_cast<int*>(static_cast<char*>(tab.p) + ib);
     NSC_HIP(hipMemcpyAsync(imgs_dev, imgs.data(), sizeof(RImg<T>) * n, hipMemcpyHostToDevice, s));
     NSC_HIP(hipMemcpyAsync(tile_dev, tile_img.data(), sizeof(int) * (size_t)nt, hipMemcpyHostToDevice, s));
-    const int rc = recon_run_scratch<T>(imgs_dev, imgs[0], tile_dev, (int)nt, pixels, conn_all, G, s);
+    int rc;
+    if constexpr (HD) {
+        Scratch sc;
+        NSC_CHECK(sc.alloc(recon_scratch_bytes((int)nt), s));
+        const ReconBufs B = recon_carve(sc.p, (int)nt);
+        recon_clear(B, s);
+        rc = recon_passes<float, true>(imgs_dev, imgs[0], tile_dev, (int)nt, pixels, conn_all, 1, B, s);
+    } else {
+        rc = recon_run_scratch<T>(imgs_dev, imgs[0], tile_dev, (int)nt, pixels, conn_all, G, s);
+    }
     // the host tables must outlive the copies (pageable copies complete before returning; be explicit)
     NSC_HIP(stream_sync(s));
     return rc;
+}
+
+template <typename T>
+int recon_batched_impl(const nsc_recon_desc* d, int n, hipStream_t s) {
+    return recon_batched_run<T, false>(d, n, 0.0f, s);
+}
+int recon_hmin_batched_impl(const nsc_recon_desc* d, int n, float depth, hipStream_t s) {
+    return recon_batched_run<float, true>(d, n, depth, s);
 }
 
 template int recon_impl<uint8_t>(const uint8_t*, const uint8_t*, uint8_t*, int, int, int, hipStream_t);
@@ -1358,7 +1436,7 @@ extern "C" int nsc_imreconstruct_u8_noalloc(const uint8_t* marker, const uint8_t
     using namespace nsc;
     NSC_ARG(marker && mask && out && w > 0 && h > 0 && valid_conn(conn), "imreconstruct_u8_noalloc");
     NSC_CHECK(ensure_init());
-    RImg<uint8_t> one{marker, mask, out, w, h, (int)cdiv(w, OW), (int)cdiv(h, OH), conn, 0, 0, 0};
+    RImg<uint8_t> one{marker, mask, out, w, h, (int)cdiv(w, OW), (int)cdiv(h, OH), conn, 0, 0, 0, 0, 0, 0.0f, 0};
     const int G = region_side<uint8_t>();
     set_regions(one, G);
     const long long nt = (long long)one.rgx * one.rgy;
