@@ -57,31 +57,19 @@ struct Dev {
     const uint8_t* cls;
     const uint16_t* lvl0;
     const int32_t* run;  // canonical run id (1..R) for F pixels
-    // F items (indexed by pixel)
-    uint8_t* st;     // 0 none, 1 queued, 2 popped
-    uint8_t* ilvl;
-    int32_t* pseq;
-    int32_t* parent;  // pusher pixel, -1 = initial push
-    int32_t* bnode;   // item id
-    int32_t* popidx;
-    int32_t* lab;     // label decided in the run's flood
-    int32_t* qnext;   // FIFO links, indexed by item id
+    // Items: id < N is an F pixel or a B pixel queued in the initial scan, id >= N a leaf slot.  A record is
+    // written when the item is queued, its pop index when it pops; records of other ids hold anything.
+    // {run, largest-key item of the push chain, level << 24 | pop index, pusher (pixel, -1 = initial push)}
+    int4* wr;
+    int32_t* lab;  // F pixel: label decided in its run's flood, 0 = never queued there
+    int32_t* qnext;  // FIFO links of the global-memory floods, indexed by item id
     // leaves
-    int32_t* head;    // per B pixel: first leaf slot or -1
+    int32_t* head;  // per B pixel: first leaf slot or -1
     int32_t* lf_b;
-    int32_t* lf_run;
-    uint8_t* lf_lvl;
-    int32_t* lf_pseq;
-    int32_t* lf_parent;
-    int32_t* lf_bnode;
-    int32_t* lf_popidx;
     int32_t* lf_next;
     int* nleaf;
     int leafcap;
     int* flags;
-    // per item, packed after phase 1 for the pop-order walks: {run, bnode, popidx, parent} and level
-    int4* wr;
-    uint8_t* wl;
 };
 
 // A value every lane of the wave holds (or the one active lane's), as a wave-uniform value: the
@@ -106,31 +94,23 @@ __device__ __forceinline__ int c_diff(const uint8_t* a, const uint8_t* b) {
     return max(max(db, dg), dr);
 }
 
-// ---- item accessors: id < N -> F pixel or initially queued B pixel; id >= N -> leaf slot ----
-__device__ __forceinline__ int it_lvl(const Dev& D, int x) {
-    if (x >= D.N) return D.lf_lvl[x - D.N];
-    return D.cls[x] == C_F ? D.ilvl[x] : D.lvl0[x];
-}
-__device__ __forceinline__ int it_parent(const Dev& D, int x) {
-    if (x >= D.N) return D.lf_parent[x - D.N];
-    return D.cls[x] == C_F ? D.parent[x] : -1;
-}
-__device__ __forceinline__ int it_pseq(const Dev& D, int x) {
-    if (x >= D.N) return D.lf_pseq[x - D.N];
-    return D.cls[x] == C_F ? D.pseq[x] : 0;
-}
+// ---- item accessors ----
+constexpr int kPopMax = 1 << 24;
+__device__ __forceinline__ int rec_lvl(const int4& r) { return (int)((uint32_t)r.z >> 24); }
+__device__ __forceinline__ int rec_pop(const int4& r) { return r.z & (kPopMax - 1); }
+__device__ __forceinline__ int it_lvl(const Dev& D, int x) { return rec_lvl(D.wr[x]); }
+__device__ __forceinline__ int it_parent(const Dev& D, int x) { return D.wr[x].w; }
 
 // x pops before y in the merged phase-1 flood (x != y); sets FB_CMP if the walk is too long.
-// Reads the packed item records (k_pack_items), so a step is two dependent loads: the records of
-// x and y, then those of their chains' largest-key items.
+// A step is two dependent loads: the records of x and y, then those of their chains' largest-key items.
 __device__ bool before_from(const Dev& D, int x, int y, int step0) {
     for (int step = step0; step < CMP_MAX_STEPS; ++step) {
         if (x == y) return false;
-        const int4 rx = D.wr[x], ry = D.wr[y];  // {run, bnode, popidx, parent}
-        if (rx.x == ry.x) return rx.z < ry.z;
+        const int4 rx = D.wr[x], ry = D.wr[y];
+        if (rx.x == ry.x) return rec_pop(rx) < rec_pop(ry);
         const int a = rx.y, b = ry.y;
         const int4 ra = D.wr[a], rb = D.wr[b];
-        const int la = D.wl[a], lb = D.wl[b];
+        const int la = rec_lvl(ra), lb = rec_lvl(rb);
         if (la != lb) return la < lb;
         const int pa = ra.w, pb = rb.w;
         if (pa < 0 && pb < 0) return a < b;  // both queued in the initial raster scan
@@ -153,7 +133,7 @@ struct ItemKey {
 __device__ __forceinline__ ItemKey item_key(const Dev& D, int x) {
     const int4 rx = D.wr[x];
     const int4 ra = D.wr[rx.y];
-    return ItemKey{x, rx.x, rx.z, rx.y, (int)D.wl[rx.y], ra.w};
+    return ItemKey{x, rx.x, rec_pop(rx), rx.y, rec_lvl(ra), ra.w};
 }
 // before(D, kx.item, ky.item), its first step taken from the keys
 __device__ __forceinline__ bool before_keyed(const Dev& D, const ItemKey& kx, const ItemKey& ky) {
@@ -204,7 +184,7 @@ __global__ void k_classify(Dev D, uint8_t* cls, uint16_t* lvl0, uint8_t* fmask, 
         cls[i] = c;
         lvl0[i] = L;
         fmask[i] = (c == C_F) ? 1 : 0;
-        D.st[i] = 0;
+        D.lab[i] = 0;
         D.head[i] = -1;
         D.m[i] = frame ? WSHED : (v < 0 ? 0 : v);
         local += (c == C_F);
@@ -237,7 +217,7 @@ __global__ void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun, cons
     int* head = qh + (size_t)r * NQ;  // per run (run ids are unique across the tiers)
     int* tail = qt + (size_t)r * NQ;
     for (int l = 0; l < NQ; ++l) { head[l] = -1; tail[l] = -1; }
-    int active = NQ, seq = 0, popc = 0;
+    int active = NQ, popc = 0;
     auto enq = [&](int l, int x) {
         D.qnext[x] = -1;
         if (tail[l] >= 0) D.qnext[tail[l]] = x;
@@ -245,23 +225,16 @@ __global__ void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun, cons
         tail[l] = x;
         if (l < active) active = l;
     };
-    // key of an F item or leaf of this run: (level, pseq)
-    auto key_less = [&](int a, int b) {
-        const int la = it_lvl(D, a), lb = it_lvl(D, b);
-        if (la != lb) return la < lb;
-        return it_pseq(D, a) < it_pseq(D, b);
-    };
+    constexpr int QUEUED = -3;  // lab of a pixel that waits in a FIFO
+    auto record = [&](int x, int top, int parent, int level) { D.wr[x] = make_int4(id, top, level << 24, parent); };
     const int minx = box5[nrun + r], maxx = box5[2 * nrun + r];
     const int miny = box5[3 * nrun + r], maxy = box5[4 * nrun + r];
     for (int y = miny; y <= maxy; ++y)
         for (int x = minx; x <= maxx; ++x) {
             const int i = y * W + x;
             if (D.cls[i] == C_F && D.run[i] == id && D.lvl0[i] != NOPUSH) {
-                D.ilvl[i] = (uint8_t)D.lvl0[i];
-                D.pseq[i] = seq++;
-                D.parent[i] = -1;
-                D.bnode[i] = i;
-                D.st[i] = 1;
+                record(i, i, -1, D.lvl0[i]);
+                D.lab[i] = QUEUED;
                 enq(D.lvl0[i], i);
             }
         }
@@ -278,90 +251,86 @@ __global__ void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun, cons
         const int nx = D.qnext[x];
         head[active] = nx;
         if (nx < 0) tail[active] = -1;
-        if (x >= D.N) {  // leaf: record when it pops, nothing else
-            D.lf_popidx[x - D.N] = popc++;
-            continue;
-        }
+        if (popc == kPopMax) { atomicOr(D.flags, FB_LEAF_CAP); return; }
+        D.wr[x].z |= popc++;
+        if (x >= D.N) continue;  // a leaf: when it pops, nothing else
         const int p = x;
-        D.popidx[p] = popc++;
         int lab = 0;
         for (int d = 0; d < 4; ++d) {
             const int s = p + dirs[d];
             int t = 0;
             const uint8_t cs = D.cls[s];
             if (cs == C_SEED) t = D.m0[s];
-            else if (cs == C_F && D.st[s] == 2) t = D.lab[s];
+            else if (cs == C_F) t = D.lab[s];  // positive once popped and labelled
             if (t > 0) { if (lab == 0) lab = t; else if (t != lab) lab = WSHED; }
         }
         D.lab[p] = lab;
-        D.st[p] = 2;
         if (lab == WSHED) continue;
         const uint8_t* ptr = D.img + 3 * (size_t)p;
-        const int bp = D.bnode[p];
+        const int bp = D.wr[p].y;
+        const int bl = it_lvl(D, bp);  // a new item's key is the larger one at the same level (pushed later)
         for (int d = 0; d < 4; ++d) {
             const int s = p + dirs[d];
             const uint8_t cs = D.cls[s];
             if (cs == C_F) {
-                if (D.st[s] != 0) continue;
+                if (D.lab[s] != 0) continue;
                 const int l = c_diff(ptr, D.img + 3 * (size_t)s);
-                D.ilvl[s] = (uint8_t)l;
-                D.pseq[s] = seq++;
-                D.parent[s] = p;
-                D.bnode[s] = key_less(bp, s) ? s : bp;
-                D.st[s] = 1;
+                record(s, bl <= l ? s : bp, p, l);
+                D.lab[s] = QUEUED;
                 enq(l, s);
             } else if (cs == C_B && D.lvl0[s] == NOPUSH) {
                 bool done = false;  // queued already by an earlier labelled neighbour of this run
                 for (int e = 0; e < 4; ++e) {
                     const int f2 = s + dirs[e];
-                    if (f2 != p && D.cls[f2] == C_F && D.run[f2] == id && D.st[f2] == 2 && D.lab[f2] > 0) done = true;
+                    if (f2 != p && D.cls[f2] == C_F && D.run[f2] == id && D.lab[f2] > 0) done = true;
                 }
                 if (done) continue;
                 const int slot = atomicAdd(D.nleaf, 1);
                 if (slot >= D.leafcap) { atomicOr(D.flags, FB_LEAF_CAP); continue; }
                 const int l = c_diff(ptr, D.img + 3 * (size_t)s);
-                D.lf_b[slot] = s;
-                D.lf_run[slot] = id;
-                D.lf_lvl[slot] = (uint8_t)l;
-                D.lf_pseq[slot] = seq++;
-                D.lf_parent[slot] = p;
-                D.lf_popidx[slot] = -1;
+                D.lf_b[slot] = s;  // linked into head[s] by k_link_leaves
                 const int lid = D.N + slot;
-                D.lf_bnode[slot] = key_less(bp, lid) ? lid : bp;  // linked into head[s] by k_link_leaves
+                record(lid, bl <= l ? lid : bp, p, l);
                 enq(l, lid);
             }
         }
     }
 }
 
-// Store to element i of a per-pixel or per-leaf array through a 32-bit byte offset (the
-// decomposition runs on images below 2^28 pixels, so every offset fits): with a uniform base the
-// compiler uses the scalar-base form of the vector store instead of forming a 64-bit address in
-// vector registers for each store.
-template <typename T, typename V>
-__device__ __forceinline__ void gst(T* base, uint32_t i, V v) {
-    *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (size_t)(i * (uint32_t)sizeof(T))) = (T)v;
-}
-
 // ---- phase 1 with the run's neighbourhood staged in LDS ----
-// Same flood as k_phase1, for runs whose bounding box plus a 2-pixel margin has at most LCAP
-// pixels.  The wave stages the frame into LDS (class, in-run flag, seed labels, and the push level
-// of every pixel towards its right and lower neighbour, from the colours), numbers the initial
-// items in raster order with ballots and links them into their level FIFOs chunk by chunk; lane 0
-// then runs the flood with every read in LDS, writing the per-item records to global memory as it
-// goes.  Each queued F pixel carries the key (level, push sequence) and frame index of its chain's
-// largest-key item, so a push compares keys without following pointers.  The 2-pixel margin keeps
-// every neighbour of a leaf candidate inside the frame.  Leaf slots are reserved per run up front
-// (one per B pixel of the frame that could become a leaf), so no atomic sits on the flood's
-// critical path; unused slots keep lf_b = -1.
-// LDS per frame pixel: 15 bytes (class 1, label 4, chain key 4, push levels 2, chain item or leaf
-// index 2, FIFO link 2), so a CU holds as many concurrent floods as its LDS allows for the tier.
+// Same flood as k_phase1, for runs whose bounding box plus a 2-pixel margin has at most LCAP pixels, by
+// one wave per run.  The frame is staged into LDS (the 2-pixel margin keeps every neighbour of a leaf
+// candidate inside it), the initial items are numbered in raster order with ballots, and the wave pops
+// item by item.
+// A flood is one chain of pops by one wave, so a pop costs the instructions it issues and the round
+// trips it waits for.  With one lane driving it through LDS FIFOs that was 1800 cycles (round trips for
+// the head, the neighbours and each pushed FIFO's tail, one per empty level passed over; some fifty
+// branches).  Here
+//  * everything a pixel holds is 16 bytes of LDS, and lanes 0..3 read the four neighbours and lane 4
+//    the pixel itself in one instruction: the pop's only round trip;
+//  * the four neighbours are judged, numbered and recorded side by side in their lanes, each item with
+//    one 16-byte record;
+//  * their FIFOs' entries are read together as soon as the levels are known, behind the label, the
+//    numbering and the records; pushes of one level are chained inside the quad;
+//  * a level that has run out finds the next queued one in one read of all 256 entries.
+//  * labels and pop indexes stay in LDS and leave for the image in one sweep after the last pop.
+// Measured: a pop takes 930 cycles; the longest flood of a 512 x 512 tile (704 pops, staging included)
+// 509 -> 291 us; the runs with frames up to 1024 pixels of a 4096 x 4096 tile 1400 -> 823 us.
+// Each queued F pixel carries the key (level, push sequence) and frame index of its chain's largest-key
+// item, so a push compares keys without following pointers.  Leaf slots are reserved per run up front
+// (one per B pixel of the frame that could become a leaf), so no atomic sits on the flood's critical
+// path; unused slots get lf_b = -1.
 constexpr uint16_t NIL16 = 0xFFFF;
 // phase-1 FIFO links: an item index below 0x7FFF (frames hold at most 6400 pixels), P1_LEAF when
 // the item is a leaf, P1_NIL for none
-constexpr uint32_t P1_NIL = 0x7FFF, P1_LEAF = 0x8000;
-enum { K_INRUN = 4, K_ST1 = 8, K_ST2 = 16, K_LV = 32 };
+constexpr uint32_t P1_NIL = 0x7FFF, P1_LEAF = 0x8000, P1_EMPTY = P1_NIL << 16 | P1_NIL;
+// the frame pixel's flags: of the run; not queued yet and pushed by a labelled neighbour as an F item /
+// as a leaf; queued in the initial scan
+enum { K_INRUN = 4, K_CANF = 8, K_CANL = 16, K_LV = 32 };
 constexpr int P1_MARGIN = 2;
+// parts of a 16-byte entry, accessed beside the whole entry
+typedef uint32_t __attribute__((may_alias)) any_u32;
+typedef uint16_t __attribute__((may_alias)) any_u16;
 
 __device__ __forceinline__ int cdiff_packed(uint32_t a, uint32_t b) {
     const int d0 = abs((int)(a & 255) - (int)(b & 255));
@@ -370,19 +339,61 @@ __device__ __forceinline__ int cdiff_packed(uint32_t a, uint32_t b) {
     return max(max(d0, d1), d2);
 }
 
+// the lane's quad (lanes 4 q .. 4 q + 3) combined by max / min: every lane of it gets the result
+__device__ __forceinline__ int quad_swap1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true); }
+__device__ __forceinline__ int quad_swap2(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true); }
+__device__ __forceinline__ int quad_max(int v) {
+    v = max(v, quad_swap1(v));
+    return max(v, quad_swap2(v));
+}
+__device__ __forceinline__ uint32_t quad_min(uint32_t v) {
+    v = min(v, (uint32_t)quad_swap1((int)v));
+    return min(v, (uint32_t)quad_swap2((int)v));
+}
+// pop_label of the four values in a quad's lanes, at least one of them positive
+__device__ __forceinline__ int quad_label(int t) {
+    const int mx = quad_max(t);
+    const uint32_t mn1 = quad_min((uint32_t)t - 1u);
+    return (int)mn1 + 1 == mx ? mx : WSHED;
+}
+__device__ __forceinline__ uint32_t lane_of(uint32_t v, int lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+__device__ __forceinline__ int lanes_below(unsigned long long m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// v of lane (lane + R) & 3 of the lane's quad
+template <int R>
+__device__ __forceinline__ uint32_t quad_rot(uint32_t v) {
+    constexpr int ctrl = R == 1 ? 0x39 : (R == 2 ? 0x4E : 0x93);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+// {level - 4 * lane << 16 | head} of the lowest queued level of a lane's four FIFO entries, P1_NIL for none
+__device__ __forceinline__ uint32_t first_queued(uint4 q) {
+    const uint32_t h0 = q.x & 0xFFFFu, h1 = q.y & 0xFFFFu, h2 = q.z & 0xFFFFu, h3 = q.w & 0xFFFFu;
+    uint32_t v = h3 != P1_NIL ? 3u << 16 | h3 : P1_NIL;
+    v = h2 != P1_NIL ? 2u << 16 | h2 : v;
+    v = h1 != P1_NIL ? 1u << 16 | h1 : v;
+    return h0 != P1_NIL ? h0 : v;
+}
+
 template <int LCAP>
 __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restrict__ box5, int nrun,
                                                    const int* __restrict__ list, const int* __restrict__ count,
                                                    int* __restrict__ next_run) {
-    __shared__ uint8_t code[LCAP];
-    __shared__ int32_t lk[LCAP];     // known label: seed label, label of a popped F pixel, else 0
-    __shared__ uint32_t bkey[LCAP];  // queued F pixel: (level << 16 | push seq) of its chain's largest-key item
-                                     // (the pixel's colour while the frame is staged)
-    __shared__ uint16_t dif[LCAP];   // push level towards the right (low byte) and lower (high byte) neighbour
-    __shared__ uint16_t bloc[LCAP];  // queued F pixel: frame index of that item; B pixel: its leaf index
-    __shared__ uint16_t qn[LCAP];    // FIFO link of the item at this pixel (an F item, or a B pixel's leaf)
-    __shared__ uint16_t qhead[NQ], qtail[NQ];
+    // per frame pixel: x = class and flags | push level to the right << 8 | to the lower neighbour << 16 |
+    // level of its initial push << 24; y = frame index of a queued F pixel's chain's largest-key item, or a
+    // leaf's index in the run | FIFO link << 16; z = known label (seed label, label of a popped F pixel,
+    // else 0); w = that largest-key item's key (level << 16 | push seq), then the pixel's pop index (and
+    // its colour while the frame is staged)
+    __shared__ uint4 px[LCAP];
+    __shared__ uint4 qlv[NQ / 4];  // per level its FIFO's tail << 16 | head; empty while the head is P1_NIL
     __shared__ int sh_base, sh_it;
+    any_u32* const word = reinterpret_cast<any_u32*>(px);
+    any_u16* const half = reinterpret_cast<any_u16*>(px);  // pixel k's link: half[8 k + 3]
+    any_u32* const entry = reinterpret_cast<any_u32*>(qlv);
+    any_u16* const head = reinterpret_cast<any_u16*>(qlv);  // head[2 l]
 
     // a fixed grid takes the tier's runs from a work counter, one at a time, so a workgroup that
     // drew short runs takes more of them (a fixed stride over the list left the tier's time set by
@@ -393,254 +404,206 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
     for (;;) {
     if (threadIdx.x == 0) sh_it = atomicAdd(next_run, 1);
     __syncthreads();
-    const int it = sh_it;
+    const int it = uni(sh_it);
     if (it >= nr) break;
     [&]() {  // one run; `return` ends the run
-    const int r = list[it];
+    const int r = uni(list[it]);
     const int lane = threadIdx.x;
     const int W = D.W, H = D.H, id = r + 1;
-    const int ox = box5[nrun + r] - P1_MARGIN, oy = box5[3 * nrun + r] - P1_MARGIN;
-    const int lw = box5[2 * nrun + r] - ox + 1 + P1_MARGIN, lh = box5[4 * nrun + r] - oy + 1 + P1_MARGIN;
+    const int ox = uni(box5[nrun + r]) - P1_MARGIN, oy = uni(box5[3 * nrun + r]) - P1_MARGIN;
+    const int lw = uni(box5[2 * nrun + r]) - ox + 1 + P1_MARGIN, lh = uni(box5[4 * nrun + r]) - oy + 1 + P1_MARGIN;
     const int L = lw * lh;  // <= LCAP (bucketed by the host)
     // k / lw by multiply-high (exact for k < 2^16)
     const uint32_t magic = (uint32_t)((0x100000000ull + (unsigned)lw - 1) / (unsigned)lw);
-    const int gbase = oy * W + ox;
-    auto gidx = [&](int k) {
-        const int ky = (int)__umulhi((uint32_t)k, magic);
-        return gbase + ky * W + (k - ky * lw);
-    };
+    const int gbase = oy * W + ox, gstep = W - lw;
+    auto gidx = [&](int k) { return gbase + k + (int)__umulhi((uint32_t)k, magic) * gstep; };
 
-    for (int k = lane; k < L; k += 64) {
-        const int ky = (int)__umulhi((uint32_t)k, magic), kx = k - ky * lw;
-        const int gx = ox + kx, gy = oy + ky;
-        uint8_t cd = C_FRAME;
-        int32_t l0 = 0;
-        uint32_t cc = 0;
-        if (gx >= 0 && gx < W && gy >= 0 && gy < H) {  // the margin may step one pixel off the image
-            const int g = gy * W + gx;
-            const uint8_t c = D.cls[g];
-            cd = c;
-            if (c == C_F && D.run[g] == id) cd |= K_INRUN;
-            if (c == C_SEED) l0 = D.m0[g];
-            if (D.lvl0[g] != NOPUSH) cd |= K_LV;
-            const uint8_t* q = D.img + 3 * (size_t)g;
-            cc = (uint32_t)q[0] | ((uint32_t)q[1] << 8) | ((uint32_t)q[2] << 16);
+    qlv[lane] = make_uint4(P1_EMPTY, P1_EMPTY, P1_EMPTY, P1_EMPTY);
+    // four chunks of 64 pixels at a time, every load from a clamped (always valid) pixel before any use
+    for (int k0 = 0; k0 < L; k0 += 256) {
+        uint8_t c[4], q0[4], q1[4], q2[4];
+        uint16_t l0[4];
+        int32_t rn[4], m0[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = min(k0 + 64 * j + lane, L - 1);
+            const int ky = (int)__umulhi((uint32_t)k, magic);
+            const size_t g = (size_t)clampi(oy + ky, 0, H - 1) * W + clampi(ox + k - ky * lw, 0, W - 1);
+            c[j] = D.cls[g];
+            rn[j] = D.run[g];
+            m0[j] = D.m0[g];
+            l0[j] = D.lvl0[g];
+            q0[j] = D.img[3 * g];
+            q1[j] = D.img[3 * g + 1];
+            q2[j] = D.img[3 * g + 2];
         }
-        code[k] = cd;
-        lk[k] = l0;
-        bkey[k] = cc;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = k0 + 64 * j + lane;
+            if (k >= L) continue;
+            const int ky = (int)__umulhi((uint32_t)k, magic), gx = ox + k - ky * lw, gy = oy + ky;
+            const bool in = gx >= 0 && gx < W && gy >= 0 && gy < H;  // the margin may step one pixel off the image
+            const bool lv = l0[j] != NOPUSH;
+            uint32_t cd = c[j];
+            if (cd == C_F) cd |= K_CANF | (rn[j] == id ? K_INRUN : 0);
+            if (cd == C_B && !lv) cd |= K_CANL;
+            if (lv) cd |= K_LV | (uint32_t)l0[j] << 24;
+            px[k] = make_uint4(in ? cd : (uint32_t)C_FRAME, P1_NIL << 16, in && c[j] == C_SEED ? (uint32_t)m0[j] : 0u,
+                               in ? q0[j] | (uint32_t)q1[j] << 8 | (uint32_t)q2[j] << 16 : 0u);
+        }
     }
-    for (int l = lane; l < NQ; l += 64) { qhead[l] = P1_NIL; qtail[l] = P1_NIL; }
     __syncthreads();
     // push levels between 4-neighbours (a pair that wraps around a frame row is never used: pushes
     // start at run pixels, which lie the margin away from the frame's edge)
     for (int k = lane; k < L; k += 64) {
-        const uint32_t c = bkey[k];
-        const int rt = k + 1 < L ? cdiff_packed(c, bkey[k + 1]) : 0;
-        const int dn = k + lw < L ? cdiff_packed(c, bkey[k + lw]) : 0;
-        dif[k] = (uint16_t)(rt | (dn << 8));
+        const uint32_t c = word[4 * k + 3], cr = word[4 * min(k + 1, L - 1) + 3], cl = word[4 * min(k + lw, L - 1) + 3];
+        const uint32_t rt = (uint32_t)cdiff_packed(c, cr), dn = (uint32_t)cdiff_packed(c, cl);
+        word[4 * k] |= rt << 8 | dn << 16;
     }
     __syncthreads();
-    // leaf candidates (B, never initially queued, 4-adjacent to the run) and initial items in
-    // raster order: an initial item's records are written here, and the chunk's items of one level
-    // are linked behind that level's FIFO tail (the first of them reads the tail, the last moves it)
-    int cnt = 0, ninit = 0;
+    // leaf candidates (B, never initially queued, 4-adjacent to the run) and initial items in raster
+    // order: a chunk's items of one level are linked in a row behind that level's FIFO (the first of
+    // them reads the entry, the last writes it)
+    int cnt = 0, seq = 0;
     for (int k0 = 0; k0 < L; k0 += 64) {
-        const int k = k0 + lane;
-        bool cand = false, init = false;
-        if (k < L) {
-            const uint8_t cd = code[k];
-            const int ky = (int)__umulhi((uint32_t)k, magic), kx = k - ky * lw;
-            if ((cd & 3) == C_B && !(cd & K_LV) && kx > 0 && kx < lw - 1 && ky > 0 && ky < lh - 1)
-                cand = ((code[k - 1] | code[k + 1] | code[k - lw] | code[k + lw]) & K_INRUN) != 0;
-            init = (cd & K_INRUN) && (cd & K_LV);
-        }
-        const unsigned long long bc = __ballot(cand), bi = __ballot(init);
-        cnt += __popcll(bc);
+        const int k = k0 + lane, kc = min(k, L - 1);
+        const int ky = (int)__umulhi((uint32_t)kc, magic), kx = kc - ky * lw;
+        const bool inner = k < L && kx > 0 && kx < lw - 1 && ky > 0 && ky < lh - 1;
+        const int kn = inner ? kc : min(lw + 1, L - 1);  // a pixel whose neighbours exist (frames are 5 x 5 at least)
+        const uint32_t cd = word[4 * kc];
+        const uint32_t nb = word[4 * (kn - 1)] | word[4 * (kn + 1)] | word[4 * (kn - lw)] | word[4 * (kn + lw)];
+        const bool cand = inner && (cd & K_CANL) && (nb & K_INRUN);
+        const bool init = k < L && (cd & K_INRUN) && (cd & K_LV);
+        const unsigned long long bi = __ballot(init);
+        cnt += __popcll(__ballot(cand));
         if (!bi) continue;
-        int lvl = -1, g = 0;
-        if (init) {
-            g = gidx(k);
-            lvl = D.lvl0[g];
-        }
-        int prevk = -1, nextk = -1;  // this chunk's previous and next initial item of the same level
+        const int lvl = init ? (int)(cd >> 24) : -1, q = seq + lanes_below(bi);
+        int first = -1, prev = -1, next = -1;  // lanes of this chunk's first, previous and next item of the level
         for (unsigned long long m = bi; m; m &= m - 1) {
-            const int j = __ffsll((long long)m) - 1;
-            const int lj = __builtin_amdgcn_readlane(lvl, j);
-            if (lj == lvl) {
-                if (j < lane) prevk = k0 + j;
-                else if (j > lane && nextk < 0) nextk = k0 + j;
-            }
+            const int j = __builtin_ctzll(m);
+            const bool same = (int)lane_of((uint32_t)lvl, j) == lvl;
+            first = same && first < 0 ? j : first;
+            prev = same && j < lane ? j : prev;
+            next = same && j > lane && next < 0 ? j : next;
         }
         if (init) {
-            const int q = ninit + __popcll(bi & ((1ull << lane) - 1ull));
-            bkey[k] = ((uint32_t)lvl << 16) | (uint32_t)q;
-            bloc[k] = (uint16_t)k;
-            code[k] |= K_ST1;
-            qn[k] = nextk < 0 ? P1_NIL : (uint16_t)nextk;
-            gst(D.ilvl, g, (uint8_t)lvl);
-            gst(D.pseq, g, q);
-            gst(D.parent, g, -1);
-            gst(D.bnode, g, g);
-            gst(D.st, g, 1);
-            if (prevk < 0) {
-                const uint16_t t = qtail[lvl];
-                if (t == P1_NIL) qhead[lvl] = (uint16_t)k;
-                else qn[t] = (uint16_t)k;
-            }
-            if (nextk < 0) qtail[lvl] = (uint16_t)k;
+            const int g = gidx(k);
+            px[k] = make_uint4(cd & ~(uint32_t)K_CANF, (next < 0 ? P1_NIL : (uint32_t)(k0 + next)) << 16 | (uint32_t)k, 0u,
+                               (uint32_t)lvl << 16 | (uint32_t)q);
+            D.wr[g] = make_int4(id, g, lvl << 24, -1);
+            const uint32_t e = entry[lvl], h = e & 0xFFFFu;
+            if (prev < 0 && h != P1_NIL) half[8 * (e >> 16) + 3] = (uint16_t)k;
+            if (next < 0) entry[lvl] = (uint32_t)k << 16 | (h == P1_NIL ? (uint32_t)(k0 + first) : h);
         }
-        ninit += __popcll(bi);
+        seq += __popcll(bi);
     }
     if (lane == 0) sh_base = atomicAdd(D.nleaf, cnt);
     __syncthreads();
-    const int base = sh_base;
-    // every reserved slot below the capacity reads as unused until a leaf fills it
-    for (int j = base + lane; j < min(base + cnt, D.leafcap); j += 64) gst(D.lf_b, j, -1);
+    const int base = uni(sh_base);
     if (base + cnt > D.leafcap) {
+        // every reserved slot below the capacity reads as unused
+        for (int j = base + lane; j < D.leafcap; j += 64) D.lf_b[j] = -1;
         if (lane == 0) atomicOr(D.flags, FB_LEAF_CAP);
         return;
     }
-    __syncthreads();
-    if (lane != 0) return;
 
-    int active = 0;  // no queued item below this level
-    int hx = qhead[0];  // head of the active level's FIFO (a copy of qhead[active])
-    // FIFO of level l; the flood resumes at the lowest queued level.  Links and heads carry the
-    // queued item's kind (P1_LEAF), so a leaf's pop knows what it pops before reading anything.
-    auto enq = [&](int l, int x, uint32_t kind) {
-        qn[x] = P1_NIL;
-        const uint32_t t = uni(qtail[l]);
-        const uint32_t xv = (uint32_t)x | kind;
-        if (t != P1_NIL) qn[t] = (uint16_t)xv;
-        else qhead[l] = (uint16_t)xv;
-        qtail[l] = (uint16_t)x;
-        if (t == P1_NIL && l <= active) {  // nothing is queued below `active`: l was empty
-            active = l;
-            hx = (int)xv;
+    // lanes 0..3: the neighbours in push order (left, right, up, down); the others read the pixel itself
+    // (queued, so never pushed)
+    const int loff = lane == 0 ? -1 : (lane == 1 ? 1 : (lane == 2 ? -lw : (lane == 3 ? lw : 0)));
+    const int goff = lane == 0 ? -1 : (lane == 1 ? 1 : (lane == 2 ? -W : (lane == 3 ? W : 0)));
+    const int lsh = lane < 2 ? 8 : 16;  // where the level of the push over that edge is, in the pixel itself (lanes
+                                        // 1, 3) or in the neighbour (0, 2)
+    int popc = 0, nlf = 0, active = 0;
+    uint32_t hx = P1_NIL;  // the next item to pop, of level `active`; P1_NIL: of the lowest queued level
+    while (popc < L) {  // (a pixel pops at most once)
+        if (hx == P1_NIL) {
+            const uint32_t f = first_queued(qlv[lane]);
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(f != P1_NIL);
+            if (!m) break;
+            const int l4 = __builtin_ctzll(m);
+            const uint32_t v = lane_of(f, l4);
+            active = 4 * l4 + (int)(v >> 16);
+            hx = v & 0xFFFFu;
         }
-    };
-    int seq = ninit, popc = 0, nlf = 0;
-    const int ld[4] = {-1, 1, -lw, lw};
-    const int gd[4] = {-1, 1, -W, W};
-    for (;;) {
-        int xv = hx;
-        if (xv == P1_NIL) {
-            int l = active + 1;
-            while (l < NQ && uni(qhead[l]) == P1_NIL) ++l;
-            if (l == NQ) break;
-            active = l;
-            xv = uni(qhead[l]);
+        const int x = (int)(hx & P1_NIL);
+        const uint4 s = px[x + loff];
+        const uint32_t cw = lane_of(s.x, 4), yw = lane_of(s.y, 4), key = lane_of(s.w, 4);
+        const uint32_t nx = yw >> 16;
+        if (lane == 4) head[2 * active] = (uint16_t)nx;
+        const int lvl = (int)(((lane & 1) ? cw : s.x) >> lsh & 255u);
+        const uint32_t e = entry[lvl];  // used by the pushes below; everything up to them runs while it loads
+        const int ql = uni(quad_label((int)s.z));
+        const int lab = hx & P1_LEAF ? 0 : ql;  // a leaf's pop is only counted: no label, no pushes
+        // the neighbours to push (none from a leaf or a dam).  A neighbour's state may have changed since the
+        // read only through this pop's own pushes, which go to other pixels.  A B pixel queued already is a
+        // leaf pushed by an earlier labelled neighbour of this run (every popped F pixel of the run is labelled
+        // or a dam, and a labelled one queues its B neighbours)
+        const bool isl = s.x & K_CANL, push = lab > 0 && (s.x & (K_CANF | K_CANL));
+        const uint32_t m = (uint32_t)__builtin_amdgcn_ballot_w64(push), ml = m & (uint32_t)__builtin_amdgcn_ballot_w64(isl);
+        const int sk = x + loff;
+        const int sq = (int)__builtin_amdgcn_mbcnt_lo(m, (uint32_t)seq), j = (int)__builtin_amdgcn_mbcnt_lo(ml, (uint32_t)nlf);
+        const uint32_t nkey = (uint32_t)lvl << 16 | (uint32_t)sq, bl = yw & 0xFFFFu;
+        const bool newer = key < nkey;  // the new item has the larger key on its chain
+        if (push || lane == 4) {
+            const uint32_t y = P1_NIL << 16 | (isl ? (uint32_t)j : (newer ? (uint32_t)sk : bl));
+            px[sk] = make_uint4(s.x & ~(uint32_t)(K_CANF | K_CANL), push ? y : s.y, push ? s.z : (uint32_t)lab,
+                                push ? max(key, nkey) : (uint32_t)popc);
         }
-        const int x = xv & (int)P1_NIL;
-        if (xv & P1_LEAF) {  // a leaf: record when it pops
-            uint32_t nx = qn[x];
-            int bl = bloc[x];
-            asm volatile("" : "+v"(nx), "+v"(bl));
-            nx = uni(nx);
-            bl = uni(bl);
-            qhead[active] = (uint16_t)nx;
-            hx = (int)nx;
-            if (nx == P1_NIL) qtail[active] = P1_NIL;
-            gst(D.lf_popidx, base + bl, popc++);
-            continue;
+        ++popc;
+        hx = nx;
+        if (!m) continue;
+        seq += __popc(m);
+        nlf += __popc(ml);
+        // pushes of one level go one behind the other, the first of them behind the FIFO's tail; lanes that
+        // push nothing hold levels of their own
+        const uint32_t pl = push ? (uint32_t)lvl : 256u + (uint32_t)lane, qx = (uint32_t)sk | (isl ? P1_LEAF : 0u);
+        const bool s1 = quad_rot<1>(pl) == pl, s2 = quad_rot<2>(pl) == pl, s3 = quad_rot<3>(pl) == pl;
+        const uint32_t q1 = quad_rot<1>(qx), q2 = quad_rot<2>(qx), q3 = quad_rot<3>(qx);
+        const bool b1 = s3 && lane >= 1, b2 = s2 && lane >= 2, b3 = s1 && lane >= 3;  // one, two, three lanes before
+        const bool last = !((s1 && lane <= 2) || (s2 && lane <= 1) || (s3 && lane == 0));
+        const uint32_t first = b3 ? q1 : (b2 ? q2 : (b1 ? q3 : qx)), prev = b1 ? q3 : (b2 ? q2 : q1);
+        const bool chained = b1 || b2 || b3;
+        if (push) {
+            const int gp = gidx(x), gs = gp + goff, gt = gidx((int)bl);
+            const int me = isl ? D.N + base + j : gs;
+            D.wr[me] = make_int4(id, newer ? me : gt, lvl << 24, gp);
         }
-        // an F item: its link, class and chain entry and its neighbours' values, in one round
-        // trip (the compiler would otherwise sink the push-side reads past the dam test and fetch
-        // them in a second round trip)
-        uint32_t nx = qn[x], cpc = code[x];
-        int nl[4];
-        uint32_t nc[4];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            nl[d] = lk[x + ld[d]];
-            nc[d] = code[x + ld[d]];
+        // the level to go on with: a pushed one below the active level, or at it if its FIFO has run out
+        const uint32_t lo = (uint32_t)uni((int)quad_min(pl << 2 | (uint32_t)(lane & 3)));
+        const int ll = (int)(lo >> 2);
+        if (ll + (nx != P1_NIL ? 1 : 0) <= active) {
+            active = ll;
+            hx = lane_of(qx, (int)(lo & 3u));
         }
-        uint32_t dleft = dif[x - 1], dhere = dif[x], dup = dif[x - lw];
-        uint32_t bk = bkey[x];
-        int bl = bloc[x];
-        asm volatile("" : "+v"(nx), "+v"(cpc), "+v"(nl[0]), "+v"(nl[1]), "+v"(nl[2]), "+v"(nl[3]), "+v"(nc[0]),
-                     "+v"(nc[1]), "+v"(nc[2]), "+v"(nc[3]), "+v"(dleft), "+v"(dhere), "+v"(dup), "+v"(bk), "+v"(bl));
-        // one lane floods: every value it read is the same for the wave, so the bookkeeping below
-        // runs on the scalar unit with scalar branches instead of masked vector code
-        nx = uni(nx);
-        cpc = uni(cpc);
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            nl[d] = uni(nl[d]);
-            nc[d] = uni(nc[d]);
-        }
-        dleft = uni(dleft);
-        dhere = uni(dhere);
-        dup = uni(dup);
-        bk = uni(bk);
-        bl = uni(bl);
-        qhead[active] = (uint16_t)nx;
-        hx = (int)nx;
-        if (nx == P1_NIL) qtail[active] = P1_NIL;
-        const int p = x;
-        const int lvd[4] = {(int)(dleft & 255), (int)(dhere & 255), (int)(dup >> 8), (int)(dhere >> 8)};
-        const int gp = gidx(p);
-        gst(D.popidx, gp, popc++);
-        const int lab = pop_label(nl[0], nl[1], nl[2], nl[3]);
-        lk[p] = lab;
-        code[p] = (uint8_t)((cpc & ~K_ST1) | K_ST2);
-        gst(D.lab, gp, lab);
-        gst(D.st, gp, 2);
-        if (lab == WSHED) continue;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const int sk = p + ld[d];
-            // a neighbour's state may have changed since the batch read only through this pop's own
-            // earlier pushes, which go to other pixels
-            const uint32_t cs = nc[d];
-            if ((cs & 3) == C_F) {
-                if (cs & (K_ST1 | K_ST2)) continue;
-                const int l = lvd[d];
-                const int gs = gp + gd[d];
-                const uint32_t key = ((uint32_t)l << 16) | (uint32_t)seq;
-                const bool newer = bk < key;  // the new item has the larger key on its chain
-                bkey[sk] = newer ? key : bk;
-                bloc[sk] = (uint16_t)(newer ? sk : bl);
-                code[sk] = cs | K_ST1;
-                gst(D.ilvl, gs, (uint8_t)l);
-                gst(D.pseq, gs, seq);
-                gst(D.parent, gs, gp);
-                gst(D.bnode, gs, newer ? gs : gidx(bl));
-                gst(D.st, gs, 1);
-                ++seq;
-                enq(l, sk, 0);
-            } else if ((cs & 3) == C_B && !(cs & (K_LV | K_ST1))) {
-                // K_ST1 on a B pixel: queued already, by an earlier labelled neighbour of this run
-                // (every popped F pixel of the run is labelled or a dam, and a labelled one queues
-                // its B neighbours)
-                if (nlf >= cnt) { atomicOr(D.flags, FB_LEAF_CAP); continue; }
-                const int j = nlf++;
-                const int slot = base + j;
-                bloc[sk] = (uint16_t)j;
-                code[sk] = cs | K_ST1;
-                const int l = lvd[d];
-                const uint32_t key = ((uint32_t)l << 16) | (uint32_t)seq;
-                gst(D.lf_b, slot, gp + gd[d]);
-                gst(D.lf_run, slot, id);
-                gst(D.lf_lvl, slot, (uint8_t)l);
-                gst(D.lf_pseq, slot, seq);
-                gst(D.lf_parent, slot, gp);
-                gst(D.lf_popidx, slot, -1);
-                gst(D.lf_bnode, slot, bk < key ? D.N + slot : gidx(bl));
-                ++seq;
-                enq(l, sk, P1_LEAF);
-            }
-        }
-        if (seq >= 65535) { atomicOr(D.flags, FB_LEAF_CAP); return; }
+        const uint32_t h = e & 0xFFFFu;
+        const uint32_t tail = chained ? prev & P1_NIL : e >> 16;
+        if (push && (chained || h != P1_NIL)) half[8 * tail + 3] = (uint16_t)qx;
+        if (push && last) entry[lvl] = (uint32_t)sk << 16 | (h == P1_NIL ? first : h);
     }
+    // labels and pop indexes (low half of a record's third word) of the run's queued pixels and of its
+    // leaves (every queued item has popped)
+    auto pop_of = [&](int item) -> any_u16& { return reinterpret_cast<any_u16*>(D.wr + item)[4]; };
+    for (int k = lane; k < L; k += 64) {
+        const uint4 s = px[k];
+        const int g = gidx(k);
+        if ((s.x & (K_INRUN | K_CANF)) == K_INRUN) {
+            pop_of(g) = (uint16_t)s.w;
+            D.lab[g] = (int)s.z;
+        } else if ((s.x & (3 | K_LV | K_CANL)) == C_B) {
+            const int j = base + (int)(s.y & 0xFFFFu);
+            pop_of(D.N + j) = (uint16_t)s.w;
+            D.lf_b[j] = g;
+        }
+    }
+    for (int j = base + nlf + lane; j < base + cnt; j += 64) D.lf_b[j] = -1;
     }();
     __syncthreads();  // the LDS arrays are reused by the next run
     }
 }
 
 // LDS bytes of one k_phase1_lds<LCAP> workgroup (the host sizes each tier's grid from it)
-constexpr int p1_lds_bytes(int lcap) { return 15 * lcap + 4 * NQ + 8; }
+constexpr int p1_lds_bytes(int lcap) { return 16 * lcap + 4 * NQ + 8; }
 
 // grid of a k_phase1_lds<LCAP> launch: the workgroups the device holds at once (LDS-bound), at most
 // one per run of the image
@@ -694,35 +657,8 @@ __global__ void k_link_leaves(Dev D, int* __restrict__ blist, int* __restrict__ 
     }
 }
 
-// The item records before() walks, from the phase-1 results: F pixels (run, chain's largest-key
-// item, pop index, pusher, level), B pixels queued in the initial scan (run -(x + 2), themselves,
-// pop index 0, no pusher, initial level) and used leaf slots (ids N + slot).  Other ids are never
-// visited by a walk and keep whatever the memory held.
-__global__ void k_pack_items(Dev D) {
-    const int N = D.N;
-    const int nl = min(*D.nleaf, D.leafcap);
-    const size_t total = (size_t)N + nl;
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-        if (t < (size_t)N) {
-            const int x = (int)t;
-            const uint8_t c = D.cls[x];
-            if (c == C_F) {
-                D.wr[x] = make_int4(D.run[x], D.bnode[x], D.popidx[x], D.parent[x]);
-                D.wl[x] = D.ilvl[x];
-            } else if (c == C_B && D.lvl0[x] != NOPUSH) {
-                D.wr[x] = make_int4(-(x + 2), x, 0, -1);
-                D.wl[x] = (uint8_t)D.lvl0[x];
-            }
-        } else {
-            const int sl = (int)(t - N);
-            if (D.lf_b[sl] < 0) continue;
-            D.wr[t] = make_int4(D.lf_run[sl], D.lf_bnode[sl], D.lf_popidx[sl], D.lf_parent[sl]);
-            D.wl[t] = D.lf_lvl[sl];
-        }
-    }
-}
-
-// B pixels queued in the initial scan (next to a seed)
+// B pixels queued in the initial scan (next to a seed): their list and their records (each a run of its
+// own, without a pusher)
 __global__ void k_collect_b0(Dev D, int* __restrict__ blist, int* __restrict__ bcount) {
     const int stride = gridDim.x * blockDim.x;
     const int n_up = ((D.N + 63) / 64) * 64;
@@ -731,6 +667,7 @@ __global__ void k_collect_b0(Dev D, int* __restrict__ blist, int* __restrict__ b
         const uint8_t c = D.cls[j];
         const uint16_t l0 = D.lvl0[j];
         const bool take = i < D.N && c == C_B && l0 != NOPUSH;
+        if (take) D.wr[i] = make_int4(-(i + 2), i, (int)l0 << 24, -1);
         wave_append(take, i, blist, bcount);
     }
 }
@@ -760,13 +697,12 @@ __global__ void k_bucket_runs(const int32_t* __restrict__ box5, int nrun, int* _
 // per neighbour); only the pop-order walk stays conditional.
 __device__ int b_label(const Dev& D, int b, int r, int W) {
     const int dirs[4] = {-1, 1, -W, W};
-    uint8_t cs[4], ss[4];
+    uint8_t cs[4];
     int ms[4], ls[4];
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         const int s = b + dirs[d];
         cs[d] = D.cls[s];
-        ss[d] = D.st[s];
         ms[d] = D.m0[s];
         ls[d] = D.lab[s];
     }
@@ -774,7 +710,7 @@ __device__ int b_label(const Dev& D, int b, int r, int W) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
         const bool seed = cs[d] == C_SEED;
-        const bool fcand = cs[d] == C_F && ss[d] == 2 && ls[d] > 0;
+        const bool fcand = cs[d] == C_F && ls[d] > 0;
         int t = seed ? ms[d] : 0;
         if (!seed && fcand && before(D, b + dirs[d], r)) t = ls[d];
         if (t > 0) { if (lab == 0) lab = t; else if (t != lab) lab = WSHED; }
@@ -800,7 +736,7 @@ __global__ void k_bresolve(Dev D, int32_t* __restrict__ real, int* __restrict__ 
             else {
                 for (int sl = D.head[b]; sl >= 0; sl = D.lf_next[sl]) {
                     const int lid = D.N + sl;
-                    if (r < 0 || before(D, D.lf_parent[sl], it_parent(D, r))) r = lid;
+                    if (r < 0 || before(D, it_parent(D, lid), it_parent(D, r))) r = lid;
                 }
             }
             real[b] = r;
@@ -883,14 +819,19 @@ __global__ void k_t1_state(Dev D, const int32_t* __restrict__ real, const int* _
     const int b1 = info[0], b1i = info[1], Y1 = info[2];
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < D.N; p += gridDim.x * blockDim.x) {
         uint8_t pm = 0, kd = 0;
-        // the pixel's class, state, label, pusher and queue entry are loaded together (each one
-        // behind the class test would be another dependent round trip)
-        const uint8_t c = D.cls[p], stp = D.st[p];
-        const int labp = D.lab[p], parp = D.parent[p], r = real[p];
+        // the pixel's class, label and queue entry are loaded together (each one behind the class
+        // test would be another dependent round trip); its record, where it has one, by the walk
+        const uint8_t c = D.cls[p];
+        const int labp = D.lab[p], r = real[p];
         if (c == C_F) {
             int v = 0;
-            if (stp == 2 && (b1 < 0 || before(D, p, b1i))) v = labp;
-            else if (stp >= 1 && (parp < 0 || b1 < 0 || before(D, parp, b1i))) { v = IN_QUEUE; kd = 1; }
+            if (labp != 0) {  // queued, and popped, in its run's flood
+                if (b1 < 0 || before(D, p, b1i)) v = labp;
+                else {
+                    const int par = it_parent(D, p);
+                    if (par < 0 || before(D, par, b1i)) { v = IN_QUEUE; kd = 1; }
+                }
+            }
             D.m[p] = v;
         } else if (c == C_B) {
             int v = 0;
@@ -971,12 +912,13 @@ struct P2 {
 // b1 flood's layer, then in raster order, and the caller checks that the order does not matter).
 // The data this reads of one item is packed once, so that a sort compares cached values:
 // bit 63 = queued by the b1 flood (kind 2); then, for kind 2, its label (the layer) in the low 32
-// bits; else (pusher + 1) in bits 32..62 and the push sequence in the low 32 bits.
+// bits; else (pusher + 1) in bits 32..62 and the pusher's direction (its push order) in the low 32 bits.
 __device__ long long push_key(const Dev& D, const int32_t* real, const uint8_t* kind, int a) {
     if (kind[a] == 2) return (long long)(1ull << 63) | (long long)(uint32_t)D.lab[a];
     const int ia = D.cls[a] == C_B ? real[a] : a;
-    const int pa = it_parent(D, ia);
-    return ((long long)(uint32_t)(pa + 1) << 32) | (long long)(uint32_t)it_pseq(D, ia);
+    const int pa = it_parent(D, ia), d = a - pa;
+    const uint32_t dir = d == -1 ? 0 : (d == 1 ? 1 : (d < 0 ? 2 : 3));  // pushes go left, right, up, down
+    return ((long long)(uint32_t)(pa + 1) << 32) | (long long)dir;
 }
 // a pushed before b, from their packed data
 __device__ bool push_before_key(const Dev& D, const int32_t* real, int a, long long ka, int b, long long kb) {
@@ -1004,7 +946,7 @@ __device__ int item_level(const Dev& D, const int32_t* real, const uint8_t* kind
         const uint8_t* c = D.img + 3 * (size_t)p;
         return max(max((int)c[0], (int)c[1]), (int)c[2]);
     }
-    return D.cls[p] == C_B ? it_lvl(D, real[p]) : D.ilvl[p];
+    return it_lvl(D, D.cls[p] == C_B ? real[p] : p);
 }
 
 // binary heap on (level << 24 | seq) packed keys, values = pixel ids
@@ -1592,19 +1534,12 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
     *ok = 0;
     if (N >= (size_t)INT_MAX / 8) return NSC_OK;
     Carver measure(nullptr);
-    auto carve = [&](Carver& c, uint8_t*& cls, uint16_t*& lvl0, uint8_t*& fmask, int32_t*& run, uint8_t*& st,
-                     uint8_t*& ilvl, int32_t*& pseq, int32_t*& parent, int32_t*& bnode, int32_t*& popidx, int32_t*& lab,
-                     int32_t*& head, int32_t*& real, int32_t*& lab2, uint8_t*& kind, int*& small) {
+    auto carve = [&](Carver& c, uint8_t*& cls, uint16_t*& lvl0, uint8_t*& fmask, int32_t*& run, int32_t*& lab, int32_t*& head,
+                     int32_t*& real, int32_t*& lab2, uint8_t*& kind, int*& small) {
         cls = c.take<uint8_t>(N);
         lvl0 = c.take<uint16_t>(N);
         fmask = c.take<uint8_t>(N);
         run = c.take<int32_t>(N);
-        st = c.take<uint8_t>(N);
-        ilvl = c.take<uint8_t>(N);
-        pseq = c.take<int32_t>(N);
-        parent = c.take<int32_t>(N);
-        bnode = c.take<int32_t>(N);
-        popidx = c.take<int32_t>(N);
         lab = c.take<int32_t>(N);
         head = c.take<int32_t>(N);
         real = c.take<int32_t>(N);
@@ -1612,15 +1547,15 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
         kind = c.take<uint8_t>(N);
         small = c.take<int>(64 + B1_BLOCKS);  // counters, then the per-block b1 winners
     };
-    uint8_t *cls, *fmask, *st, *ilvl, *kind;
+    uint8_t *cls, *fmask, *kind;
     uint16_t* lvl0;
-    int32_t *run, *pseq, *parent, *bnode, *popidx, *lab, *head, *real, *lab2;
+    int32_t *run, *lab, *head, *real, *lab2;
     int* small;
-    carve(measure, cls, lvl0, fmask, run, st, ilvl, pseq, parent, bnode, popidx, lab, head, real, lab2, kind, small);
+    carve(measure, cls, lvl0, fmask, run, lab, head, real, lab2, kind, small);
     Scratch sc;
     NSC_CHECK(sc.alloc(measure.size(), s));
     Carver cut(sc.p);
-    carve(cut, cls, lvl0, fmask, run, st, ilvl, pseq, parent, bnode, popidx, lab, head, real, lab2, kind, small);
+    carve(cut, cls, lvl0, fmask, run, lab, head, real, lab2, kind, small);
     // small[]: 0 nF, 1 nrun, 2 nleaf, 3 flags, 4 ncand, 8..10 info, 16 ncomp, 20 deferred tie components,
     // 24..25 tie pool bump pointer (long long), 26..31 run bucket sizes, 32..34 LDS flood queue counts,
     // 35 B pixels with queue entries, 40..44 phase-1 tier work counters
@@ -1628,8 +1563,7 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
 
     Dev D{};
     D.img = img; D.W = W; D.H = H; D.N = (int)N; D.m0 = m0; D.m = m; D.cls = cls; D.lvl0 = lvl0; D.run = run;
-    D.st = st; D.ilvl = ilvl; D.pseq = pseq; D.parent = parent; D.bnode = bnode; D.popidx = popidx; D.lab = lab;
-    D.head = head; D.nleaf = &small[2]; D.flags = &small[3];
+    D.lab = lab; D.head = head; D.nleaf = &small[2]; D.flags = &small[3];
     {  // real[] is unused until B resolution: it holds the per-workgroup counts
         const unsigned nb = (unsigned)std::min<size_t>(cdiv(N, 256), 1u << 14);
         hipLaunchKernelGGL(k_classify, dim3(nb), dim3(256), 0, s, D, cls, lvl0, fmask, real);
@@ -1643,33 +1577,28 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
     NSC_HIP(hipMemcpyAsync(hostc, small, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     NSC_HIP(stream_sync(s));
     const int nF = hostc[0], nrun = hostc[1];
-    // phase-1 scratch: run boxes, per-run FIFO heads/tails, queue links, leaf table
+    // phase-1 scratch: run boxes, per-run FIFO heads/tails, queue links, leaf table, item records
     const int leafcap = std::max(1024, std::min((int)std::min(N, (size_t)INT_MAX / 4), 4 * nF + 1024));
     Carver m2(nullptr);
-    auto carve2 = [&](Carver& c, int32_t*& box5, int*& qh, int*& qt, int32_t*& qnext, int32_t*& lf) {
+    auto carve2 = [&](Carver& c, int32_t*& box5, int*& qh, int*& qt, int32_t*& qnext, int32_t*& lf, int4*& wr) {
         box5 = c.take<int32_t>(5 * (size_t)std::max(nrun, 1));
         qh = c.take<int>((size_t)std::max(nrun, 1) * (NQ + kRunTiers));  // run buckets, then FIFO heads
         qt = c.take<int>((size_t)std::max(nrun, 1) * NQ);
         qnext = c.take<int32_t>(N + (size_t)leafcap);
-        lf = c.take<int32_t>((size_t)leafcap * 8);
+        lf = c.take<int32_t>((size_t)leafcap * 2);
+        wr = c.take<int4>(N + (size_t)leafcap);
     };
     int32_t *box5, *qnext, *lf;
     int *qh, *qt;
-    carve2(m2, box5, qh, qt, qnext, lf);
+    carve2(m2, box5, qh, qt, qnext, lf, D.wr);
     Scratch sc2;
     NSC_CHECK(sc2.alloc(m2.size(), s));
     Carver cut2(sc2.p);
-    carve2(cut2, box5, qh, qt, qnext, lf);
+    carve2(cut2, box5, qh, qt, qnext, lf, D.wr);
     D.qnext = qnext;
     D.leafcap = leafcap;
     D.lf_b = lf;
-    D.lf_run = lf + (size_t)leafcap;
-    D.lf_pseq = lf + 2 * (size_t)leafcap;
-    D.lf_parent = lf + 3 * (size_t)leafcap;
-    D.lf_bnode = lf + 4 * (size_t)leafcap;
-    D.lf_popidx = lf + 5 * (size_t)leafcap;
-    D.lf_next = lf + 6 * (size_t)leafcap;
-    D.lf_lvl = reinterpret_cast<uint8_t*>(lf + 7 * (size_t)leafcap);
+    D.lf_next = lf + (size_t)leafcap;
     if (nrun > 0) {
         NSC_CHECK(bbox_impl(run, W, H, nrun, box5, nullptr, s));
         int* lists = reinterpret_cast<int*>(qh);  // kRunTiers * nrun ints
@@ -1736,12 +1665,6 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
     int* blist = qnext;  // N + leafcap ints
     hipLaunchKernelGGL(k_collect_b0, grid1(N), dim3(256), 0, s, D, blist, &small[35]);
     if (nrun > 0) hipLaunchKernelGGL(k_link_leaves, grid1(N), dim3(256), 0, s, D, blist, &small[35]);
-    // item records for the pop-order walks (every walk comes after this point)
-    Scratch sc_items;
-    NSC_CHECK(sc_items.alloc((sizeof(int4) + 1) * ((size_t)N + leafcap) + 256, s));
-    D.wr = sc_items.as<int4>();
-    D.wl = reinterpret_cast<uint8_t*>(D.wr + ((size_t)N + leafcap));
-    hipLaunchKernelGGL(k_pack_items, grid1(N), dim3(256), 0, s, D);
     tick("phase1", &small[2]);
     // B resolution and b1
     int* cand = lab2;  // reuse (N ints)
