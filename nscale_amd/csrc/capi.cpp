@@ -289,11 +289,6 @@ hipError_t stream_sync(hipStream_t s) {
     return hipStreamSynchronize(s);
 }
 
-SideStream& side_stream() {
-    static thread_local SideStream ss;
-    return ss;
-}
-
 int ensure_init() {
     static std::once_flag once;
     static int status = NSC_OK;

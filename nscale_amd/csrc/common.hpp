@@ -163,36 +163,6 @@ inline int valid_conn(int c) { return c == 4 || c == 8; }
 
 inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
 
-// ---- fork/join onto a side stream ---------------------------------------------------------
-// Independent launches (e.g. long-latency work on a few runs beside many short ones) can overlap
-// on per-thread side streams (default priority); join() makes the caller's stream wait for them.
-struct SideStream {
-    static constexpr int K = 3;
-    hipStream_t side[K] = {nullptr, nullptr, nullptr};
-    hipEvent_t forked = nullptr, joined[K] = {nullptr, nullptr, nullptr};
-    int fork(hipStream_t s) {
-        if (!forked) {
-            NSC_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
-            for (int k = 0; k < K; ++k) {
-                NSC_HIP(hipStreamCreateWithFlags(&side[k], hipStreamNonBlocking));
-                NSC_HIP(hipEventCreateWithFlags(&joined[k], hipEventDisableTiming));
-            }
-        }
-        NSC_HIP(hipEventRecord(forked, s));
-        for (int k = 0; k < K; ++k) NSC_HIP(hipStreamWaitEvent(side[k], forked, 0));
-        return NSC_OK;
-    }
-    int join(hipStream_t s) {
-        for (int k = 0; k < K; ++k) {
-            NSC_HIP(hipEventRecord(joined[k], side[k]));
-            NSC_HIP(hipStreamWaitEvent(s, joined[k], 0));
-        }
-        return NSC_OK;
-    }
-};
-// one per host thread: concurrent callers never share a side stream
-SideStream& side_stream();
-
 // Wait for the stream.  By default the thread spins (lowest latency); a thread that has asked for
 // blocking waits (the server's workers, many of which wait at once) sleeps on an event instead.
 hipError_t stream_sync(hipStream_t s);

@@ -206,12 +206,10 @@ __global__ __launch_bounds__(1024) void k_sum_partials(const int* __restrict__ p
     if (threadIdx.x == 0) *out = t;
 }
 
-// ---- phase 1: one lane floods one run ----
-__global__ void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun, const int* __restrict__ list,
-                         const int* __restrict__ count, int* __restrict__ qh, int* __restrict__ qt) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= *count) return;
-    const int r = list[idx];
+// ---- phase 1: the flood of one run ----
+// in global memory, by one lane, for runs whose frame exceeds the LDS tiers
+__device__ void flood_global(const Dev& D, const int32_t* __restrict__ box5, int nrun, int r, int* __restrict__ qh,
+                             int* __restrict__ qt) {
     const int W = D.W;
     const int id = r + 1;
     int* head = qh + (size_t)r * NQ;  // per run (run ids are unique across the tiers)
@@ -297,9 +295,8 @@ __global__ void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun, cons
     }
 }
 
-// ---- phase 1 with the run's neighbourhood staged in LDS ----
-// Same flood as k_phase1, for runs whose bounding box plus a 2-pixel margin has at most LCAP pixels, by
-// one wave per run.  The frame is staged into LDS (the 2-pixel margin keeps every neighbour of a leaf
+// with the run's neighbourhood staged in LDS, by one wave, for runs whose bounding box plus a 2-pixel
+// margin has at most 6400 pixels: the same flood.  The frame is staged into LDS (the 2-pixel margin keeps every neighbour of a leaf
 // candidate inside it), the initial items are numbered in raster order with ballots, and the wave pops
 // item by item.
 // A flood is one chain of pops by one wave, so a pop costs the instructions it issues and the round
@@ -315,7 +312,7 @@ __global__ void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun, cons
 //  * a level that has run out finds the next queued one in one read of all 256 entries.
 //  * labels and pop indexes stay in LDS and leave for the image in one sweep after the last pop.
 // Measured: a pop takes 930 cycles; the longest flood of a 512 x 512 tile (704 pops, staging included)
-// 509 -> 291 us; the runs with frames up to 1024 pixels of a 4096 x 4096 tile 1400 -> 823 us.
+// 509 -> 291 us.
 // Each queued F pixel carries the key (level, push sequence) and frame index of its chain's largest-key
 // item, so a push compares keys without following pointers.  Leaf slots are reserved per run up front
 // (one per B pixel of the frame that could become a leaf), so no atomic sits on the flood's critical
@@ -378,54 +375,55 @@ __device__ __forceinline__ uint32_t first_queued(uint4 q) {
     return h0 != P1_NIL ? h0 : v;
 }
 
-template <int LCAP>
-__global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restrict__ box5, int nrun,
-                                                   const int* __restrict__ list, const int* __restrict__ count,
-                                                   int* __restrict__ next_run) {
-    // per frame pixel: x = class and flags | push level to the right << 8 | to the lower neighbour << 16 |
-    // level of its initial push << 24; y = frame index of a queued F pixel's chain's largest-key item, or a
-    // leaf's index in the run | FIFO link << 16; z = known label (seed label, label of a popped F pixel,
-    // else 0); w = that largest-key item's key (level << 16 | push seq), then the pixel's pop index (and
-    // its colour while the frame is staged)
-    __shared__ uint4 px[LCAP];
-    __shared__ uint4 qlv[NQ / 4];  // per level its FIFO's tail << 16 | head; empty while the head is P1_NIL
-    __shared__ int sh_base, sh_it;
+// pixels of run r's frame: its box plus the margin
+__device__ __forceinline__ int run_frame(const int32_t* __restrict__ box5, int nrun, int r) {
+    const long long L = (long long)(box5[2 * nrun + r] - box5[nrun + r] + 1 + 2 * P1_MARGIN) *
+                        (box5[4 * nrun + r] - box5[3 * nrun + r] + 1 + 2 * P1_MARGIN);
+    return (int)min(L, (long long)INT_MAX);
+}
+
+// the wave's n of a counter
+__device__ __forceinline__ int wave_take(int* counter, int n) {
+    int v = 0;
+    if ((threadIdx.x & 63) == 0) v = atomicAdd(counter, n);
+    return uni(v);
+}
+
+// the wave's own LDS accesses before this point come before those after it
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// qlv (64 entries): per level its FIFO's tail << 16 | head; empty while the head is P1_NIL.
+// px (one entry per frame pixel): x = class and flags | push level to the right << 8 | to the lower
+// neighbour << 16 | level of its initial push << 24; y = frame index of a queued F pixel's chain's
+// largest-key item, or a leaf's index in the run | FIFO link << 16; z = known label (seed label, label of a
+// popped F pixel, else 0); w = that largest-key item's key (level << 16 | push seq), then the pixel's pop
+// index (and its colour while the frame is staged)
+__device__ __forceinline__ void flood_lds(const Dev& D, const int32_t* __restrict__ box5, int nrun, int r, uint4* qlv, uint4* px) {
     any_u32* const word = reinterpret_cast<any_u32*>(px);
     any_u16* const half = reinterpret_cast<any_u16*>(px);  // pixel k's link: half[8 k + 3]
     any_u32* const entry = reinterpret_cast<any_u32*>(qlv);
     any_u16* const head = reinterpret_cast<any_u16*>(qlv);  // head[2 l]
-
-    // a fixed grid takes the tier's runs from a work counter, one at a time, so a workgroup that
-    // drew short runs takes more of them (a fixed stride over the list left the tier's time set by
-    // the workgroup that drew several long floods); launching one workgroup per run of the whole
-    // image (most of them idle for this tier) would hold the large LDS allocation of every idle
-    // workgroup across the device
-    const int nr = *count;
-    for (;;) {
-    if (threadIdx.x == 0) sh_it = atomicAdd(next_run, 1);
-    __syncthreads();
-    const int it = uni(sh_it);
-    if (it >= nr) break;
-    [&]() {  // one run; `return` ends the run
-    const int r = uni(list[it]);
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     const int W = D.W, H = D.H, id = r + 1;
     const int ox = uni(box5[nrun + r]) - P1_MARGIN, oy = uni(box5[3 * nrun + r]) - P1_MARGIN;
     const int lw = uni(box5[2 * nrun + r]) - ox + 1 + P1_MARGIN, lh = uni(box5[4 * nrun + r]) - oy + 1 + P1_MARGIN;
-    const int L = lw * lh;  // <= LCAP (bucketed by the host)
+    const int L = lw * lh;
     // k / lw by multiply-high (exact for k < 2^16)
     const uint32_t magic = (uint32_t)((0x100000000ull + (unsigned)lw - 1) / (unsigned)lw);
     const int gbase = oy * W + ox, gstep = W - lw;
     auto gidx = [&](int k) { return gbase + k + (int)__umulhi((uint32_t)k, magic) * gstep; };
 
     qlv[lane] = make_uint4(P1_EMPTY, P1_EMPTY, P1_EMPTY, P1_EMPTY);
-    // four chunks of 64 pixels at a time, every load from a clamped (always valid) pixel before any use
-    for (int k0 = 0; k0 < L; k0 += 256) {
-        uint8_t c[4], q0[4], q1[4], q2[4];
-        uint16_t l0[4];
-        int32_t rn[4], m0[4];
+    // eight chunks of 64 pixels at a time, every load from a clamped (always valid) pixel before any use
+    for (int k0 = 0; k0 < L; k0 += 512) {
+        uint8_t c[8], q0[8], q1[8], q2[8];
+        uint16_t l0[8];
+        int32_t rn[8], m0[8];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < 8; ++j) {
             const int k = min(k0 + 64 * j + lane, L - 1);
             const int ky = (int)__umulhi((uint32_t)k, magic);
             const size_t g = (size_t)clampi(oy + ky, 0, H - 1) * W + clampi(ox + k - ky * lw, 0, W - 1);
@@ -439,7 +437,7 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < 8; ++j) {
             const int k = k0 + 64 * j + lane;
             if (k >= L) continue;
             const int ky = (int)__umulhi((uint32_t)k, magic), gx = ox + k - ky * lw, gy = oy + ky;
@@ -453,7 +451,7 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
                                in ? q0[j] | (uint32_t)q1[j] << 8 | (uint32_t)q2[j] << 16 : 0u);
         }
     }
-    __syncthreads();
+    wave_lds_fence();
     // push levels between 4-neighbours (a pair that wraps around a frame row is never used: pushes
     // start at run pixels, which lie the margin away from the frame's edge)
     for (int k = lane; k < L; k += 64) {
@@ -461,7 +459,7 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
         const uint32_t rt = (uint32_t)cdiff_packed(c, cr), dn = (uint32_t)cdiff_packed(c, cl);
         word[4 * k] |= rt << 8 | dn << 16;
     }
-    __syncthreads();
+    wave_lds_fence();
     // leaf candidates (B, never initially queued, 4-adjacent to the run) and initial items in raster
     // order: a chunk's items of one level are linked in a row behind that level's FIFO (the first of
     // them reads the entry, the last writes it)
@@ -498,9 +496,8 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
         }
         seq += __popcll(bi);
     }
-    if (lane == 0) sh_base = atomicAdd(D.nleaf, cnt);
-    __syncthreads();
-    const int base = uni(sh_base);
+    wave_lds_fence();
+    const int base = wave_take(D.nleaf, cnt);
     if (base + cnt > D.leafcap) {
         // every reserved slot below the capacity reads as unused
         for (int j = base + lane; j < D.leafcap; j += 64) D.lf_b[j] = -1;
@@ -581,6 +578,7 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
         if (push && (chained || h != P1_NIL)) half[8 * tail + 3] = (uint16_t)qx;
         if (push && last) entry[lvl] = (uint32_t)sk << 16 | (h == P1_NIL ? first : h);
     }
+    wave_lds_fence();
     // labels and pop indexes (low half of a record's third word) of the run's queued pixels and of its
     // leaves (every queued item has popped)
     auto pop_of = [&](int item) -> any_u16& { return reinterpret_cast<any_u16*>(D.wr + item)[4]; };
@@ -597,29 +595,138 @@ __global__ __launch_bounds__(64) void k_phase1_lds(Dev D, const int32_t* __restr
         }
     }
     for (int j = base + nlf + lane; j < base + cnt; j += 64) D.lf_b[j] = -1;
-    }();
-    __syncthreads();  // the LDS arrays are reused by the next run
+}
+
+// ---- all run floods, from a pool of LDS per CU ----
+// One workgroup of 16 waves per CU holds all its LDS; each wave takes the next run, largest frames first,
+// and the LDS that run's frame needs, in 1 KB units.  A flood is a chain of dependent steps that leaves most
+// issue slots of its SIMD idle, so what counts is how many are in flight: by frame size (launches per size
+// tier, each with its tier's LDS, held a third less and each tier ended with its own few longest floods).
+// Measured: 363 -> 315 us for a 512 x 512 tile (its longest flood alone is 290), 823 -> 689 us for a
+// 4096 x 4096 one.
+constexpr int P1_WAVES = 16, P1_UNITS = 158;  // 64 frame pixels a unit
+constexpr int kRunTiers = 6;
+// runs by the size of their LDS frame: tier b holds frames of at most kRunTier[b] pixels; the last one
+// floods from global memory
+__constant__ int kRunTier[kRunTiers - 1] = {512, 1024, 2048, 4096, 6400};
+
+struct LdsPool {
+    unsigned long long used[3];
+    int lock;
+    // the lowest n free units in a row, taken (-1: none now).  Wave-uniform.
+    __device__ int take(int n, int lane) {
+        enter(lane);
+        unsigned long long f[3], r[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            f[k] = ~used[k];
+            r[k] = f[k];
+        }
+        for (int len = 1; len < n;) {  // r: units that start len free ones
+            const int sh = min(len, n - len);
+            if (sh == 64) {
+                r[0] &= r[1]; r[1] &= r[2]; r[2] = 0;
+            } else {
+                r[0] &= r[0] >> sh | r[1] << (64 - sh);
+                r[1] &= r[1] >> sh | r[2] << (64 - sh);
+                r[2] &= r[2] >> sh;
+            }
+            len += sh;
+        }
+        int at = -1;
+#pragma unroll
+        for (int k = 2; k >= 0; --k) at = r[k] ? 64 * k + __builtin_ctzll(r[k]) : at;
+        at = uni(at);
+        if (at >= 0) mark(at, n, lane, true);
+        leave(lane);
+        return at;
+    }
+    __device__ void give(int at, int n, int lane) {
+        enter(lane);
+        mark(at, n, lane, false);
+        leave(lane);
+    }
+    __device__ void mark(int at, int n, int lane, bool on) {
+        if (lane < 3) {
+            const int lo = max(at - 64 * lane, 0), hi = min(at + n - 64 * lane, 64);
+            if (lo < hi) {
+                const unsigned long long m = (hi - lo == 64 ? ~0ull : (1ull << (hi - lo)) - 1ull) << lo;
+                used[lane] = on ? used[lane] | m : used[lane] & ~m;
+            }
+        }
+    }
+    __device__ void enter(int lane) {
+        if (lane == 0) {
+            int was = 0;
+            while (!__hip_atomic_compare_exchange_strong(&lock, &was, 1, __ATOMIC_ACQUIRE, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_WORKGROUP)) {
+                was = 0;
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __device__ void leave(int lane) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) __hip_atomic_store(&lock, 0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+};
+
+__global__ __launch_bounds__(64 * P1_WAVES) void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun,
+                                                          const int* __restrict__ lists, const int* __restrict__ counts,
+                                                          int* __restrict__ next_run, int* __restrict__ qh, int* __restrict__ qt) {
+    __shared__ uint4 pool[64 * P1_UNITS];
+    __shared__ LdsPool P;
+    const int lane = threadIdx.x & 63, wave = uni((int)(threadIdx.x >> 6));
+    if (threadIdx.x == 0) {
+        P.used[0] = P.used[1] = 0;
+        P.used[2] = ~0ull << (P1_UNITS - 128);
+        P.lock = 0;
+    }
+    __syncthreads();  // the only one: the waves go their own ways below
+    // first runs spread over the workgroups, further ones from the counter
+    int it = wave * (int)gridDim.x + (int)blockIdx.x;
+    for (;;) {
+        int r = -1, tier = 0, k = it;
+        for (int t = kRunTiers - 1; t >= 0 && r < 0; --t) {
+            const int c = uni(counts[t]);
+            if (k < c) {
+                r = uni(lists[(size_t)t * nrun + k]);
+                tier = t;
+            } else {
+                k -= c;
+            }
+        }
+        if (r < 0) break;
+        if (tier == kRunTiers - 1) {
+            if (lane == 0) flood_global(D, box5, nrun, r, qh, qt);
+        } else {
+            const int L = uni(run_frame(box5, nrun, r));
+            const int n = 1 + (L + 63) / 64;  // 102 at most: the pool holds it once the floods in flight are done
+            int at;
+            while ((at = P.take(n, lane)) < 0) __builtin_amdgcn_s_sleep(64);
+            flood_lds(D, box5, nrun, r, pool + 64 * at, pool + 64 * (at + 1));
+            P.give(at, n, lane);
+        }
+        it = wave_take(next_run, 1) + P1_WAVES * (int)gridDim.x;
     }
 }
 
-// LDS bytes of one k_phase1_lds<LCAP> workgroup (the host sizes each tier's grid from it)
-constexpr int p1_lds_bytes(int lcap) { return 16 * lcap + 4 * NQ + 8; }
 
-// grid of a k_phase1_lds<LCAP> launch: the workgroups the device holds at once (LDS-bound), at most
-// one per run of the image
-template <int LCAP>
-int p1_grid(int nrun) {
-    static const int g = [] {
-        int dev = 0, per_cu = 0, cus = 0;
+// compute units of the current device (the grid of the run floods)
+static int device_cus() {
+    static const int n = [] {
+        int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_phase1_lds<LCAP>, 64, 0) != hipSuccess) {
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
             (void)hipGetLastError();
-            return 256 * std::max(1, 160 * 1024 / p1_lds_bytes(LCAP));
+            return 256;
         }
-        return std::max(1, per_cu) * std::max(1, cus);
+        return std::max(1, cus);
     }();
-    return std::max(1, std::min(nrun, g));
+    return n;
 }
 
 // wave-aggregated append of the lanes whose `take` is set
@@ -672,18 +779,12 @@ __global__ void k_collect_b0(Dev D, int* __restrict__ blist, int* __restrict__ b
     }
 }
 
-// runs by the size of their LDS frame (box + 1-pixel margin): bucket b holds frames of at most
-// kRunTier[b] pixels; the last bucket floods from global memory
-constexpr int kRunTiers = 6;
-
-__constant__ int kRunTier[kRunTiers - 1] = {512, 1024, 2048, 4096, 6400};
 // (one append per wave and bucket: an atomic per run on the few bucket counters serialises)
 __global__ void k_bucket_runs(const int32_t* __restrict__ box5, int nrun, int* __restrict__ lists, int* __restrict__ counts) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     int b = -1;
     if (r < nrun) {
-        const long long L = (long long)(box5[2 * nrun + r] - box5[nrun + r] + 1 + 2 * P1_MARGIN) *
-                            (box5[4 * nrun + r] - box5[3 * nrun + r] + 1 + 2 * P1_MARGIN);
+        const int L = run_frame(box5, nrun, r);
         b = 0;
         while (b < kRunTiers - 1 && L > kRunTier[b]) ++b;
     }
@@ -1624,41 +1725,9 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
             for (int b = 0; b < kRunTiers; ++b)
                 fprintf(stderr, "[ws] tier %d: runs %d, box px %lld, max %lld\n", b, bc[b], area[b], amax[b]);
         }
-        auto L = [&](int b) { return lists + (size_t)b * nrun; };
-        // the few large runs set the latency: the largest tiers start first, each on a side stream,
-        // beside the many small runs on the caller's stream (the 1024 tier, then the 512 tier: the
-        // tiers share the LDS, so the order decides little; measured against the 512 tier after the
-        // 2048 tier, this was 0.07 ms shorter on the same box)
-        // grids: the workgroups the device holds at once per tier (idle ones exit at once); on a
-        // serving thread the tier counts are read and each grid holds one workgroup per run at most
-        // (idle workgroups of the large tiers would wait for a CU with their LDS free, beside the
-        // other slots' kernels), and empty tiers launch nothing
-        int tier_runs[kRunTiers];
-        const bool exact = thread_serving();
-        if (exact) {
-            NSC_HIP(hipMemcpyAsync(tier_runs, bcount, sizeof(tier_runs), hipMemcpyDeviceToHost, s));
-            NSC_HIP(stream_sync(s));
-        }
-        auto grid = [&](int b, int resident) { return exact ? std::min(tier_runs[b], resident) : resident; };
-        SideStream& ss = side_stream();
-        NSC_CHECK(ss.fork(s));
-        int* next_run = &small[40];  // per-tier work counters (zeroed with small[])
-        if (const int g = grid(4, std::min(nrun, 64)))
-            hipLaunchKernelGGL(k_phase1_lds<6400>, dim3(g), dim3(64), 0, ss.side[0], D, box5, nrun, L(4), bcount + 4,
-                               next_run + 4);
-        if (const int g = exact ? (int)cdiv(tier_runs[5], 64) : (int)cdiv(nrun, 64))
-            hipLaunchKernelGGL(k_phase1, dim3(g), dim3(64), 0, ss.side[0], D, box5, nrun, L(5), bcount + 5, qh2, qt);
-        if (const int g = grid(3, p1_grid<4096>(nrun)))
-            hipLaunchKernelGGL(k_phase1_lds<4096>, dim3(g), dim3(64), 0, ss.side[1], D, box5, nrun, L(3), bcount + 3,
-                               next_run + 3);
-        if (const int g = grid(2, p1_grid<2048>(nrun)))
-            hipLaunchKernelGGL(k_phase1_lds<2048>, dim3(g), dim3(64), 0, ss.side[2], D, box5, nrun, L(2), bcount + 2,
-                               next_run + 2);
-        if (const int g = grid(1, p1_grid<1024>(nrun)))
-            hipLaunchKernelGGL(k_phase1_lds<1024>, dim3(g), dim3(64), 0, s, D, box5, nrun, L(1), bcount + 1, next_run + 1);
-        if (const int g = grid(0, p1_grid<512>(nrun)))
-            hipLaunchKernelGGL(k_phase1_lds<512>, dim3(g), dim3(64), 0, s, D, box5, nrun, L(0), bcount, next_run);
-        NSC_CHECK(ss.join(s));
+        // four runs a workgroup (one per SIMD) before a further CU is taken whole
+        const int g = std::max(1, std::min((int)cdiv(nrun, 4), device_cus()));
+        hipLaunchKernelGGL(k_phase1, dim3(g), dim3(64 * P1_WAVES), 0, s, D, box5, nrun, lists, bcount, &small[40], qh2, qt);
     }
     // B pixels with a queue entry: initially queued ones, then those with leaves (the phase-1
     // queue links are dead from here on and hold the list)
