@@ -16,7 +16,8 @@
 //      - row state (lane = row, after a transpose through LDS): left-right and right-left
 //        sweeps, out = min(max(out, left, up-left, down-left), mask) (the diagonal neighbours only
 //        with 8-connectivity; right instead of left for the right-left sweep).
-//    The two sweeps of each state run as two interleaved chains updating the values in place.
+//    The two sweeps of each state run as two interleaved chains updating the values in place
+//    (uint8: both in one packed register, see recon_tile_u8).
 //    A fixpoint of these four sweeps satisfies every 8- (or 4-) neighbour constraint.
 //  * Pass 0 runs every tile once, reading marker and mask (halo = min(marker, mask)) and writing
 //    the output: 3 bytes/px for uint8, the algorithmic minimum.  A tile whose owned border
@@ -43,6 +44,7 @@ namespace {
 #ifndef RECON_WAVES
 #define RECON_WAVES 2
 #endif
+template <typename T> constexpr int recon_waves() { return sizeof(T) == 1 ? 4 : RECON_WAVES; }
 
 constexpr int TW = 64;  // window width (= wave size)
 constexpr int TH = 64;  // window height
@@ -168,9 +170,9 @@ __device__ __forceinline__ int32_t nbr3(int32_t pc) {
 
 // Mask of a window in both orientations, in registers, so the sweeps never touch LDS for it:
 // column state (mc: the lane's column, filled while the window loads) and row state (mr: the
-// lane's row, read back transposed from the LDS staging copy).  uint8: packed four to a register
-// (rows / columns 4j..4j+3).  Four-byte types: one value per register (192 registers with the
-// window itself, which keeps two waves per SIMD with the staging buffer shared by the transposes).
+// lane's row, read back transposed from the LDS staging copy).  One value per register (192 registers
+// with the window itself, which keeps two waves per SIMD with the staging buffer shared by the
+// transposes).
 template <typename T>
 struct WinMask {
     using R = typename RegOf<T>::type;
@@ -186,39 +188,13 @@ struct WinMask {
     __device__ __forceinline__ R clamp_row(R v, R n, int x) const { return clamp_up(v, n, mr[x]); }
     static __device__ __forceinline__ void fence(int) {}
 };
-template <>
-struct WinMask<uint8_t> {
-    const uint8_t (*lm)[TW + 4];
-    int lane;
-    uint32_t mc[TH / 4], mr[TW / 4];
-    // mc is filled while the window loads; mr comes from the LDS copy (row `lane`, 4-byte words)
-    __device__ __forceinline__ void build() {
-#pragma unroll
-        for (int j = 0; j < TW / 4; ++j) mr[j] = *reinterpret_cast<const uint32_t*>(&lm[lane][4 * j]);
-    }
-    // called at the top of every round: hides the packed words from loop-invariant code motion,
-    // which would otherwise unpack all 124 masks once before the loop and spill them
-    __device__ __forceinline__ void opaque() {
-#pragma unroll
-        for (int j = 0; j < TH / 4; ++j) asm volatile("" : "+v"(mc[j]), "+v"(mr[j]));
-    }
-    // min(max(v, n), mask byte): the byte extraction folds into the min as an SDWA operand select
-    __device__ __forceinline__ uint32_t clamp_col(uint32_t v, uint32_t n, int y) const {
-        return min(max(v, n), (mc[y >> 2] >> (8 * (y & 3))) & 0xFFu);
-    }
-    __device__ __forceinline__ uint32_t clamp_row(uint32_t v, uint32_t n, int x) const {
-        return min(max(v, n), (mr[x >> 2] >> (8 * (x & 3))) & 0xFFu);
-    }
-    static __device__ __forceinline__ void fence(int) {}
-};
-
 // one round of the four direction sweeps over a window held in v (column state on entry and exit).
 // The down and up sweeps run as two interleaved chains, each updating v in place: step k moves the
 // down chain to row k and the up chain to row 63 - k, so the two dependency chains overlap in the
 // pipeline instead of one waiting on the other.  Every update is min(max(v, neighbours), mask) of
 // current values, a valid relaxation whatever the other chain has written, and past the middle each
 // chain reads what the other has already raised.  Rows likewise with the left and right sweeps.
-// (uint8: whether anything changed is decided by the caller from column sums)
+// (whether anything changed is decided by the caller from column sums)
 template <typename T, int CONN>
 __device__ __forceinline__ void sweep_round(typename RegOf<T>::type (&v)[TH], WinMask<T>& M, T (*tr)[TW + 1],
                                             int lane) {
@@ -289,13 +265,266 @@ __device__ __forceinline__ auto col_sum(const R (&v)[TH]) {
     return s;
 }
 
+// ---- uint8 windows: two values to a register -------------------------------------------------
+// The two chains of a sweep start at opposite ends, so values k and 63 - k of the lane's line share a
+// register as 16-bit halves (pair k) and one packed max / min steps both chains.  Past the middle each
+// chain runs on in the other half: the carried value is swapped once.  Against a value per register
+// this halves the sweeps' registers (116: four waves per SIMD instead of two) and, with 4-connectivity,
+// their instructions; transposes move pairs (LDS word [row][k] = pair k of the row) and read or write the
+// lane's column half by half.
+//  * Loads: the lane's row of the window, 64 contiguous bytes in four 16-byte loads (all of a window's
+//    loads in flight at once).  Windows that would read before the first or past the last pixel of the
+//    plane take 4-byte loads at addresses clamped into it.
+//  * A window is stable once a sweep of each orientation in turn changes nothing, and a sweep that changed
+//    something satisfies its own constraints with 4-connectivity (a line's two chains reach the line's
+//    fixpoint), so there the first unchanged sweep after another ends the solve.
+// With 8-connectivity the column sweep takes the diagonals too, as the row sweep does: without them a
+// step is 2 instructions instead of 5, but the first pass of a batch was 12 % slower and a 512 x 512 chain's
+// passes a third (more rounds).
+// Measured: the passes of 64 pairs (370 Mpixel) 4160 -> 2420 us, the first of them 1327 -> 641; a 4096 x 4096
+// pair's first pass 79 -> 52; the 21 passes of a 512 x 512 chain 316 -> 276.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t __attribute__((may_alias)) any_u16;
+typedef uint32_t __attribute__((ext_vector_type(4), may_alias)) u32x4;
+// accesses at any address
+typedef uint32_t __attribute__((ext_vector_type(4), aligned(1), may_alias)) u32x4_any;
+typedef uint32_t __attribute__((aligned(1), may_alias)) u32_any;
+typedef uint16_t __attribute__((aligned(1), may_alias)) u16_any;
+#define GLOBAL_AS __attribute__((address_space(1)))
+template <>
+struct RShared<uint8_t> {
+    alignas(16) uint32_t t[TH][TW / 2 + 4];  // rows 144 bytes apart: 16-byte accesses of 16 rows meet no bank twice
+    unsigned chg_bits;
+};
+
+__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+// maximum of three pairs of values up to 255: as half floats these are subnormal numbers, which have the
+// integers' order and pass through the maximum unchanged
+__device__ __forceinline__ uint32_t pk_max3(uint32_t a, uint32_t b, uint32_t c) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_maximum(
+        __builtin_elementwise_maximum(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b)), __builtin_bit_cast(f16x2, c)));
+}
+// one step: v raised by the pair p before it and, with DIAG, by p of both lane neighbours (lanes 0 and 63,
+// always frozen, see 0 outside the wave), under the mask m
+template <bool DIAG>
+__device__ __forceinline__ uint32_t pk_step(uint32_t v, uint32_t p, uint32_t m) {
+    uint32_t n = pk_max(v, p);
+    if (DIAG) {
+        const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p, 0x138, 0xF, 0xF, true);
+        const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)p, 0x130, 0xF, 0xF, true);
+        n = pk_max3(l, r, n);
+    }
+    return pk_min(n, m);
+}
+// both chains of a line, in place; pair 0 (the halo) is only read
+template <bool DIAG>
+__device__ __forceinline__ void pk_sweep(uint32_t (&v)[TW / 2], const uint32_t (&m)[TW / 2]) {
+    uint32_t p = v[0];
+#pragma unroll
+    for (int k = 1; k < TW / 2; ++k) p = v[k] = pk_step<DIAG>(v[k], p, m[k]);
+    p = __builtin_amdgcn_alignbit(p, p, 16);
+#pragma unroll
+    for (int k = TW / 2 - 1; k > 0; --k) p = v[k] = pk_step<DIAG>(v[k], p, m[k]);
+}
+// sums of both halves (64 x 255 fits 16 bits)
+__device__ __forceinline__ uint32_t pk_sum(const uint32_t (&v)[TW / 2]) {
+    uint32_t a = v[0] + v[1], b = v[2] + v[3];
+#pragma unroll
+    for (int k = 4; k < TW / 2; k += 4) {
+        a += v[k] + v[k + 1];
+        b += v[k + 2] + v[k + 3];
+    }
+    return a + b;
+}
+// byte x of a row of 16 words, as the low (x) and high (63 - x) half of a pair
+__device__ __forceinline__ uint32_t pk_unpack(const uint32_t (&d)[TW / 4], int x) {
+    return __builtin_amdgcn_perm(d[15 - (x >> 2)], d[x >> 2], (uint32_t)(0x0C000C00 | (x & 3) | (7 - (x & 3)) << 16));
+}
+
+// 64 bytes at element a of a plane of n bytes (reads stay inside the plane; bytes outside it are anything)
+__device__ __forceinline__ void load_row64(const GLOBAL_AS uint8_t* p, long long a, long long n, bool whole,
+                                           uint32_t (&d)[TW / 4]) {
+    if (whole) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x4_any q = *reinterpret_cast<const GLOBAL_AS u32x4_any*>(p + a + 16 * j);
+            d[4 * j] = q.x; d[4 * j + 1] = q.y; d[4 * j + 2] = q.z; d[4 * j + 3] = q.w;
+        }
+    } else if (n >= 4) {
+#pragma unroll
+        for (int j = 0; j < TW / 4; ++j) {
+            const long long e = a + 4 * j, c = e < 0 ? 0 : (e > n - 4 ? n - 4 : e);
+            const uint32_t q = *reinterpret_cast<const GLOBAL_AS u32_any*>(p + c);
+            const int s = (int)(e - c < -3 ? -3 : (e - c > 3 ? 3 : e - c));  // bytes the word was moved by
+            d[j] = s < 0 ? q << (-8 * s) : q >> (8 * s);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < TW / 4; ++j) {
+            d[j] = 0;
+            for (int b = 0; b < 4; ++b) {
+                const long long e = a + 4 * j + b;
+                if (e >= 0 && e < n) d[j] |= (uint32_t)p[e] << (8 * b);
+            }
+        }
+    }
+}
+
+template <int CONN>
+__device__ __forceinline__ void recon_tile_u8(const RImg<uint8_t>& im, int tile, int pass, RShared<uint8_t>& sh,
+                                              int* __restrict__ next_list, int* __restrict__ next_count,
+                                              unsigned* __restrict__ stamp, unsigned long long* dirty) {
+    constexpr int HW = TW / 2;
+    const int w = im.w, h = im.h, tiles_x = im.tiles_x, tiles_y = im.tiles_y;
+    const int tx = tile % tiles_x, ty = tile / tiles_x;
+    const int lane = threadIdx.x;
+    const int gx0 = tx * OW - 1, gy = ty * OH - 1 + lane;
+    const bool row_in = gy >= 0 && gy < h;
+    if (lane == 0) sh.chg_bits = 0;
+
+    uint32_t v[HW], mr[HW], mc[HW];  // the window in the current state, its mask in row and in column state
+    {
+        const long long n = (long long)w * h, a = (long long)clampi(gy, 0, h - 1) * w + gx0;
+        const bool whole = __all(a >= 0 && a + TW <= n);
+        uint32_t ds[TW / 4], dm[TW / 4];
+        load_row64(as_global(pass == 0 ? im.marker : (const uint8_t*)im.out), a, n, whole, ds);
+        load_row64(as_global(im.mask), a, n, whole, dm);
+        __builtin_amdgcn_sched_barrier(0);
+        const bool inside = gx0 >= 0 && gx0 + TW <= w;
+#pragma unroll
+        for (int k = 0; k < HW; ++k) {
+            uint32_t keep = row_in ? ~0u : 0u;  // pixels outside the image hold the frame value 0
+            if (!inside)
+                keep &= (gx0 + k >= 0 && gx0 + k < w ? 0xFFFFu : 0u) | (gx0 + TW - 1 - k < w ? 0xFFFF0000u : 0u);
+            const uint32_t mk = pk_unpack(dm, k) & keep;
+            v[k] = pk_min(pk_unpack(ds, k), mk);
+            // frozen: the halo rows and columns (the rest outside the image is 0 under 0)
+            mr[k] = k == 0 || lane == 0 || lane == TW - 1 ? v[k] : mk;
+        }
+    }
+    const uint32_t init_lr = v[1], init_row = pk_sum(v);
+    const int col = lane < HW ? 2 * lane : 2 * (TW - 1 - lane) + 1;  // the lane's column: a 16-bit half of a row's words
+    any_u16* const tc = reinterpret_cast<any_u16*>(&sh.t[0][0]) + col;
+    constexpr int RS = 2 * (HW + 4);  // halves from row to row
+    auto put_rows = [&](const uint32_t (&x)[HW]) {
+#pragma unroll
+        for (int k = 0; k < HW; k += 4)
+            *reinterpret_cast<u32x4*>(&sh.t[lane][k]) = u32x4{x[k], x[k + 1], x[k + 2], x[k + 3]};
+    };
+    auto get_cols = [&](uint32_t (&x)[HW]) {
+#pragma unroll
+        for (int k = 0; k < HW; ++k) {
+            u16x2 q;
+            q.x = tc[k * RS];
+            q.y = tc[(TH - 1 - k) * RS];
+            x[k] = __builtin_bit_cast(uint32_t, q);
+        }
+    };
+    put_rows(mr);
+    __syncthreads();
+    get_cols(mc);
+    __syncthreads();
+
+    uint32_t row_sum = init_row;
+    bool still = false;  // the last column sweep changed nothing
+    for (int round = 0; round < 4096; ++round) {
+        pk_sweep<CONN == 8>(v, mr);
+        const uint32_t rs = pk_sum(v);
+        const bool same = !__any(rs != row_sum);
+        if (same && (still || (CONN == 4 && round > 0))) break;
+        put_rows(v);
+        __syncthreads();
+        get_cols(v);
+        const uint32_t cs = pk_sum(v);
+        pk_sweep<CONN == 8>(v, mc);
+        still = !__any(pk_sum(v) != cs);
+#pragma unroll
+        for (int k = 0; k < HW; ++k) {
+            const u16x2 q = __builtin_bit_cast(u16x2, v[k]);
+            tc[k * RS] = q.x;
+            tc[(TH - 1 - k) * RS] = q.y;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < HW; k += 4) {
+            const u32x4 q = *reinterpret_cast<const u32x4*>(&sh.t[lane][k]);
+            v[k] = q.x; v[k + 1] = q.y; v[k + 2] = q.z; v[k + 3] = q.w;
+        }
+        __syncthreads();
+        row_sum = pk_sum(v);
+        if (still && (same || CONN == 4)) break;
+    }
+    const bool row_changed = row_sum != init_row;  // (the last row sweep of a finished solve changed nothing)
+    // pass 0 writes every owned pixel (the output starts as min(marker, mask)); later passes only
+    // rewrite tiles that changed
+    if (pass != 0 && !__any(row_changed)) return;
+
+    // ---- the lane's owned pixels: bytes 1..62 of its row ----
+    if (lane >= 1 && lane <= TW - 2 && row_in) {
+        uint32_t d[TW / 4], o[TW / 4];
+#pragma unroll
+        for (int j = 0; j < TW / 8; ++j) {
+            const uint32_t a = __builtin_amdgcn_perm(v[4 * j + 1], v[4 * j], 0x02060400u);      // x, x + 1, mirrored
+            const uint32_t b = __builtin_amdgcn_perm(v[4 * j + 3], v[4 * j + 2], 0x02060400u);
+            d[j] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+            d[15 - j] = __builtin_amdgcn_perm(a, b, 0x07060302u);
+        }
+#pragma unroll
+        for (int j = 0; j < TW / 4; ++j) o[j] = j < 15 ? __builtin_amdgcn_alignbit(d[j + 1], d[j], 8) : d[j] >> 8;
+        const auto g = as_global(im.out) + (size_t)gy * w + tx * OW;
+        const int nc = min(OW, w - tx * OW);  // owned columns inside the image
+        if (nc == OW) {
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                u32x4_any q = {o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]};
+                *reinterpret_cast<GLOBAL_AS u32x4_any*>(g + 16 * j) = q;
+            }
+#pragma unroll
+            for (int j = 12; j < 15; ++j) *reinterpret_cast<GLOBAL_AS u32_any*>(g + 4 * j) = o[j];
+            *reinterpret_cast<GLOBAL_AS u16_any*>(g + 60) = (uint16_t)o[15];
+        } else {
+#pragma unroll
+            for (int j = 0; j < TW / 4; ++j) {
+                if (4 * j + 4 <= nc) *reinterpret_cast<GLOBAL_AS u32_any*>(g + 4 * j) = o[j];
+                else
+                    for (int b = 0; b < 4; ++b)
+                        if (4 * j + b < nc) g[4 * j + b] = (uint8_t)(o[j] >> (8 * b));
+            }
+        }
+    }
+    // ---- owned-border changes -> mark neighbours ----
+    unsigned bits = 0;
+    if (lane >= 1 && lane <= TW - 2) {
+        if (lane == 1 && row_changed) bits |= CH_TOP;
+        if (lane == TW - 2 && row_changed) bits |= CH_BOT;
+        if ((v[1] ^ init_lr) & 0xFFFFu) bits |= CH_LEFT;
+        if ((v[1] ^ init_lr) >> 16) bits |= CH_RIGHT;
+    }
+    if (dirty) __threadfence();  // the owned pixels are visible before any neighbour is marked
+    if (bits) atomicOr(&sh.chg_bits, bits);
+    __syncthreads();
+    if (dirty)
+        mark_neighbours_bits(lane, sh.chg_bits, tx, ty, tiles_x, tiles_y, im.base, false, dirty);
+    else
+        mark_neighbours(lane, sh.chg_bits, tx, ty, tiles_x, tiles_y, im.base, false, (unsigned)pass + 1, stamp, next_list,
+                        next_count);
+}
+
 // one tile of one image: load window, sweep to stability, write owned pixels, mark neighbours
 template <typename T, int CONN, bool HD = false>
 __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass, RShared<T>& sh, int* __restrict__ next_list,
                                            int* __restrict__ next_count, unsigned* __restrict__ stamp,
                                            unsigned long long* dirty = nullptr) {
+    if constexpr (std::is_same<T, uint8_t>::value) {
+        recon_tile_u8<CONN>(im, tile, pass, sh, next_list, next_count, stamp, dirty);
+    } else {
     using R = typename RegOf<T>::type;
-    constexpr bool U8 = std::is_same<T, uint8_t>::value;
     auto& lm = sh.lm;
     auto& init_l = sh.init_l;
     auto& init_r = sh.init_r;
@@ -348,12 +577,7 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
             v[y] = val;
             const R mw = frozen ? val : mk;
             lm[y][lane] = (T)mw;
-            if constexpr (U8) {
-                if ((y & 3) == 0) M.mc[y >> 2] = 0;
-                M.mc[y >> 2] |= (uint32_t)mw << (8 * (y & 3));
-            } else {
-                M.mc[y] = mw;
-            }
+            M.mc[y] = mw;
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -423,6 +647,7 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
     else
         mark_neighbours(lane, chg_bits, tx, ty, tiles_x, tiles_y, im.base, false, (unsigned)pass + 1, stamp, next_list,
                         next_count);
+    }
 }
 
 // Pass 0 runs every tile of every image; pass k > 0 runs the tiles listed by pass k - 1.  Blocks
@@ -450,7 +675,7 @@ __device__ __forceinline__ void recon_tiles_body(RShared<T>& sh, const RImg<T>* 
 }
 
 template <typename T, int CONN, bool HD>
-__global__ __launch_bounds__(64, RECON_WAVES) void recon_tiles(const RImg<T>* __restrict__ imgs, RImg<T> one, const int* __restrict__ tile_img,
+__global__ __launch_bounds__(64, recon_waves<T>()) void recon_tiles(const RImg<T>* __restrict__ imgs, RImg<T> one, const int* __restrict__ tile_img,
                                                   int ntiles, const int* __restrict__ list, const int* __restrict__ list_count,
                                                   int* __restrict__ next_list, int* __restrict__ next_count,
                                                   int* __restrict__ clear_count, unsigned* __restrict__ stamp, int pass,
@@ -520,7 +745,7 @@ __device__ __forceinline__ void drain_release(int got, unsigned long long* busy,
 }
 
 template <typename T, int CONN>
-__global__ __launch_bounds__(64, RECON_WAVES) void recon_drain(const RImg<T>* __restrict__ imgs, RImg<T> one,
+__global__ __launch_bounds__(64, recon_waves<T>()) void recon_drain(const RImg<T>* __restrict__ imgs, RImg<T> one,
                                                                const int* __restrict__ tile_img, int nwords,
                                                                unsigned long long* dirty, unsigned long long* busy,
                                                                int* running, int spin_limit) {
@@ -1231,7 +1456,7 @@ namespace {
 // passes past convergence cost a near-empty launch; the host checks the last pass's count once per
 // replay.  Every clear is a kernel (nothing a graph would record as a runtime fill).
 template <typename T, int CONN>
-__global__ __launch_bounds__(64, RECON_WAVES) void recon_tiles_graph(const RImg<T>* __restrict__ imgs,
+__global__ __launch_bounds__(64, recon_waves<T>()) void recon_tiles_graph(const RImg<T>* __restrict__ imgs,
                                                                      const int* __restrict__ tile_img, int ntiles,
                                                                      int* __restrict__ listA, int* __restrict__ listB,
                                                                      int* __restrict__ counts, unsigned* __restrict__ stamp,
