@@ -496,6 +496,7 @@ __device__ __forceinline__ void flood_lds(const Dev& D, const int32_t* __restric
         }
         seq += __popcll(bi);
     }
+    if (!seq) return;  // nothing queued initially: the run is not flooded in this phase and takes no leaf slots
     wave_lds_fence();
     const int base = wave_take(D.nleaf, cnt);
     if (base + cnt > D.leafcap) {
