@@ -11,9 +11,11 @@
 //   3. the output is the min/max over kernel rows of the run result of the matching window row.
 // Traffic: 1 byte in + 1 byte out per pixel (plus the halo re-read, r/32 of the tile).
 // The window and run results are held as 16-bit pixel pairs where that fits in LDS (morph2_kernel),
-// else as bytes (morph_kernel).  3 x 3 elements take a direct kernel instead (morph3_kernel).
+// else as bytes (morph_kernel).  3 x 3 elements (morph3_kernel) and the chain's 19 x 19 disk (morph_disk)
+// have kernels of their own.
 #include <algorithm>
 #include <cstdint>
+#include <cstdlib>
 #include <vector>
 
 #include "common.hpp"
@@ -240,6 +242,195 @@ __global__ __launch_bounds__(M2_THREADS) void morph2_kernel(const uint8_t* __res
     }
 }
 
+// ---- the chain's 19 x 19 disk ------------------------------------------------------------------
+// The disk of the chain's morphOpen is { max(|x| - 5, 0) + max(|y| - 5, 0) <= 4 }: an
+// 11 x 11 square widened by a diamond of radius 4, so its minimum is the square's (11 across, 11 down) taken
+// through four 3 x 3 crosses.  A wave runs down a strip of 512 columns with everything in registers: a
+// lane holds 8 columns as 16-bit pairs, neighbour columns come from the next lanes, and the last few
+// rows of every stage are kept (three-operand minima: values up to 255 are subnormal half floats, which
+// order as integers do).  110 instructions per row make 488 outputs; the general kernel reads 19 LDS
+// words per 4 outputs after 19 taps a pixel, and is LDS bound.
+// Rows per strip: a strip reads 18 rows more than it makes, so long strips waste less and short ones
+// fill the chip; the longest of 32, 16 and 8 that leaves two waves per SIMD.
+// Measured (erosion or dilation): 4096 x 4096 135 -> 31 us, 512 x 512 17 -> 14.
+constexpr int DSQ = 5, DDI = 4, DRAD = DSQ + DDI, DK = 2 * DRAD + 1;
+constexpr int DOUT = 61 * 8;  // output columns of a strip: lanes 1..61
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+template <bool ERODE>
+__device__ __forceinline__ uint32_t pick3(uint32_t a, uint32_t b, uint32_t c) {
+    const f16x2 x = __builtin_bit_cast(f16x2, a), y = __builtin_bit_cast(f16x2, b), z = __builtin_bit_cast(f16x2, c);
+    return __builtin_bit_cast(uint32_t, ERODE ? __builtin_elementwise_minimum(__builtin_elementwise_minimum(x, y), z)
+                                              : __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y), z));
+}
+__device__ __forceinline__ uint32_t next_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, true); }
+__device__ __forceinline__ uint32_t prev_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true); }
+// the pair that straddles pairs a and b (a before b)
+__device__ __forceinline__ uint32_t straddle(uint32_t a, uint32_t b) { return __builtin_amdgcn_alignbit(b, a, 16); }
+
+struct Row8 {
+    uint32_t p[4];  // columns 2 j, 2 j + 1 of the lane
+};
+// minimum over columns x .. x + 10
+template <bool ERODE>
+__device__ __forceinline__ Row8 across11(const Row8& r) {
+    const uint32_t* p = r.p;
+    Row8 a, b, c, o;
+    const uint32_t n0 = next_lane(p[0]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a.p[j] = pick2<ERODE>(p[j], straddle(p[j], j < 3 ? p[j + 1] : n0));  // 2
+    const uint32_t n1 = next_lane(a.p[0]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b.p[j] = pick2<ERODE>(a.p[j], j < 3 ? a.p[j + 1] : n1);  // 4
+    const uint32_t n2 = next_lane(b.p[0]), n3 = next_lane(b.p[1]);
+    c.p[0] = pick2<ERODE>(b.p[0], b.p[2]);  // 8
+    c.p[1] = pick2<ERODE>(b.p[1], b.p[3]);
+    c.p[2] = pick2<ERODE>(b.p[2], n2);
+    c.p[3] = pick2<ERODE>(b.p[3], n3);
+    const uint32_t n4 = next_lane(c.p[0]), n5 = next_lane(c.p[1]);
+    o.p[0] = pick2<ERODE>(c.p[0], straddle(c.p[1], c.p[2]));  // 11
+    o.p[1] = pick2<ERODE>(c.p[1], straddle(c.p[2], c.p[3]));
+    o.p[2] = pick2<ERODE>(c.p[2], straddle(c.p[3], n4));
+    o.p[3] = pick2<ERODE>(c.p[3], straddle(n4, n5));
+    return o;
+}
+// the 3 x 3 cross on row m, between the rows u and d
+template <bool ERODE>
+__device__ __forceinline__ Row8 cross(const Row8& u, const Row8& m, const Row8& d) {
+    uint32_t s[5];  // pairs one column to the left of pair j
+    s[0] = straddle(prev_lane(m.p[3]), m.p[0]);
+#pragma unroll
+    for (int j = 1; j < 4; ++j) s[j] = straddle(m.p[j - 1], m.p[j]);
+    s[4] = straddle(m.p[3], next_lane(m.p[0]));
+    Row8 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o.p[j] = pick3<ERODE>(pick3<ERODE>(s[j], m.p[j], s[j + 1]), u.p[j], d.p[j]);
+    return o;
+}
+
+typedef uint32_t __attribute__((ext_vector_type(2), aligned(1), may_alias)) u32x2_any;
+
+template <bool ERODE>
+__global__ __launch_bounds__(256, 3) void morph_disk(const uint8_t* __restrict__ in, uint8_t* __restrict__ out, int w, int h,
+                                                  uint8_t outside, int strips, int rows, int nwaves) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64));
+    if (wave >= nwaves) return;
+    const int lane = threadIdx.x & 63;
+    const int sx = wave % strips, y0 = (wave / strips) * rows;
+    const int nr = min(rows, h - y0);
+    const int c = sx * DOUT - DSQ - 8 + 8 * lane;  // the lane's first column; its results belong 5 columns further
+    const uint32_t ob = outside * 0x01010101u;
+    // Rows come in as 8 bytes at a column clamped into the image, so every load is issued ahead of its use;
+    // lanes across an edge then move the bytes into place and take the constant for the rest.
+    const int cc = clampi(c, 0, max(w - 8, 0)), off = clampi(c - cc, -8, 8);
+    const bool edges = __any(off != 0) || w < 8;
+    uint64_t keep = 0;  // bytes of the lane that are in the image
+    for (int i = 0; i < 8; ++i) keep |= (uint64_t)(c + i >= 0 && c + i < w ? 0xFF : 0) << (8 * i);
+    // row t of the strip's input (any row may be asked for: rows outside the image are constant)
+    auto load = [&](int t) {
+        u32x2_any q = {ob, ob};
+        const int gy = y0 - DRAD + t;
+        if (gy < 0 || gy >= h) return q;
+        const uint8_t* row = in + (size_t)gy * w;
+        if (w >= 8) return *reinterpret_cast<const u32x2_any*>(row + cc);
+        uint32_t b[8];  // narrower than a lane: every byte on its own, in place
+#pragma unroll
+        for (int i = 0; i < 8; ++i) b[i] = row[clampi(c + i, 0, w - 1)];
+        q.x = b[0] | b[1] << 8 | b[2] << 16 | b[3] << 24;
+        q.y = b[4] | b[5] << 8 | b[6] << 16 | b[7] << 24;
+        return q;
+    };
+    auto place = [&](u32x2_any& q, int t) {
+        const int gy = y0 - DRAD + t;
+        if (!edges || gy < 0 || gy >= h) return;
+        uint64_t v = (uint64_t)q.y << 32 | q.x;
+        if (w >= 8) v = off < 0 ? (off == -8 ? 0 : v << (-8 * off)) : (off == 8 ? 0 : v >> (8 * off));
+        v = (v & keep) | (((uint64_t)ob << 32 | ob) & ~keep);
+        q.x = (uint32_t)v;
+        q.y = (uint32_t)(v >> 32);
+    };
+    Row8 h1{}, h2{}, a[6]{}, b1{}, b2{}, x1[4]{}, x2[4]{};  // the rows before of each stage (x1, x2: of the crosses' inputs)
+    u32x2_any cur[4], nxt[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) cur[u] = load(u);
+    for (int t0 = 0; t0 < nr + 2 * DRAD; t0 += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) nxt[u] = load(t0 + 4 + u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int t = t0 + u;
+            place(cur[u], t);
+            Row8 r;
+            r.p[0] = __builtin_amdgcn_perm(0u, cur[u].x, 0x0C010C00u);
+            r.p[1] = __builtin_amdgcn_perm(0u, cur[u].x, 0x0C030C02u);
+            r.p[2] = __builtin_amdgcn_perm(0u, cur[u].y, 0x0C010C00u);
+            r.p[3] = __builtin_amdgcn_perm(0u, cur[u].y, 0x0C030C02u);
+            const Row8 hr = across11<ERODE>(r);
+            Row8 ar, br, s;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                ar.p[j] = pick3<ERODE>(hr.p[j], h1.p[j], h2.p[j]);        // rows t - 2 .. t
+                br.p[j] = pick3<ERODE>(ar.p[j], a[2].p[j], a[5].p[j]);    // t - 8 .. t
+                s.p[j] = pick2<ERODE>(br.p[j], b2.p[j]);                  // t - 10 .. t
+            }
+            h2 = h1;
+            h1 = hr;
+#pragma unroll
+            for (int k = 5; k > 0; --k) a[k] = a[k - 1];
+            a[0] = ar;
+            b2 = b1;
+            b1 = br;
+#pragma unroll
+            for (int k = 0; k < DDI; ++k) {  // each cross is one row behind its input
+                const Row8 o = cross<ERODE>(x2[k], x1[k], s);
+                x2[k] = x1[k];
+                x1[k] = s;
+                s = o;
+            }
+            const int o = t - 2 * DRAD;  // the strip's output row that is complete
+            if (o >= 0 && o < nr && lane >= 1 && lane <= DOUT / 8) {
+                u32x2_any q;
+                q.x = __builtin_amdgcn_perm(s.p[1], s.p[0], 0x06040200u);
+                q.y = __builtin_amdgcn_perm(s.p[3], s.p[2], 0x06040200u);
+                uint8_t* dst = out + (size_t)(y0 + o) * w + c + DSQ;
+                const int n = w - (c + DSQ);
+                if (n >= 8) {
+                    *reinterpret_cast<u32x2_any*>(dst) = q;
+                } else {
+                    for (int i = 0; i < n; ++i) dst[i] = (uint8_t)((i < 4 ? q.x : q.y) >> (8 * (i & 3)));
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) cur[u] = nxt[u];
+    }
+}
+
+// the element is that disk
+bool is_disk(const uint8_t* kernel, int k) {
+    if (k != DK) return false;
+    for (int y = -DRAD; y <= DRAD; ++y)
+        for (int x = -DRAD; x <= DRAD; ++x) {
+            const bool in = std::max(std::abs(x) - DSQ, 0) + std::max(std::abs(y) - DSQ, 0) <= DDI;
+            if ((kernel[(y + DRAD) * DK + x + DRAD] != 0) != in) return false;
+        }
+    return true;
+}
+
+int launch_disk(const uint8_t* in, uint8_t* out, int w, int h, int outside, bool erode, hipStream_t s) {
+    const int strips = (int)cdiv(w, DOUT);
+    int rows = 32;
+    while (rows > 8 && (size_t)strips * cdiv(h, rows) < 2048) rows /= 2;
+    const int nwaves = strips * (int)cdiv(h, rows);
+    const dim3 grid(cdiv(nwaves, 4));
+    if (erode)
+        hipLaunchKernelGGL((morph_disk<true>), grid, dim3(256), 0, s, in, out, w, h, (uint8_t)outside, strips, rows, nwaves);
+    else
+        hipLaunchKernelGGL((morph_disk<false>), grid, dim3(256), 0, s, in, out, w, h, (uint8_t)outside, strips, rows, nwaves);
+    NSC_HIP(hipGetLastError());
+    return NSC_OK;
+}
+
 // 3 x 3 elements (the cross of HistologicalEntities.cpp:330 and :498): a thread makes four
 // consecutive outputs of one row from the 3 x 6 input bytes around them (read as one aligned word
 // per row plus its two edge bytes when `words`: both planes 4-byte aligned and the row width a
@@ -373,6 +564,7 @@ int morph_impl(const uint8_t* in, uint8_t* out, int w, int h, const uint8_t* ker
         NSC_HIP(hipGetLastError());
         return NSC_OK;
     }
+    if (is_disk(kernel, k)) return launch_disk(in, out, w, h, outside, erode, s);
     const size_t lds2 = 2 * ((size_t)WW * WW + (size_t)P.nrun * WW * MT);
     if (lds2 <= 160 * 1024) {
         const bool words = (w & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0;
