@@ -94,6 +94,13 @@ __device__ __forceinline__ int c_diff(const uint8_t* a, const uint8_t* b) {
     return max(max(db, dg), dr);
 }
 
+__device__ __forceinline__ int cdiff_packed(uint32_t a, uint32_t b) {
+    const int d0 = abs((int)(a & 255) - (int)(b & 255));
+    const int d1 = abs((int)((a >> 8) & 255) - (int)((b >> 8) & 255));
+    const int d2 = abs((int)((a >> 16) & 255) - (int)((b >> 16) & 255));
+    return max(max(d0, d1), d2);
+}
+
 // ---- item accessors ----
 constexpr int kPopMax = 1 << 24;
 __device__ __forceinline__ int rec_lvl(const int4& r) { return (int)((uint32_t)r.z >> 24); }
@@ -147,47 +154,112 @@ __device__ __forceinline__ bool before_keyed(const Dev& D, const ItemKey& kx, co
 }
 
 // ---- classification ----
+// One pixel: class and initial push level from its marker and colour and its four neighbours' (left, right,
+// up, down; pos: the neighbour is a seed off the frame).
+struct PixelClass {
+    uint8_t cls;
+    uint16_t lvl0;
+};
+__device__ __forceinline__ PixelClass classify(bool frame, int v, uint32_t col, const bool (&pos)[4], const uint32_t (&ncol)[4]) {
+    int best = 256;  // smallest colour step to a neighbouring seed
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int d = cdiff_packed(col, ncol[k]);
+        best = pos[k] ? min(best, d) : best;
+    }
+    return {(uint8_t)(frame ? C_FRAME : (v > 0 ? C_SEED : (col == 0 ? C_B : C_F))),
+            (uint16_t)(frame || v > 0 || best >= 256 ? NOPUSH : best)};
+}
+
 // nF: this workgroup's count goes to partial[blockIdx.x] (summed by k_sum_partials): one atomic
 // per workgroup on a single counter would serialise over a grid this large.
+// Four pixels in a row (of the plane's linear order) to a thread: their markers and colours and those of
+// the rows above and below come in 11 wide loads instead of 80 single ones, and go out in six stores.  The
+// first and last row's groups, whose neighbour rows would leave the plane, take pixel by pixel loads.
+// Bound by its 23 bytes per pixel; measured, 4098 x 4098: 164 -> 93 us.
+typedef int32_t __attribute__((ext_vector_type(4), aligned(4), may_alias)) i32x4_any;
+typedef uint32_t __attribute__((ext_vector_type(3), aligned(1), may_alias)) u32x3_any;
+typedef uint32_t __attribute__((aligned(1), may_alias)) u32_any;
+// the four colours of 12 bytes
+__device__ __forceinline__ void colours4(u32x3_any q, uint32_t (&c)[4]) {
+    c[0] = q.x & 0xFFFFFFu;
+    c[1] = __builtin_amdgcn_alignbit(q.y, q.x, 24) & 0xFFFFFFu;
+    c[2] = __builtin_amdgcn_alignbit(q.z, q.y, 16) & 0xFFFFFFu;
+    c[3] = q.z >> 8;
+}
+__device__ __forceinline__ uint32_t colour1(const uint8_t* p) { return p[0] | (uint32_t)p[1] << 8 | (uint32_t)p[2] << 16; }
+
 __global__ void k_classify(Dev D, uint8_t* cls, uint16_t* lvl0, uint8_t* fmask, int* partial) {
-    const int W = D.W, H = D.H;
+    const int W = D.W, H = D.H, N = D.N;
     int local = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < D.N; i += gridDim.x * blockDim.x) {
-        const int x = i % W, y = i / W;
-        const bool frame = (x == 0 || y == 0 || x == W - 1 || y == H - 1);
-        // the pixel's and its four neighbours' markers and colours, all loads issued together
-        // (a frame pixel, whose neighbours may leave the image, reads itself five times and
-        // ignores the copies); the decisions below are selects on loaded values
-        const int nb[4] = {frame ? i : i - 1, frame ? i : i + 1, frame ? i : i - W, frame ? i : i + W};
-        const int v = D.m0[i];
-        int vn[4];
-        uint8_t pc[3], nc[4][3];
+    const int groups = (N + 3) / 4;
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < groups; t += gridDim.x * blockDim.x) {
+        const int i0 = 4 * t;
+        if (i0 >= W && i0 + 3 + W < N) {
+            const i32x4_any mo = *reinterpret_cast<const i32x4_any*>(D.m0 + i0), mu = *reinterpret_cast<const i32x4_any*>(D.m0 + i0 - W),
+                            md = *reinterpret_cast<const i32x4_any*>(D.m0 + i0 + W);
+            const int ml = D.m0[i0 - 1], mr = D.m0[i0 + 4];
+            const uint8_t* px = D.img + 3 * (size_t)i0;
+            const u32x3_any qo = *reinterpret_cast<const u32x3_any*>(px), qu = *reinterpret_cast<const u32x3_any*>(px - 3 * (size_t)W),
+                            qd = *reinterpret_cast<const u32x3_any*>(px + 3 * (size_t)W);
+            const uint32_t ql = *reinterpret_cast<const u32_any*>(px - 4), qr = *reinterpret_cast<const u32_any*>(px + 12);
+            int y = i0 / W, x = i0 - y * W;
+            uint32_t co[4], cu[4], cd[4];
+            colours4(qo, co);
+            colours4(qu, cu);
+            colours4(qd, cd);
+            const int m[6] = {ml, mo.x, mo.y, mo.z, mo.w, mr}, up[4] = {mu.x, mu.y, mu.z, mu.w}, dn[4] = {md.x, md.y, md.z, md.w};
+            const uint32_t c[6] = {ql >> 8, co[0], co[1], co[2], co[3], qr & 0xFFFFFFu};
+            uint32_t ocls = 0, omask = 0, ol[2] = {0, 0};
+            i32x4_any om;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) vn[k] = D.m0[nb[k]];
-#pragma unroll
-        for (int ch = 0; ch < 3; ++ch) {
-            pc[ch] = D.img[3 * (size_t)i + ch];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) nc[k][ch] = D.img[3 * (size_t)nb[k] + ch];
+            for (int j = 0; j < 4; ++j) {
+                const bool frame = x == 0 || y == 0 || x == W - 1 || y == H - 1;
+                const bool pos[4] = {x > 1 && m[j] > 0, x < W - 2 && m[j + 2] > 0, y > 1 && up[j] > 0, y < H - 2 && dn[j] > 0};
+                const uint32_t nc[4] = {c[j], c[j + 2], cu[j], cd[j]};
+                const int v = m[j + 1];
+                const PixelClass q = classify(frame, v, c[j + 1], pos, nc);
+                ocls |= (uint32_t)q.cls << (8 * j);
+                ol[j >> 1] |= (uint32_t)q.lvl0 << (16 * (j & 1));
+                omask |= (q.cls == C_F ? 1u : 0u) << (8 * j);
+                om[j] = frame ? WSHED : (v < 0 ? 0 : v);
+                if (++x == W) {
+                    x = 0;
+                    ++y;
+                }
+            }
+            local += __popc(omask);
+            *reinterpret_cast<u32_any*>(cls + i0) = ocls;
+            *reinterpret_cast<u32_any*>(fmask + i0) = omask;
+            *reinterpret_cast<u32_any*>(lvl0 + i0) = ol[0];
+            *reinterpret_cast<u32_any*>(lvl0 + i0 + 2) = ol[1];
+            *reinterpret_cast<i32x4_any*>(D.lab + i0) = i32x4_any{0, 0, 0, 0};
+            *reinterpret_cast<i32x4_any*>(D.head + i0) = i32x4_any{-1, -1, -1, -1};
+            *reinterpret_cast<i32x4_any*>(D.m + i0) = om;
+            continue;
         }
-        int best = 256;  // smallest colour step to a neighbouring seed off the frame
-        const int nx[4] = {x - 1, x + 1, x, x}, ny[4] = {y, y, y - 1, y + 1};
+        for (int i = i0; i < min(i0 + 4, N); ++i) {
+            const int x = i % W, y = i / W;
+            const bool frame = x == 0 || y == 0 || x == W - 1 || y == H - 1;
+            // (a frame pixel, whose neighbours may leave the plane, reads itself)
+            const int nb[4] = {frame ? i : i - 1, frame ? i : i + 1, frame ? i : i - W, frame ? i : i + W};
+            bool pos[4] = {x > 1, x < W - 2, y > 1, y < H - 2};
+            uint32_t nc[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const bool pos = !(nx[k] == 0 || ny[k] == 0 || nx[k] == W - 1 || ny[k] == H - 1) && vn[k] > 0;
-            const int d = c_diff(pc, nc[k]);
-            best = pos ? min(best, d) : best;
+            for (int k = 0; k < 4; ++k) {
+                pos[k] = pos[k] && D.m0[nb[k]] > 0;
+                nc[k] = colour1(D.img + 3 * (size_t)nb[k]);
+            }
+            const int v = D.m0[i];
+            const PixelClass q = classify(frame, v, colour1(D.img + 3 * (size_t)i), pos, nc);
+            cls[i] = q.cls;
+            lvl0[i] = q.lvl0;
+            fmask[i] = q.cls == C_F ? 1 : 0;
+            D.lab[i] = 0;
+            D.head[i] = -1;
+            D.m[i] = frame ? WSHED : (v < 0 ? 0 : v);
+            local += q.cls == C_F;
         }
-        const bool black = pc[0] == 0 && pc[1] == 0 && pc[2] == 0;
-        const uint8_t c = frame ? C_FRAME : (v > 0 ? C_SEED : (black ? C_B : C_F));
-        const uint16_t L = (frame || v > 0 || best >= 256) ? NOPUSH : (uint16_t)best;
-        cls[i] = c;
-        lvl0[i] = L;
-        fmask[i] = (c == C_F) ? 1 : 0;
-        D.lab[i] = 0;
-        D.head[i] = -1;
-        D.m[i] = frame ? WSHED : (v < 0 ? 0 : v);
-        local += (c == C_F);
     }
     const int bs = block_sum(local);
     if (threadIdx.x == 0) partial[blockIdx.x] = bs;
@@ -328,13 +400,6 @@ constexpr int P1_MARGIN = 2;
 // parts of a 16-byte entry, accessed beside the whole entry
 typedef uint32_t __attribute__((may_alias)) any_u32;
 typedef uint16_t __attribute__((may_alias)) any_u16;
-
-__device__ __forceinline__ int cdiff_packed(uint32_t a, uint32_t b) {
-    const int d0 = abs((int)(a & 255) - (int)(b & 255));
-    const int d1 = abs((int)((a >> 8) & 255) - (int)((b >> 8) & 255));
-    const int d2 = abs((int)((a >> 16) & 255) - (int)((b >> 16) & 255));
-    return max(max(d0, d1), d2);
-}
 
 // the lane's quad (lanes 4 q .. 4 q + 3) combined by max / min: every lane of it gets the result
 __device__ __forceinline__ int quad_swap1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true); }
@@ -916,41 +981,80 @@ __global__ __launch_bounds__(1024) void k_b1_reduce(Dev D, const int32_t* __rest
 }
 
 // queue state at T1 (after b1's pop); P pixels (B, never queued) -> pmask
+// Four pixels to a thread, their planes in wide loads, and the two dependent record reads of each pixel's
+// place in the pop order (its record, its chain's largest-key item's) side by side; b1's are read once.  An F
+// pixel popped before b1 has its label, a B pixel is a dam; one whose pusher popped before b1 is queued
+// (an item pops after its pusher, so the second question follows a no to the first).
+// Bound by 31 bytes per pixel and those reads; measured, 4098 x 4098: 172 -> 132 us.
 __global__ void k_t1_state(Dev D, const int32_t* __restrict__ real, const int* __restrict__ info, uint8_t* __restrict__ pmask,
                            uint8_t* __restrict__ kind) {
     const int b1 = info[0], b1i = info[1], Y1 = info[2];
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < D.N; p += gridDim.x * blockDim.x) {
-        uint8_t pm = 0, kd = 0;
-        // the pixel's class, label and queue entry are loaded together (each one behind the class
-        // test would be another dependent round trip); its record, where it has one, by the walk
-        const uint8_t c = D.cls[p];
-        const int labp = D.lab[p], r = real[p];
-        if (c == C_F) {
-            int v = 0;
-            if (labp != 0) {  // queued, and popped, in its run's flood
-                if (b1 < 0 || before(D, p, b1i)) v = labp;
-                else {
-                    const int par = it_parent(D, p);
-                    if (par < 0 || before(D, par, b1i)) { v = IN_QUEUE; kd = 1; }
-                }
+    ItemKey kb{};
+    if (b1 >= 0) kb = item_key(D, b1i);
+    const int groups = (D.N + 3) / 4;
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < groups; t += gridDim.x * blockDim.x) {
+        const int p0 = 4 * t, n = min(4, D.N - p0);
+        uint8_t c[4];
+        int lab[4], r[4], it[4];
+        if (n == 4) {
+            const uint32_t c4 = *reinterpret_cast<const u32_any*>(D.cls + p0);
+            const i32x4_any l4 = *reinterpret_cast<const i32x4_any*>(D.lab + p0), r4 = *reinterpret_cast<const i32x4_any*>(real + p0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                c[j] = (uint8_t)(c4 >> (8 * j));
+                lab[j] = l4[j];
+                r[j] = r4[j];
             }
-            D.m[p] = v;
-        } else if (c == C_B) {
-            int v = 0;
-            if (p == b1) v = Y1;
-            else if (r >= 0) {
-                const int par = D.wr[r].w;  // the queue entry's pusher, from its packed record
-                const bool queued = par < 0 || b1 < 0 || before(D, par, b1i);
-                if (queued) {
-                    if (b1 < 0 || before(D, r, b1i)) v = WSHED;
-                    else { v = IN_QUEUE; kd = 1; }
-                }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int p = p0 + min(j, n - 1);
+                c[j] = j < n ? D.cls[p] : (uint8_t)C_FRAME;
+                lab[j] = D.lab[p];
+                r[j] = real[p];
             }
-            if (v == 0) pm = 1;
-            D.m[p] = v;
         }
-        pmask[p] = pm;
-        kind[p] = kd;
+        int4 rec[4], top[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // the pixel's queue entry, -1 for none
+            const int p = p0 + j;
+            it[j] = c[j] == C_F ? (lab[j] != 0 ? p : -1) : (c[j] == C_B && p != b1 ? r[j] : -1);
+            if (it[j] >= 0) rec[j] = D.wr[it[j]];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (it[j] >= 0) top[j] = D.wr[rec[j].y];
+        uint32_t pm = 0, kd = 0;
+        int v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v[j] = c[j] == C_B && p0 + j == b1 ? Y1 : 0;
+            if (it[j] >= 0) {
+                const ItemKey k{it[j], rec[j].x, rec_pop(rec[j]), rec[j].y, rec_lvl(top[j]), top[j].w};
+                if (b1 < 0 || before_keyed(D, k, kb)) v[j] = c[j] == C_F ? lab[j] : WSHED;
+                else if (rec[j].w < 0 || before(D, rec[j].w, b1i)) {
+                    v[j] = IN_QUEUE;
+                    kd |= 1u << (8 * j);
+                }
+            }
+            if (c[j] == C_B && v[j] == 0) pm |= 1u << (8 * j);
+        }
+        const bool all = (c[0] & 2) && (c[1] & 2) && (c[2] & 2) && (c[3] & 2);  // F or B: the others keep their value
+        if (all) *reinterpret_cast<i32x4_any*>(D.m + p0) = i32x4_any{v[0], v[1], v[2], v[3]};
+        else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (c[j] & 2) D.m[p0 + j] = v[j];
+        }
+        if (n == 4) {
+            *reinterpret_cast<u32_any*>(pmask + p0) = pm;
+            *reinterpret_cast<u32_any*>(kind + p0) = kd;
+        } else {
+            for (int j = 0; j < n; ++j) {
+                pmask[p0 + j] = (uint8_t)(pm >> (8 * j));
+                kind[p0 + j] = (uint8_t)(kd >> (8 * j));
+            }
+        }
     }
 }
 
@@ -1747,7 +1851,7 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
         hipLaunchKernelGGL(k_b1_reduce, dim3(1), dim3(1024), 0, s, D, real, partial, &small[8]);
     }
     tick("b1", &small[8]);
-    hipLaunchKernelGGL(k_t1_state, grid1(N), dim3(256), 0, s, D, real, &small[8], fmask, kind);
+    hipLaunchKernelGGL(k_t1_state, grid1((N + 3) / 4), dim3(256), 0, s, D, real, &small[8], fmask, kind);
     // flood from b1 over the never-queued B pixels (fmask marks them): geodesic distance from b1
     {
         unsigned* dist = reinterpret_cast<unsigned*>(head);  // head[] is dead after k_bresolve
