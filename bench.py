@@ -27,13 +27,12 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# The served step runs 8 server slots, each with its own stream and three side streams; HIP maps a
-# process's streams onto GPU_MAX_HW_QUEUES hardware queues (4 by default), where kernels of
-# unrelated streams wait behind each other: with 4 queues a kernel trace of the served step never
-# shows more than 4 kernels running at once.  16 queues measured 5% more served throughput than 8
-# and 8 about 7% more than 4 (the plain path is unchanged).  --hw-queues sets it (0 keeps the
-# environment's value); it must be set before the HIP runtime starts (before torch touches the GPU),
-# so it is read from the command line here, ahead of the argument parser.
+# The served step runs 8 server slots, each with its own stream; HIP maps a process's streams onto
+# GPU_MAX_HW_QUEUES hardware queues (4 by default), where kernels of unrelated streams wait behind each
+# other: with 4 queues a kernel trace of the served step never shows more than 4 kernels running at
+# once.  --hw-queues sets it (0 keeps the environment's value); it must be set before the HIP runtime
+# starts (before torch touches the GPU), so it is read from the command line here, ahead of the
+# argument parser.
 def _hw_queues_arg(argv):
     for i, a in enumerate(argv):
         if a == "--hw-queues" and i + 1 < len(argv):

@@ -37,8 +37,8 @@ __global__ void k_lmax_cand(const float* __restrict__ c, const float* __restrict
         const size_t ru = (size_t)(y > 0 ? y - 1 : y) * w, r0 = (size_t)y * w, rd = (size_t)(y + 1 < h ? y + 1 : y) * w;
         const float rc = MIN ? -rec[i] : rec[i], v = gc[i];
         const float n0 = gc[r0 + xl], n1 = gc[r0 + xr], n2 = gc[ru + x], n3 = gc[rd + x];
-        auto above = [&](float q) { return MIN ? q < v : v < q; };
-        bool g = above(n0) | above(n1) | above(n2) | above(n3);
+        auto above = [&](float q) -> int { return MIN ? q < v : v < q; };
+        int g = above(n0) | above(n1) | above(n2) | above(n3);
         if (CONN == 8) {
             const float n4 = gc[ru + xl], n5 = gc[ru + xr], n6 = gc[rd + xl], n7 = gc[rd + xr];
             g = g | above(n4) | above(n5) | above(n6) | above(n7);

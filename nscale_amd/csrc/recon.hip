@@ -156,12 +156,6 @@ __device__ __forceinline__ R nbr3(R pc) {
     return smax(pc, smax(l, r));
 }
 template <>
-__device__ __forceinline__ uint32_t nbr3(uint32_t pc) {
-    const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)pc, 0x138, 0xF, 0xF, true);
-    const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)pc, 0x130, 0xF, 0xF, true);
-    return max(max(l, pc), r);
-}
-template <>
 __device__ __forceinline__ int32_t nbr3(int32_t pc) {
     const int32_t l = __builtin_amdgcn_update_dpp(0, pc, 0x138, 0xF, 0xF, true);
     const int32_t r = __builtin_amdgcn_update_dpp(0, pc, 0x130, 0xF, 0xF, true);
@@ -249,19 +243,16 @@ __device__ __forceinline__ void sweep_round(typename RegOf<T>::type (&v)[TH], Wi
 // Change detection: values only rise, so a column changed in a round iff the sum of an
 // order-preserving unsigned key of its values rose.  The sweeps carry no per-step compares (the
 // compiler would keep all 248 compare results in scalar registers and OR them as a tree).
-__device__ __forceinline__ uint32_t order_key(uint32_t v) { return v; }
 __device__ __forceinline__ uint32_t order_key(int32_t v) { return (uint32_t)v ^ 0x80000000u; }
 __device__ __forceinline__ uint32_t order_key(float v) {
     const uint32_t b = __builtin_bit_cast(uint32_t, v);
     return b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
 }
 template <typename R>
-__device__ __forceinline__ auto col_sum(const R (&v)[TH]) {
-    // uint8 values: 64 x 255 fits 32 bits; four-byte keys need 64
-    using S = typename std::conditional<std::is_same<R, uint32_t>::value, uint32_t, uint64_t>::type;
-    S s = 0;
+__device__ __forceinline__ uint64_t col_sum(const R (&v)[TH]) {
+    uint64_t s = 0;
 #pragma unroll
-    for (int y = 0; y < TH; ++y) s += (S)order_key(v[y]);
+    for (int y = 0; y < TH; ++y) s += order_key(v[y]);
     return s;
 }
 

@@ -1764,7 +1764,7 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
     carve(cut, cls, lvl0, fmask, run, lab, head, real, lab2, kind, small);
     // small[]: 0 nF, 1 nrun, 2 nleaf, 3 flags, 4 ncand, 8..10 info, 16 ncomp, 20 deferred tie components,
     // 24..25 tie pool bump pointer (long long), 26..31 run bucket sizes, 32..34 LDS flood queue counts,
-    // 35 B pixels with queue entries, 40..44 phase-1 tier work counters
+    // 35 B pixels with queue entries, 40 run flood work counter
     NSC_HIP(hipMemsetAsync(small, 0, 64 * sizeof(int), s));
 
     Dev D{};
