@@ -121,45 +121,53 @@ __device__ __forceinline__ float flip_sign(float v, uint32_t flip) {
     return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) ^ flip);
 }
 
+// ---- four-byte windows: integer keys -----------------------------------------------------------
+// int32 values as they are, floats as their order-preserving keys (the same bits for positive values, the
+// lower 31 flipped for negative ones; an involution), so a step is integer maxima and a minimum instead of
+// comparisons and selects.  NaN as the float comparisons had it: a NaN marker's pixel stays NaN and feeds
+// nobody (kNan under kNan: the lowest key, whose float is a NaN), a NaN mask bounds nothing (the highest key).
+// Measured: the passes of the h-minima of 16 maps of 512..2048 460 -> 375 us, of the two reconstructions of a
+// 512 x 512 chain 237 -> 185, of a 4096 x 4096 one 630 -> 509.  (Variants that were slower: all 128 loads of a
+// window issued first; rows of 272 bytes read 16 at a time; changes by xor in every step.)
+constexpr int32_t kNan = INT32_MIN;
+__device__ __forceinline__ int32_t to_key(int32_t v) { return v; }
+__device__ __forceinline__ int32_t to_key(float v) {
+    const int32_t b = __builtin_bit_cast(int32_t, v);
+    return b ^ (b >> 31 & INT32_MAX);
+}
+template <typename T>
+__device__ __forceinline__ T from_key(int32_t k);
+template <>
+__device__ __forceinline__ int32_t from_key<int32_t>(int32_t k) { return k; }
+template <>
+__device__ __forceinline__ float from_key<float>(int32_t k) {
+    return __builtin_bit_cast(float, k ^ (k >> 31 & INT32_MAX));
+}
+
 template <typename T>
 struct RShared {
-    using R = typename RegOf<T>::type;
+    using R = int32_t;
     // the window's mask (frozen pixels: mask = value) is staged here only to be read back
     // transposed into registers; the sweeps' transposes then reuse the same LDS (one wave per
     // workgroup, so the staging reads precede the first transpose write in program order)
     union {
-        T lm[TH][TW + 4];
-        T tr[TH][TW + 1];
+        R lm[TH][TW + 4];
+        R tr[TH][TW + 1];
     };
     R init_l[TH], init_r[TH];
     unsigned chg_bits;
 };
 
 // ---- per-step arithmetic of the window sweeps ------------------------------------------------
-// Values only rise (out starts at min(marker, mask) <= mask), so min(max(v, n), mk) = med3(v, n, mk)
-// for integer types.  Frozen pixels have mk = v, hence med3(v, n, v) = v whatever n holds; that is
-// why the neighbour maxima may read zero-filled DPP lanes (lanes 0 and 63 are always frozen).
-template <typename R>
-__device__ __forceinline__ R clamp_up(R v, R n, R mk) { return smin(smax(v, n), mk); }
-template <>
-__device__ __forceinline__ int32_t clamp_up(int32_t v, int32_t n, int32_t mk) {
-    int32_t r;
-    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(n), "v"(mk));
-    return r;
-}
+// Values only rise (out starts at min(marker, mask) <= mask).  Frozen pixels have mk = v, hence
+// min(max(v, n), v) = v whatever n holds; that is why the neighbour maxima may read zero-filled DPP lanes (lanes 0 and 63 are always frozen).
+__device__ __forceinline__ int32_t clamp_up(int32_t v, int32_t n, int32_t mk) { return min(max(v, n), mk); }
 // max of a value and its left and right lane neighbours (8-connectivity); lanes whose DPP source
 // is outside the wave read 0 (only frozen lanes, see above)
-template <typename R>
-__device__ __forceinline__ R nbr3(R pc) {
-    const R l = __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, pc), 0x138, 0xF, 0xF, true));
-    const R r = __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, pc), 0x130, 0xF, 0xF, true));
-    return smax(pc, smax(l, r));
-}
-template <>
 __device__ __forceinline__ int32_t nbr3(int32_t pc) {
     const int32_t l = __builtin_amdgcn_update_dpp(0, pc, 0x138, 0xF, 0xF, true);
     const int32_t r = __builtin_amdgcn_update_dpp(0, pc, 0x130, 0xF, 0xF, true);
-    return max(max(l, pc), r);
+    return max(max(l, r), pc);
 }
 
 // Mask of a window in both orientations, in registers, so the sweeps never touch LDS for it:
@@ -169,13 +177,13 @@ __device__ __forceinline__ int32_t nbr3(int32_t pc) {
 // transposes).
 template <typename T>
 struct WinMask {
-    using R = typename RegOf<T>::type;
-    const T (*lm)[TW + 4];
+    using R = int32_t;
+    const R (*lm)[TW + 4];
     int lane;
     R mc[TH], mr[TW];
     __device__ __forceinline__ void build() {
 #pragma unroll
-        for (int x = 0; x < TW; ++x) mr[x] = (R)lm[lane][x];
+        for (int x = 0; x < TW; ++x) mr[x] = lm[lane][x];
     }
     __device__ void opaque() {}
     __device__ __forceinline__ R clamp_col(R v, R n, int y) const { return clamp_up(v, n, mc[y]); }
@@ -190,9 +198,9 @@ struct WinMask {
 // chain reads what the other has already raised.  Rows likewise with the left and right sweeps.
 // (whether anything changed is decided by the caller from column sums)
 template <typename T, int CONN>
-__device__ __forceinline__ void sweep_round(typename RegOf<T>::type (&v)[TH], WinMask<T>& M, T (*tr)[TW + 1],
+__device__ __forceinline__ void sweep_round(int32_t (&v)[TH], WinMask<T>& M, int32_t (*tr)[TW + 1],
                                             int lane) {
-    using R = typename RegOf<T>::type;
+    using R = int32_t;
     M.opaque();
     {
         R pd = v[0], pu = v[TH - 1];
@@ -210,10 +218,10 @@ __device__ __forceinline__ void sweep_round(typename RegOf<T>::type (&v)[TH], Wi
     }
     // ---- transpose to row state (lane = row) ----
 #pragma unroll
-    for (int y = 0; y < TH; ++y) tr[y][lane] = (T)v[y];
+    for (int y = 0; y < TH; ++y) tr[y][lane] = v[y];
     __syncthreads();
 #pragma unroll
-    for (int x = 0; x < TW; ++x) v[x] = (R)tr[lane][x];
+    for (int x = 0; x < TW; ++x) v[x] = tr[lane][x];
     M.opaque();
     {
         // with 8-connectivity the row sweeps take the diagonal neighbours too (the rows above and
@@ -233,10 +241,10 @@ __device__ __forceinline__ void sweep_round(typename RegOf<T>::type (&v)[TH], Wi
         }
     }
 #pragma unroll
-    for (int x = 0; x < TW; ++x) tr[lane][x] = (T)v[x];
+    for (int x = 0; x < TW; ++x) tr[lane][x] = v[x];
     __syncthreads();
 #pragma unroll
-    for (int y = 0; y < TH; ++y) v[y] = (R)tr[y][lane];
+    for (int y = 0; y < TH; ++y) v[y] = tr[y][lane];
     __syncthreads();
 }
 
@@ -244,10 +252,6 @@ __device__ __forceinline__ void sweep_round(typename RegOf<T>::type (&v)[TH], Wi
 // order-preserving unsigned key of its values rose.  The sweeps carry no per-step compares (the
 // compiler would keep all 248 compare results in scalar registers and OR them as a tree).
 __device__ __forceinline__ uint32_t order_key(int32_t v) { return (uint32_t)v ^ 0x80000000u; }
-__device__ __forceinline__ uint32_t order_key(float v) {
-    const uint32_t b = __builtin_bit_cast(uint32_t, v);
-    return b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
-}
 template <typename R>
 __device__ __forceinline__ uint64_t col_sum(const R (&v)[TH]) {
     uint64_t s = 0;
@@ -515,7 +519,7 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
     if constexpr (std::is_same<T, uint8_t>::value) {
         recon_tile_u8<CONN>(im, tile, pass, sh, next_list, next_count, stamp, dirty);
     } else {
-    using R = typename RegOf<T>::type;
+    using R = int32_t;
     auto& lm = sh.lm;
     auto& init_l = sh.init_l;
     auto& init_r = sh.init_r;
@@ -544,12 +548,12 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
     // scheduling fences stop the compiler from sinking loads to their uses)
 #pragma unroll
     for (int c = 0; c < TH; c += 16) {
-        R m_ld[16], s_ld[16];
+        T m_ld[16], s_ld[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const size_t i = (size_t)clampi(ty * OH - 1 + c + j, 0, h - 1) * w + gxc;
-            m_ld[j] = (R)gmask[i];  // unconditional: the address is valid
-            s_ld[j] = (R)gsrc[i];
+            m_ld[j] = gmask[i];  // unconditional: the address is valid
+            s_ld[j] = gsrc[i];
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -562,12 +566,17 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
                 m_ld[j] = z ? FLT_MAX : flip_sign(m_ld[j], im.in_flip);
                 s_ld[j] = pass == 0 ? m_ld[j] - im.depth : flip_sign(s_ld[j], im.out_flip);
             }
-            const R mk = keep_bits(m_ld[j], keep);
-            const R val = keep_bits(smin(s_ld[j], m_ld[j]), keep);
+            R mk = to_key(m_ld[j]), val = to_key(s_ld[j]);
+            if constexpr (std::is_same<T, float>::value) {
+                if (m_ld[j] != m_ld[j]) mk = INT32_MAX;
+                if (s_ld[j] != s_ld[j]) val = mk = kNan;
+            }
+            val = (R)((uint32_t)min(val, mk) & keep);
+            mk = (R)((uint32_t)mk & keep);
             const bool frozen = col_frozen || y == 0 || y == TH - 1 || !inb;
             v[y] = val;
             const R mw = frozen ? val : mk;
-            lm[y][lane] = (T)mw;
+            lm[y][lane] = mw;
             M.mc[y] = mw;
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -609,8 +618,8 @@ __device__ __forceinline__ void recon_tile(const RImg<T>& im, int tile, int pass
         for (int y = 1; y < TH - 1; ++y) {
             const int gy = ty * OH - 1 + y;
             if (gy < h) {
-                if constexpr (HD) gcol[(size_t)gy * w] = flip_sign(v[y], im.out_flip);
-                else gcol[(size_t)gy * w] = (T)v[y];
+                if constexpr (HD) gcol[(size_t)gy * w] = flip_sign(from_key<float>(v[y]), im.out_flip);
+                else gcol[(size_t)gy * w] = from_key<T>(v[y]);
             }
         }
     }
