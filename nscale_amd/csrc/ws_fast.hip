@@ -32,6 +32,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "common.hpp"
+#include "ws_rules.hpp"
 
 namespace nsc {
 
@@ -177,6 +178,7 @@ __device__ __forceinline__ PixelClass classify(bool frame, int v, uint32_t col, 
 // the rows above and below come in 11 wide loads instead of 80 single ones, and go out in six stores.  The
 // first and last row's groups, whose neighbour rows would leave the plane, take pixel by pixel loads.
 // Bound by its 23 bytes per pixel; measured, 4098 x 4098: 164 -> 93 us.
+// (which groups' loads stay inside both planes: classify_wide, ws_rules.hpp)
 typedef int32_t __attribute__((ext_vector_type(4), aligned(4), may_alias)) i32x4_any;
 typedef uint32_t __attribute__((ext_vector_type(3), aligned(1), may_alias)) u32x3_any;
 typedef uint32_t __attribute__((aligned(1), may_alias)) u32_any;
@@ -195,7 +197,7 @@ __global__ void k_classify(Dev D, uint8_t* cls, uint16_t* lvl0, uint8_t* fmask, 
     const int groups = (N + 3) / 4;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < groups; t += gridDim.x * blockDim.x) {
         const int i0 = 4 * t;
-        if (i0 >= W && i0 + 3 + W < N) {
+        if (classify_wide(i0, W, N)) {
             const i32x4_any mo = *reinterpret_cast<const i32x4_any*>(D.m0 + i0), mu = *reinterpret_cast<const i32x4_any*>(D.m0 + i0 - W),
                             md = *reinterpret_cast<const i32x4_any*>(D.m0 + i0 + W);
             const int ml = D.m0[i0 - 1], mr = D.m0[i0 + 4];
