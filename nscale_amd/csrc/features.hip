@@ -17,6 +17,7 @@
 #include <cmath>
 
 #include "common.hpp"
+#include "features_rules.hpp"
 
 namespace nsc {
 namespace {
@@ -145,7 +146,8 @@ __global__ __launch_bounds__(256) void k_object_features(const int32_t* __restri
         // cell (cx, cy) has pixel (minx + cx, miny + cy) as its last corner, so the walk over the cells
         // meets every pixel of the box once.  A thread's cells lie 256 apart; the position advances by
         // that step instead of being divided out.
-        const int cw = bw + 1, ch = bh + 1, dy = 256 / cw, dx = 256 - dy * cw;
+        const CellWalk cells = cell_walk(bw, bh);  // no cells in an empty box: nothing is read for it
+        const int cw = cells.cw, ch = cells.ch, dy = 256 / cw, dx = 256 - dy * cw;
         for (int cy = t / cw, cx = t - cy * cw; cy < ch; cy += dy, cx += dx, cy += cx >= cw ? 1 : 0, cx -= cx >= cw ? cw : 0) {
             const int x = minx + cx, y = miny + cy;
             // the four labels from clamped (always valid) addresses, all issued together
