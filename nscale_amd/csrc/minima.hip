@@ -106,6 +106,10 @@ extern "C" {
 
 int nsc_imhmin_f32_batched(const nsc_recon_desc* descs, int n, float hval, void* stream) {
     NSC_ARG(descs && n > 0, "imhmin_f32_batched");
+    // before the sizes and pointers are used
+    for (int i = 0; i < n; ++i)
+        NSC_ARG(descs[i].mask && descs[i].out && descs[i].w > 0 && descs[i].h > 0 && valid_conn(descs[i].conn),
+                "imhmin_f32_batched: descriptor");
     NSC_CHECK(ensure_init());
     hipStream_t s = as_stream(stream);
     // Every image is read until the last pass: where an output overlaps an input (in place, or another
