@@ -1374,10 +1374,12 @@ static int recon_batched_run(const nsc_recon_desc* d, int n, float depth, hipStr
     int rc;
     if constexpr (HD) {
         Scratch sc;
-        NSC_CHECK(sc.alloc(recon_scratch_bytes((int)nt), s));
-        const ReconBufs B = recon_carve(sc.p, (int)nt);
-        recon_clear(B, s);
-        rc = recon_passes<float, true>(imgs_dev, imgs[0], tile_dev, (int)nt, pixels, conn_all, 1, B, s);
+        rc = sc.alloc(recon_scratch_bytes((int)nt), s);
+        if (rc == NSC_OK) {
+            const ReconBufs B = recon_carve(sc.p, (int)nt);
+            recon_clear(B, s);
+            rc = recon_passes<float, true>(imgs_dev, imgs[0], tile_dev, (int)nt, pixels, conn_all, 1, B, s);
+        }
     } else {
         rc = recon_run_scratch<T>(imgs_dev, imgs[0], tile_dev, (int)nt, pixels, conn_all, G, s);
     }
