@@ -11,16 +11,20 @@
 // waiting for it, counts as an unsafe call and would end that capture.  The events here are recorded on streams
 // that are not captured and the answer only chooses a block, so the cache asks in relaxed mode.
 // Bounds: kCacheBlock bytes a block, kCacheTotal over all threads.  Blocks come from the pool and
-// return to it when they are outgrown, when none of kCacheWindow calls needed a quarter of one, and when
-// the thread ends.
+// return to it when they are outgrown, when none of kCacheWindow calls on one needed a quarter of it, when
+// its thread's calls have passed it over kCacheAge times, when the thread ends, and, whichever thread
+// holds them, when an allocation fails (a call that holds its block keeps it).  The lock of a thread's cache is for
+// that last case; otherwise only its own thread takes it.
 #include <algorithm>
 #include <atomic>
+#include <mutex>
+#include <vector>
 
 #include "scratch.hpp"
 
 namespace nsc {
 namespace {
-constexpr int kCacheSlots = 4, kCacheWindow = 64;
+constexpr int kCacheSlots = 4, kCacheWindow = 64, kCacheAge = 2 * kCacheWindow;
 constexpr size_t kCacheBlock = (size_t)1 << 30, kCacheTotal = (size_t)4 << 30, kCacheStep = (size_t)2 << 20;
 std::atomic<size_t> g_cache_bytes{0};
 
@@ -33,6 +37,7 @@ struct CacheSlot {
     size_t want = 0;       // bytes the last call that did not fit would have needed
     size_t recent = 0;     // most bytes a call needed in the current window
     int calls = 0;         // calls in the current window
+    int passed = 0;        // calls of the thread since this block's last one
 };
 
 // relaxed capture mode of the calling thread while it lives
@@ -56,12 +61,34 @@ void free_block(void* p) {
     if (own) (void)hipStreamDestroy(own);
 }
 
+struct CallCache;
+// every thread's cache (never destroyed: threads may end after the statics have)
+struct Registry {
+    std::mutex m;
+    std::vector<CallCache*> caches;
+};
+Registry& registry() {
+    static Registry* const r = new Registry;
+    return *r;
+}
+
 struct CallCache {
+    std::mutex m;
     CacheSlot slots[kCacheSlots];
     CacheSlot* cur = nullptr;  // the current call's block
     int live = 0;              // its buffers not yet released
     size_t peak = 0, missed = 0;
+    CallCache() {
+        Registry& r = registry();
+        const std::lock_guard<std::mutex> lock(r.m);
+        r.caches.push_back(this);
+    }
     ~CallCache() {
+        {
+            Registry& r = registry();
+            const std::lock_guard<std::mutex> lock(r.m);
+            r.caches.erase(std::find(r.caches.begin(), r.caches.end(), this));
+        }
         const RelaxedCapture relaxed;
         for (CacheSlot& c : slots) {
             if (c.pending) (void)hipEventSynchronize(c.done);
@@ -140,27 +167,59 @@ void resize_block(CacheSlot& c, size_t cap, hipStream_t s) {
     c.arena.base = static_cast<uint8_t*>(p);
     c.arena.cap = cap;
 }
+// gives back, on stream s, the blocks of device dev that no call holds, over all threads; s waits for those
+// whose work is still going on.  Whether there were any.
+bool give_back_unused(int dev, hipStream_t s) {
+    Registry& r = registry();
+    const std::lock_guard<std::mutex> all(r.m);
+    bool any = false;
+    for (CallCache* C : r.caches) {
+        const std::lock_guard<std::mutex> lock(C->m);
+        for (CacheSlot& c : C->slots) {
+            if (!c.arena.base || c.dev != dev || (C->live > 0 && &c == C->cur)) continue;
+            if (!slot_idle(c) && hipStreamWaitEvent(s, c.done, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
+            }
+            resize_block(c, 0, s);
+            any = true;
+        }
+    }
+    return any;
+}
+
+// one more call of the thread on another block: blocks that have been passed over for long go back
+void age_blocks(CallCache& C, const CacheSlot* used, hipStream_t s) {
+    for (CacheSlot& c : C.slots) {
+        if (&c == used) c.passed = 0;
+        else if (c.arena.base && ++c.passed >= kCacheAge && c.dev == used->dev && slot_idle(c)) resize_block(c, 0, s);
+    }
+}
+
+// whether s is a stream of the current device, *dev, that is not being captured
+bool plain_stream(hipStream_t s, int* dev) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    int sdev = 0;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone && hipGetDevice(dev) == hipSuccess &&
+        (!s || (hipStreamGetDevice(s, &sdev) == hipSuccess && sdev == *dev)))
+        return true;
+    (void)hipGetLastError();
+    return false;
+}
 size_t block_size(size_t bytes) { return (bytes + bytes / 8 + kCacheStep) / kCacheStep * kCacheStep; }
 }  // namespace
 
 void* call_cache_take(size_t bytes, hipStream_t s) {
     CallCache& C = call_cache();
+    const std::lock_guard<std::mutex> lock(C.m);
     if (C.live == 0) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        if (bytes > kCacheBlock) return nullptr;
-        if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
         // a block belongs to the stream's device, its event to the current one: serve where they agree
-        int dev = 0, sdev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || (s && hipStreamGetDevice(s, &sdev) != hipSuccess) || (s && sdev != dev)) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+        int dev = 0;
+        if (bytes > kCacheBlock || !plain_stream(s, &dev)) return nullptr;
         CacheSlot* c = pick_slot(C, dev, s);
         if (!c) return nullptr;
         c->stream = s;
+        age_blocks(C, c, s);
         if (++c->calls >= kCacheWindow) {
             if (c->arena.cap > 4 * c->recent && c->arena.cap > 32 * kCacheStep) resize_block(*c, block_size(2 * c->recent), s);
             c->calls = 0;
@@ -187,6 +246,7 @@ void* call_cache_take(size_t bytes, hipStream_t s) {
 
 void call_cache_give(void* p) {
     CallCache& C = call_cache();
+    const std::lock_guard<std::mutex> lock(C.m);
     CacheSlot& c = *C.cur;
     (void)c.arena.give(p);
     if (--C.live > 0) return;
@@ -200,6 +260,25 @@ void call_cache_give(void* p) {
         c.pending = false;
     }
     C.cur = nullptr;
+}
+
+hipError_t pool_alloc(void** p, size_t bytes, hipStream_t s) {
+    hipError_t e = hipMallocAsync(p, bytes, s);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    int dev = 0;
+    if (!plain_stream(s, &dev) || !give_back_unused(dev, s)) return e;
+    e = hipMallocAsync(p, bytes, s);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    // the freed blocks may be pieces that the pool holds on to: wait until they are free and let it return them
+    const RelaxedCapture relaxed;
+    hipMemPool_t pool;
+    if (hipStreamSynchronize(s) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess &&
+        hipMemPoolTrimTo(pool, 0) == hipSuccess)
+        e = hipMallocAsync(p, bytes, s);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 }  // namespace nsc

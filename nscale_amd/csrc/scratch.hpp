@@ -57,6 +57,8 @@ struct ArenaScope {
 // pool does then.
 void* call_cache_take(size_t bytes, hipStream_t s);
 void call_cache_give(void* p);
+// hipMallocAsync; where memory is short, once more after every thread's unused blocks have gone back
+hipError_t pool_alloc(void** p, size_t bytes, hipStream_t s);
 
 struct Scratch {
     void* p = nullptr;
@@ -80,7 +82,7 @@ struct Scratch {
             from_cache = true;
             return NSC_OK;
         }
-        hipError_t e = hipMallocAsync(&p, bytes, stream);
+        const hipError_t e = pool_alloc(&p, bytes, stream);
         if (e != hipSuccess) {
             p = nullptr;
             set_error("hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));

@@ -1,6 +1,7 @@
 // The call cache (nscale_amd/csrc/call_cache.cpp) against a stand-in for the HIP runtime: memory with a limit,
 // streams and events whose work is done when the test says so, and the rule that a call which is unsafe while
 // a stream is captured in global mode ends the capture.  Argument: the check to run.
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -17,11 +18,14 @@ std::recursive_mutex mu;
 struct Fake {
     std::map<void*, size_t> mem;
     size_t used = 0, limit = ~(size_t)0;
+    size_t held = 0;       // freed bytes that the pool keeps until it is trimmed (with keeps)
+    bool keeps = false;
     bool capturing = false, invalidated = false;  // some stream is being captured, in global mode
     struct Event { bool recorded = false, done = true; uintptr_t stream = 0; };
     std::vector<Event> events;
     std::map<uintptr_t, bool> busy;               // streams with work that has not ended
     std::vector<std::pair<uintptr_t, size_t>> waits;
+    std::vector<uintptr_t> freed_on;
     int bad_frees = 0, own_streams = 0;
 } F;
 thread_local hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
@@ -42,7 +46,7 @@ Arena*& thread_arena() { static thread_local Arena* a = nullptr; return a; }
 extern "C" {
 hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) {
     Lock l(mu);
-    if (F.used + n > F.limit) return hipErrorOutOfMemory;
+    if (F.used + F.held + n > F.limit) return hipErrorOutOfMemory;
     *p = std::malloc(1);
     F.mem[*p] = n;
     F.used += n;
@@ -54,6 +58,8 @@ hipError_t hipFreeAsync(void* p, hipStream_t s) {
     auto it = F.mem.find(p);
     if (it == F.mem.end()) { ++F.bad_frees; return hipErrorInvalidValue; }
     F.used -= it->second;
+    if (F.keeps) F.held += it->second;
+    F.freed_on.push_back(reinterpret_cast<uintptr_t>(s));
     F.mem.erase(it);
     return hipSuccess;
 }
@@ -110,6 +116,8 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
 }
 hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t* d) { *d = 0; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t* p, int) { *p = nullptr; return hipSuccess; }
+hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { Lock l(mu); F.held = 0; return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
 }
@@ -140,15 +148,84 @@ void capture() {
     EXPECT(mode == hipStreamCaptureModeGlobal);
     F.capturing = false;
 }
+
+// an allocation that fails finds the memory of unused blocks: this thread's and other threads', with work
+// that has ended and with work that the stream has to wait for, with a pool that reuses and one that keeps
+void pressure() {
+    for (bool keeps : {false, true}) {
+        F.keeps = keeps;
+        F.limit = ~(size_t)0;
+        for (uintptr_t s = 1; s <= 3; ++s) EXPECT(call(s, 900 * MB) == NSC_OK);
+        EXPECT(F.used > 2700 * MB);
+        F.limit = 3400 * MB;
+        F.waits.clear();
+        F.freed_on.clear();
+        EXPECT(call(4, 2500 * MB) == NSC_OK);  // above a block's bound: the pool's own
+        EXPECT(F.waits.size() == 3 && F.freed_on.size() == 4);  // three blocks, then the buffer itself
+        for (auto& w : F.waits) EXPECT(w.first == reinterpret_cast<uintptr_t>(stream(4)));
+        for (uintptr_t q : F.freed_on) EXPECT(q == reinterpret_cast<uintptr_t>(stream(4)));
+        end_work();
+        F.held = 0;
+    }
+    F.keeps = false;
+    // another thread's blocks, while it lives and makes no call
+    std::mutex gate;
+    gate.lock();
+    std::atomic<bool> ready{false};
+    std::thread other([&] {
+        EXPECT(call(8, 900 * MB) == NSC_OK);
+        EXPECT(call(9, 900 * MB) == NSC_OK);
+        ready = true;
+        gate.lock();
+        EXPECT(call(8, 100 * MB) == NSC_OK);  // and goes on without them
+        gate.unlock();
+    });
+    while (!ready) std::this_thread::yield();
+    F.limit = 3000 * MB;
+    EXPECT(call(4, 2500 * MB) == NSC_OK);
+    gate.unlock();
+    other.join();
+    // a block that a call holds is kept, and the failure is reported
+    {
+        nsc::Scratch a, b;
+        EXPECT(a.alloc(500 * MB, stream(1)) == NSC_OK);
+        const size_t before = F.used;
+        EXPECT(b.alloc(2900 * MB, stream(1)) == NSC_ERR_NOMEM);
+        EXPECT(F.used == before && F.mem.size() == 1);
+    }
+    // nothing is given back on a captured stream's behalf, and the capture goes on
+    F.capturing = true;
+    EXPECT(call(0, 2900 * MB) == NSC_ERR_NOMEM);
+    EXPECT(!F.invalidated);
+    F.capturing = false;
+}
+
+// blocks of streams that have gone quiet go back while the thread works on another one
+void age() {
+    for (uintptr_t s = 1; s <= 4; ++s) EXPECT(call(s, 300 * MB) == NSC_OK);
+    EXPECT(F.used >= 1200 * MB);
+    end_work();
+    for (int k = 0; k < 200; ++k) EXPECT(call(1, 300 * MB) == NSC_OK);
+    EXPECT(F.used >= 300 * MB && F.used < 400 * MB);
+    for (uintptr_t s = 2; s <= 4; ++s) EXPECT(call(s, 300 * MB) == NSC_OK);
+    EXPECT(F.used >= 1200 * MB);
+    // streams in turn: none of them is quiet
+    const size_t before = F.used;
+    for (int k = 0; k < 800; ++k) EXPECT(call(1 + k % 4, 300 * MB) == NSC_OK);
+    EXPECT(F.used == before);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     std::thread t([&] {  // its end gives its blocks back
         if (!std::strcmp(what, "capture")) capture();
+        else if (!std::strcmp(what, "pressure")) pressure();
+        else if (!std::strcmp(what, "age")) age();
         else EXPECT(!"a check of that name");
     });
     t.join();
+    F.limit = ~(size_t)0;
     EXPECT(F.mem.empty() && F.used == 0 && !F.bad_frees);
     if (failures) std::printf("%s: %d failures\n", what, failures);
     return failures != 0;

@@ -28,3 +28,11 @@ def _run(program, what):
 
 def test_a_capture_on_another_stream_goes_on(program):
     _run(program, "capture")
+
+
+def test_a_failing_allocation_finds_the_unused_blocks(program):
+    _run(program, "pressure")
+
+
+def test_blocks_of_quiet_streams_go_back(program):
+    _run(program, "age")
