@@ -62,6 +62,9 @@ struct Dev {
     // written when the item is queued, its pop index when it pops; records of other ids hold anything.
     // {run, largest-key item of the push chain, level << 24 | pop index, pusher (pixel, -1 = initial push)}
     int4* wr;
+    // pop indexes from popcap on (a record then holds popcap); no plane where no run can have so many pops
+    int32_t* popx;
+    int popcap;
     int32_t* lab;  // F pixel: label decided in its run's flood, 0 = never queued there
     int32_t* qnext;  // FIFO links of the global-memory floods, indexed by item id
     // leaves
@@ -105,7 +108,10 @@ __device__ __forceinline__ int cdiff_packed(uint32_t a, uint32_t b) {
 // ---- item accessors ----
 constexpr int kPopMax = 1 << 24;
 __device__ __forceinline__ int rec_lvl(const int4& r) { return (int)((uint32_t)r.z >> 24); }
-__device__ __forceinline__ int rec_pop(const int4& r) { return r.z & (kPopMax - 1); }
+__device__ __forceinline__ int rec_pop(const Dev& D, int x, const int4& r) {
+    const int q = r.z & (kPopMax - 1);
+    return D.popx && q == D.popcap ? D.popx[x] : q;
+}
 __device__ __forceinline__ int it_lvl(const Dev& D, int x) { return rec_lvl(D.wr[x]); }
 __device__ __forceinline__ int it_parent(const Dev& D, int x) { return D.wr[x].w; }
 
@@ -115,7 +121,7 @@ __device__ bool before_from(const Dev& D, int x, int y, int step0) {
     for (int step = step0; step < CMP_MAX_STEPS; ++step) {
         if (x == y) return false;
         const int4 rx = D.wr[x], ry = D.wr[y];
-        if (rx.x == ry.x) return rec_pop(rx) < rec_pop(ry);
+        if (rx.x == ry.x) return rec_pop(D, x, rx) < rec_pop(D, y, ry);
         const int a = rx.y, b = ry.y;
         const int4 ra = D.wr[a], rb = D.wr[b];
         const int la = rec_lvl(ra), lb = rec_lvl(rb);
@@ -141,7 +147,7 @@ struct ItemKey {
 __device__ __forceinline__ ItemKey item_key(const Dev& D, int x) {
     const int4 rx = D.wr[x];
     const int4 ra = D.wr[rx.y];
-    return ItemKey{x, rx.x, rec_pop(rx), rx.y, rec_lvl(ra), ra.w};
+    return ItemKey{x, rx.x, rec_pop(D, x, rx), rx.y, rec_lvl(ra), ra.w};
 }
 // before(D, kx.item, ky.item), its first step taken from the keys
 __device__ __forceinline__ bool before_keyed(const Dev& D, const ItemKey& kx, const ItemKey& ky) {
@@ -323,8 +329,9 @@ __device__ void flood_global(const Dev& D, const int32_t* __restrict__ box5, int
         const int nx = D.qnext[x];
         head[active] = nx;
         if (nx < 0) tail[active] = -1;
-        if (popc == kPopMax) { atomicOr(D.flags, FB_LEAF_CAP); return; }
-        D.wr[x].z |= popc++;
+        D.wr[x].z |= min(popc, D.popcap);
+        if (D.popx && popc >= D.popcap) D.popx[x] = popc;
+        ++popc;
         if (x >= D.N) continue;  // a leaf: when it pops, nothing else
         const int p = x;
         int lab = 0;
@@ -676,7 +683,8 @@ constexpr int P1_WAVES = 16, P1_UNITS = 158;  // 64 frame pixels a unit
 constexpr int kRunTiers = 6;
 // runs by the size of their LDS frame: tier b holds frames of at most kRunTier[b] pixels; the last one
 // floods from global memory
-__constant__ int kRunTier[kRunTiers - 1] = {512, 1024, 2048, 4096, 6400};
+constexpr int kRunTierMax = 6400;
+__constant__ int kRunTier[kRunTiers - 1] = {512, 1024, 2048, 4096, kRunTierMax};
 
 struct LdsPool {
     unsigned long long used[3];
@@ -1032,7 +1040,7 @@ __global__ void k_t1_state(Dev D, const int32_t* __restrict__ real, const int* _
         for (int j = 0; j < 4; ++j) {
             v[j] = c[j] == C_B && p0 + j == b1 ? Y1 : 0;
             if (it[j] >= 0) {
-                const ItemKey k{it[j], rec[j].x, rec_pop(rec[j]), rec[j].y, rec_lvl(top[j]), top[j].w};
+                const ItemKey k{it[j], rec[j].x, rec_pop(D, it[j], rec[j]), rec[j].y, rec_lvl(top[j]), top[j].w};
                 if (b1 < 0 || before_keyed(D, k, kb)) v[j] = c[j] == C_F ? lab[j] : WSHED;
                 else if (rec[j].w < 0 || before(D, rec[j].w, b1i)) {
                     v[j] = IN_QUEUE;
@@ -1915,6 +1923,12 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
     Dev D{};
     D.img = img; D.W = W; D.H = H; D.N = (int)N; D.m0 = m0; D.m = m; D.cls = cls; D.lvl0 = lvl0; D.run = run;
     D.lab = lab; D.head = head; D.nleaf = &small[2]; D.flags = &small[3];
+    // A run's pops are at most the image's inner pixels (a pixel pops once as F, once a run as a leaf), and an F
+    // pixel has four neighbours: only runs of larger images can outgrow the records' 24 bits, the largest index
+    // standing for itself or, with the plane, for what the plane holds.  NSC_WS_POP_CAP lowers the line (tests of
+    // the plane; not below the LDS floods' largest frame, whose indexes are always their records').
+    D.popcap = kPopMax - 1;
+    if (const char* e = getenv("NSC_WS_POP_CAP")) D.popcap = std::min(std::max(atoi(e), kRunTierMax + 1), kPopMax - 1);
     {  // real[] is unused until B resolution: it holds the per-workgroup counts
         const unsigned nb = (unsigned)std::min<size_t>(cdiv(N, 256), 1u << 14);
         hipLaunchKernelGGL(k_classify, dim3(nb), dim3(256), 0, s, D, cls, lvl0, fmask, real);
@@ -1931,21 +1945,23 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
     // phase-1 scratch: run boxes, per-run FIFO heads/tails, queue links, leaf table, item records
     const int leafcap = std::max(1024, std::min((int)std::min(N, (size_t)INT_MAX / 4), 4 * nF + 1024));
     Carver m2(nullptr);
-    auto carve2 = [&](Carver& c, int32_t*& box5, int*& qh, int*& qt, int32_t*& qnext, int32_t*& lf, int4*& wr) {
+    const bool manypops = std::min((long long)(W - 2) * (H - 2), 5ll * nF) > (long long)D.popcap + 1;
+    auto carve2 = [&](Carver& c, int32_t*& box5, int*& qh, int*& qt, int32_t*& qnext, int32_t*& lf, int4*& wr, int32_t*& popx) {
         box5 = c.take<int32_t>(5 * (size_t)std::max(nrun, 1));
         qh = c.take<int>((size_t)std::max(nrun, 1) * (NQ + kRunTiers));  // run buckets, then FIFO heads
         qt = c.take<int>((size_t)std::max(nrun, 1) * NQ);
         qnext = c.take<int32_t>(N + (size_t)leafcap);
         lf = c.take<int32_t>((size_t)leafcap * 2);
         wr = c.take<int4>(N + (size_t)leafcap);
+        popx = manypops ? c.take<int32_t>(N + (size_t)leafcap) : nullptr;
     };
     int32_t *box5, *qnext, *lf;
     int *qh, *qt;
-    carve2(m2, box5, qh, qt, qnext, lf, D.wr);
+    carve2(m2, box5, qh, qt, qnext, lf, D.wr, D.popx);
     Scratch sc2;
     NSC_CHECK(sc2.alloc(m2.size(), s));
     Carver cut2(sc2.p);
-    carve2(cut2, box5, qh, qt, qnext, lf, D.wr);
+    carve2(cut2, box5, qh, qt, qnext, lf, D.wr, D.popx);
     D.qnext = qnext;
     D.leafcap = leafcap;
     D.lf_b = lf;
