@@ -14,14 +14,17 @@
 //    one packed 16-bit operation, while dx^2 is below its best squared distance (four pairs per thread
 //    at once: with one, a turn is a round trip to LDS and 512^2 took 40 us).  A result of at most
 //    32^2 is exact: every candidate it has not seen is larger (dx > 32, or g > 32 where the cap or the
-//    missing words hide it).  Pixels further away flag their row.
+//    missing words hide it).  Pixels further away flag their row.  Two waves that the first step leaves
+//    idle find the last zero above and the first below the segment in each of its columns.
 // 3. k_edt_rows: flagged rows (the others' workgroups leave at once).  g of the whole row from the
-//    words; each flagged pixel searches outward over the row; a search that would exceed SEARCH_CAP
+//    words and those zeros; each flagged pixel searches outward over the row; a search that would exceed SEARCH_CAP
 //    columns has the row recomputed with the exact integer lower-envelope algorithm.
-// The masks are 1/8 byte per pixel, so nothing but the image and the result moves: 4096^2 nuclei mask
-// 44 us.  (With the vertical distances as a 16-bit plane, segments' carries, one pixel per lane
-// and 32-bit squares in the search, six launches: 190 us, of which the search 78, bound by its
-// instructions.)
+// The masks are 1/8 byte per pixel, the zeros beyond the segments 1/16, so little but the image and the result
+// moves: 4096^2 nuclei mask, whose rows all leave at once in step 3, 44 us.  (With the vertical distances as a
+// 16-bit plane, segments' carries, one pixel per lane and 32-bit squares in the search, six launches: 190 us, of
+// which the search 78, bound by its instructions.)  Masks with distances past 32 pay for their flagged rows: 4096^2
+// with a hole of radius 8 every 128 pixels 1080 us, of radius 4 every 300 1940 (1690 and 2520 when every
+// flagged row walked its columns' words to the next zero).
 #include "common.hpp"
 
 namespace nsc {
@@ -59,7 +62,8 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u16x2 pk(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
 
 __global__ __launch_bounds__(E_THREADS) void k_edt_tiles(const uint64_t* __restrict__ zm, int w, int h, int nseg,
-                                                      float* __restrict__ out, int* __restrict__ rowflag) {
+                                                      float* __restrict__ out, int* __restrict__ rowflag,
+                                                      uint16_t* __restrict__ above, uint16_t* __restrict__ below) {
     __shared__ uint16_t G[SEG][E_WIDE];
     const int sg = blockIdx.y, y0 = sg * SEG, x0 = blockIdx.x * E_COLS;
     if (threadIdx.x < E_WIDE) {
@@ -84,6 +88,26 @@ __global__ __launch_bounds__(E_THREADS) void k_edt_tiles(const uint64_t* __restr
             d = min(d + 1u, g[j]);  // g[j] is 0 at a zero
             G[j][threadIdx.x] = (uint16_t)d;
         }
+    } else {
+        // waves 2 and 3: the row of the column's last zero above, first zero below the segment
+        static_assert(E_WIDE == 128 && E_THREADS == 256 && E_COLS == 64, "a wave each, a lane per column");
+        const bool up = threadIdx.x < 192;  // wave-uniform
+        const int x = x0 + (int)(threadIdx.x & 63), step = up ? -1 : 1, n = up ? sg : nseg - 1 - sg;
+        const uint64_t* const col = zm + min(x, w - 1);
+        int row = -1;
+        // the next segment's word, which nearly always holds one, then eight words' loads at a time
+        auto hit = [&](uint64_t q, int s) { return s * SEG + (up ? 63 - (int)__clzll((long long)q) : (int)__ffsll((long long)q) - 1); };
+        if (n > 0)
+            if (const uint64_t q = col[(size_t)(sg + step) * w]) row = hit(q, sg + step);
+        for (int k0 = 2; k0 <= n && row < 0; k0 += 8) {
+            uint64_t q[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) q[j] = col[(size_t)(sg + step * min(k0 + j, n)) * w];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (row < 0 && q[j]) row = hit(q[j], sg + step * min(k0 + j, n));
+        }
+        if (x < w) (up ? above : below)[(size_t)sg * w + x] = row < 0 ? NONE : (uint16_t)row;
     }
     __syncthreads();
     constexpr int NP = E_COLS / 2, STEP = E_THREADS / NP, K = 4;  // pairs per row, rows per step
@@ -152,29 +176,19 @@ __device__ __forceinline__ float edt_value(long long dx2, long long g) {
 }
 
 __global__ __launch_bounds__(256) void k_edt_rows(const uint64_t* __restrict__ zm, int w, int h, int nseg,
-                                                  float* __restrict__ out, const int* __restrict__ rowflag) {
+                                                  float* __restrict__ out, const int* __restrict__ rowflag,
+                                                  const uint16_t* __restrict__ above, const uint16_t* __restrict__ below) {
     extern __shared__ uint16_t lds[];
     const int y = blockIdx.x;
     if (!rowflag[y]) return;
     uint16_t* const grow = lds;  // vertical distances of the row (NONE: no zero in the column)
     const int sg = y / SEG, j = y % SEG;
     for (int x = threadIdx.x; x < w; x += blockDim.x) {
-        const uint64_t m = zm[(size_t)sg * w + x], le = m & ((2ull << j) - 1ull), ge = m >> j;
-        uint32_t du = NONE, dd = NONE;
-        if (le) du = (uint32_t)(j - 63 + (int)__clzll((long long)le));
-        else
-            for (int s = sg - 1; s >= 0; --s)
-                if (const uint64_t q = zm[(size_t)s * w + x]) {
-                    du = (uint32_t)(y - (s * SEG + 63 - (int)__clzll((long long)q)));
-                    break;
-                }
-        if (ge) dd = (uint32_t)__ffsll((long long)ge) - 1u;
-        else
-            for (int s = sg + 1; s < nseg; ++s)
-                if (const uint64_t q = zm[(size_t)s * w + x]) {
-                    dd = (uint32_t)(s * SEG + (int)__ffsll((long long)q) - 1 - y);
-                    break;
-                }
+        const size_t i = (size_t)sg * w + x;
+        const uint64_t m = zm[i], le = m & ((2ull << j) - 1ull), ge = m >> j;
+        const uint32_t a = above[i], b = below[i];
+        const uint32_t du = le ? (uint32_t)(j - 63 + (int)__clzll((long long)le)) : (a != NONE ? (uint32_t)y - a : NONE);
+        const uint32_t dd = ge ? (uint32_t)__ffsll((long long)ge) - 1u : (b != NONE ? b - (uint32_t)y : NONE);
         grow[x] = (uint16_t)min(du, dd);
     }
     __shared__ int need, kk;
@@ -269,18 +283,22 @@ int edt_impl(const uint8_t* img, float* out, int w, int h, hipStream_t s) {
     Carver measure(nullptr);
     measure.take<uint64_t>((size_t)nseg * w);
     measure.take<int>(h);
+    measure.take<uint16_t>((size_t)nseg * w);
+    measure.take<uint16_t>((size_t)nseg * w);
     Scratch sc;
     NSC_CHECK(sc.alloc(measure.size(), s));
     Carver cut(sc.p);
     uint64_t* zm = cut.take<uint64_t>((size_t)nseg * w);
     int* rowflag = cut.take<int>(h);
+    uint16_t* above = cut.take<uint16_t>((size_t)nseg * w);
+    uint16_t* below = cut.take<uint16_t>((size_t)nseg * w);
     hipLaunchKernelGGL(k_edt_masks, dim3(cdiv(w, 64), nseg), dim3(64), 0, s, img, w, h, zm, rowflag);
-    hipLaunchKernelGGL(k_edt_tiles, dim3(cdiv(w, E_COLS), nseg), dim3(E_THREADS), 0, s, zm, w, h, nseg, out, rowflag);
+    hipLaunchKernelGGL(k_edt_tiles, dim3(cdiv(w, E_COLS), nseg), dim3(E_THREADS), 0, s, zm, w, h, nseg, out, rowflag, above, below);
     // the launch is unconditional and the workgroups of unflagged rows leave at once (no host sync)
     const size_t lds = 2 * sizeof(uint16_t) * (size_t)w;
     if (lds > 64 * 1024)
         NSC_HIP(hipFuncSetAttribute((const void*)k_edt_rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_edt_rows, dim3(h), dim3(256), lds, s, zm, w, h, nseg, out, rowflag);
+    hipLaunchKernelGGL(k_edt_rows, dim3(h), dim3(256), lds, s, zm, w, h, nseg, out, rowflag, above, below);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
 }
