@@ -27,13 +27,14 @@
 #include <cmath>
 
 #include "common.hpp"
+#include "normalize_rules.hpp"
 #include "normalize_tables.hpp"
 
 namespace nsc {
 namespace {
 
 constexpr int kNormThreads = 512;
-constexpr int kNormChunk = 4 * kNormThreads;  // pixels per work item
+constexpr int kNormChunk = 4 * kNormThreads;  // pixels per work item (at most)
 // statistics partials (8 doubles each): two workgroups per CU, few enough that every workgroup of
 // k_norm_apply can sum them itself
 constexpr int kNormMaxBlocks = 512;
@@ -203,13 +204,22 @@ __device__ __forceinline__ bool norm_bg_fast(const NormBg& G, float b, float g, 
     return sure;
 }
 
-// The image as rows of chunks; an image without gaps between its rows is taken as one long row.
+// The image as groups of four consecutive pixels of a row (a row's last group may hold fewer), numbered row by
+// row; an image without gaps between its rows is taken as one long row.  The passes take groups in turn, so
+// the lanes of a workgroup have work whatever the rows' length.  (With a row's chunks of 2048 pixels to a workgroup,
+// a crop of width 100 kept 25 of its 512 threads busy: 100 x 3900 pixels 53 us a call, by groups 18.)
 struct NormImage {
     const uint8_t* bgr;
     size_t ld;
-    size_t w;  // pixels per row
-    long long chunks_per_row, items;
+    size_t w;                    // pixels per row
+    unsigned long long per_row;  // groups per row
+    unsigned long long magic;    // of per_row (normalize_rules.hpp)
+    unsigned long long groups;
+    bool one_row;
 };
+
+// work items: a group per thread of a workgroup
+__host__ __device__ inline long long norm_items(const NormImage& I) { return (long long)((I.groups + kNormThreads - 1) / kNormThreads); }
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -217,12 +227,14 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// work item it: byte offset of its first pixel in a plane of row stride ld, and its pixel count
-__device__ __forceinline__ int norm_item(const NormImage& I, long long it, size_t ld, size_t* off) {
-    const long long y = it / I.chunks_per_row;
-    const size_t x0 = (size_t)(it - y * I.chunks_per_row) * kNormChunk;
+// group q: byte offset of its first pixel in a plane of row stride ld, and its pixel count (0 past the last).
+__device__ __forceinline__ int norm_group(const NormImage& I, unsigned long long q, size_t ld, size_t* off) {
+    *off = 0;
+    if (q >= I.groups) return 0;
+    const unsigned long long y = I.one_row ? 0ull : row_of(q, I.magic);
+    const size_t x0 = 4 * (size_t)(q - y * I.per_row);
     *off = (size_t)y * ld + 3 * x0;
-    return (int)std::min<size_t>(kNormChunk, I.w - x0);
+    return (int)std::min<size_t>(4, I.w - x0);
 }
 
 // the thread's four pixels (12 bytes; n of them exist) as three words, by words where p is aligned
@@ -264,7 +276,7 @@ __device__ __forceinline__ void stats_add(const NormConsts& C, const NormDisc& D
 }
 
 // Per-workgroup sums over the selected pixels: [sum L, sum a, sum b, sq L, sq a, sq b, count, 0].
-// Every wave goes through its own 256-pixel pieces of the work items and keeps a list of the
+// Every wave goes through its own pieces of 64 groups (256 pixels at most) and keeps a list of the
 // foreground pixels it met; whenever the list holds 64 it takes 64 off, so all lanes work, nothing
 // waits on another wave, and the order of the additions depends on the grid alone.  The next
 // piece's words are on their way while the current one is listed.
@@ -273,22 +285,19 @@ __device__ __forceinline__ void stats_add(const NormConsts& C, const NormDisc& D
 constexpr int kStatsPiece = 256;
 __global__ __launch_bounds__(kNormThreads) void k_norm_stats(NormImage I, NormConsts C, NormDisc D,
                                                              double* __restrict__ part) {
-    constexpr int kWaves = kNormThreads / 64, kPer = kNormChunk / kStatsPiece;
+    constexpr int kWaves = kNormThreads / 64;
     __shared__ double2 lg[kLogTabN];
     __shared__ uint32_t lists[kWaves][64 + kStatsPiece];
     const int wv = threadIdx.x >> 6, ln = threadIdx.x & 63;
     uint32_t* const list = lists[wv];
     double acc[7] = {0, 0, 0, 0, 0, 0, 0};
-    const long long pieces = I.items * kPer, step = (long long)gridDim.x * kWaves;
-    // a piece's words and the number of pixels the lane has of it (pieces past a row's end: none)
+    const long long pieces = (long long)((I.groups + 63) / 64), step = (long long)gridDim.x * kWaves;
+    // a piece's words and the number of pixels the lane has of it (past the last group: none)
     auto load = [&](long long pc, uint32_t wd[3]) {
-        wd[0] = wd[1] = wd[2] = 0;
-        if (pc >= pieces) return 0;
         size_t off;
-        const int q = (int)(pc % kPer) * kStatsPiece + 4 * ln;
-        const int n = norm_item(I, pc / kPer, I.ld, &off) - q;
-        const int mine = min(max(n, 0), 4);
-        norm_load4(I.bgr + off + 3 * (size_t)q, mine, wd);
+        const int mine = norm_group(I, 64ull * (unsigned long long)pc + (unsigned)ln, I.ld, &off);
+        wd[0] = wd[1] = wd[2] = 0;
+        if (mine) norm_load4(I.bgr + off, mine, wd);
         return mine;
     };
     int held = 0;  // wave-uniform
@@ -394,10 +403,11 @@ __global__ __launch_bounds__(kNormThreads, 6) void k_norm_apply(NormImage I, Nor
     // while the tables and the totals are made
     auto load = [&](long long it, uint32_t wd[3]) {
         size_t off;
-        const int mine = min(max(norm_item(I, it, I.ld, &off) - 4 * (int)threadIdx.x, 0), 4);
-        norm_load4(I.bgr + off + 12 * (size_t)threadIdx.x, mine, wd);
+        const int mine = norm_group(I, (unsigned long long)it * kNormThreads + threadIdx.x, I.ld, &off);
+        norm_load4(I.bgr + off, mine, wd);
         return mine;
     };
+    const long long items = norm_items(I);
     uint32_t wd[3];
     int mine = load(blockIdx.x, wd);  // the grid has at most one workgroup per item
     load_log_tab(T.lg);
@@ -414,7 +424,7 @@ __global__ __launch_bounds__(kNormThreads, 6) void k_norm_apply(NormImage I, Nor
     const NormParams P = sP;
     uint8_t* const by = reinterpret_cast<uint8_t*>(buf);
     int turn = 0;
-    for (long long it = blockIdx.x; it < I.items; it += gridDim.x, turn ^= 1) {
+    for (long long it = blockIdx.x; it < items; it += gridDim.x, turn ^= 1) {
         if (it != (long long)blockIdx.x) mine = load(it, wd);
         uint32_t px[4];
 #pragma unroll
@@ -460,8 +470,8 @@ __global__ __launch_bounds__(kNormThreads, 6) void k_norm_apply(NormImage I, Nor
         }
         __syncthreads();
         size_t ooff;
-        (void)norm_item(I, it, out_ld, &ooff);
-        uint8_t* q = out + ooff + 12 * (size_t)threadIdx.x;
+        (void)norm_group(I, (unsigned long long)it * kNormThreads + threadIdx.x, out_ld, &ooff);
+        uint8_t* q = out + ooff;
         if (mine == 4 && (reinterpret_cast<uintptr_t>(q) & 3) == 0) {
             uint32_t* qw = reinterpret_cast<uint32_t*>(q);
             qw[0] = buf[3 * threadIdx.x];
@@ -504,12 +514,14 @@ NormImage image_of(const uint8_t* bgr, int w, int h, size_t ld, bool dense) {
     I.bgr = bgr;
     I.ld = ld;
     I.w = dense ? (size_t)w * h : (size_t)w;
-    I.chunks_per_row = (long long)((I.w + kNormChunk - 1) / kNormChunk);
-    I.items = dense ? I.chunks_per_row : h * I.chunks_per_row;
+    I.one_row = dense;
+    I.per_row = (I.w + 3) / 4;
+    I.magic = row_magic(I.per_row);
+    I.groups = I.per_row * (dense ? 1ull : (unsigned long long)h);
     return I;
 }
 
-int stats_blocks(const NormImage& I) { return (int)std::min<long long>(I.items, kNormMaxBlocks); }
+int stats_blocks(const NormImage& I) { return (int)std::min<long long>(norm_items(I), kNormMaxBlocks); }
 
 size_t norm_scratch_bytes(int nblocks) { return sizeof(double) * 8 * ((size_t)nblocks + 1); }
 
@@ -574,7 +586,7 @@ extern "C" int nsc_normalization(const uint8_t* bgr, int w, int h, size_t ld, co
         T.ratio[k] = target_std3[k];  // k_norm_apply divides it by the image's
     }
     hipLaunchKernelGGL(k_norm_stats, dim3(nb), dim3(kNormThreads), 0, s, I, host_consts(), host_disc(), part);
-    const int nbx = (int)std::min<long long>(I.items, kApplyMaxBlocks);
+    const int nbx = (int)std::min<long long>(norm_items(I), kApplyMaxBlocks);
     hipLaunchKernelGGL(k_norm_apply, dim3(nbx), dim3(kNormThreads), 0, s, I, host_consts(), host_disc(), host_bg(), part, nb,
                        T, out, out_ld);
     NSC_HIP(hipGetLastError());
