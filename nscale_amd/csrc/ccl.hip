@@ -12,18 +12,22 @@
 // foreground F and the run starts S.
 //   1. ccl_tile: one wave per tile, lane = row.  Bit operations on F and S give the joins to unite
 //      (a run's own joins need no union), the runs, numbered in raster order, unite in LDS with
-//      atomicMin on their numbers, and the tile leaves behind its F and S words, the number of the
-//      tile-local root of every run (two bytes), the places of the roots along its four edges, and for
-//      each tile-local root its entry in the forest P (the root's own global index) with what the
-//      caller needs of it: pixel count or flag;
+//      atomicMin on their numbers, and the tile leaves behind its F and S words, a code for every run
+//      (two bytes: the number of its tile-local root, whether that root is closed, and if so whether it is
+//      selected), the places of the roots along its four edges, and for each open root its entry in the
+//      forest P (the root's own global index) with what the caller needs of it: pixel count or flag.  A
+//      component that meets no other tile is closed: its root, count and flag are final there;
 //   2. ccl_seams: two waves per tile unite the runs that meet across its left and its top edge, in P;
-//   3. ccl_roots (selections): each tile-local root finds its final root and hands its count or flag
-//      over;
+//   3. ccl_roots (selections): each open root, found along the edges, finds its final root and hands its
+//      count or flag over;
 //   4. ccl_select writes the selected pixels, ccl_label the labels: both expand the words again.
-// P is indexed by pixel but only the entries of tile-local roots exist; no other per-pixel label is
+// P is indexed by pixel but only the entries of open roots exist; no other per-pixel label is
 // stored on the way.  Bytes moved per pixel: about 0.4 for the words and roots, the image in and the
 // result out.  Labelling per pixel instead (labels in LDS, stored, seams from the stored labels, a
 // flattening pass, a consumer pass) moved 17 and was bound by instruction issue in its tile pass.
+// Only what crosses an edge is followed through memory: an image may have as many components as pixels.  With an
+// entry, a walk and a lookup for every tile-local root, area opening of 4096 x 4096 differing pixels took 1365 us
+// (183 with codes), hole filling of a checkerboard 573 (82), labels of 50 % noise 600 x 600 44 (31).
 // Pixel classes: FG_NEQ  -> foreground = value != key; neighbours join when both foreground
 //                FG_EQ   -> foreground = value != 0; neighbours join when values are equal
 //                FG_FEQ  -> foreground = cls != 0; neighbours join when float values are equal
@@ -138,10 +142,12 @@ struct RowWords {
 };
 
 // What a labelling leaves per tile: the words of its 64 rows, the number of runs before each row, the
-// number of the tile-local root of every run, the places of the roots along the four edges (kNoRoot
+// code of every run (the number of its tile-local root; kClosed where the component meets no other tile,
+// and then kSelected where a selection takes it), the places of the roots along the four edges (kNoRoot
 // for background), and, for the equal-value modes, the values of its first and last column (the seams
 // compare them).
 constexpr uint16_t kNoRoot = 0xFFFF;
+constexpr uint32_t kRunRoot = 0x0FFF, kSelected = 0x4000, kClosed = 0x8000;
 enum { E_LEFT = 0, E_RIGHT = 1, E_TOP = 2, E_BOTTOM = 3 };
 struct CclBufs {
     RowWords* rows;
@@ -242,11 +248,11 @@ __device__ __forceinline__ JoinWords joins_to_unite(uint64_t jl, uint64_t ju, ui
 // The words and joins of a tile where equal byte values join: the tile's bytes come to LDS, each lane
 // takes its row as 16 dwords (and the row above from the lane before it), and every comparison with a
 // neighbour is byte arithmetic on four pixels at a time.  (One ballot per row and comparison took 51 us
-// for a 4096 x 3071 mask, this 23 us.)
+// for a 4096 x 3071 mask, this 23 us.)  Returns the row's first and last byte, one above the other.
 constexpr int kBytePitch = 17;  // dwords per staged row: the lanes' rows start in different banks
 template <int CONN>
-__device__ __forceinline__ void tile_words_eq(const uint8_t* __restrict__ img, int w, int h, int x0, int y0, RowWords& R,
-                                              JoinWords& J, uint8_t* edge, uint32_t* stage) {
+__device__ __forceinline__ uint32_t tile_words_eq(const uint8_t* __restrict__ img, int w, int h, int x0, int y0, RowWords& R,
+                                              JoinWords& J, uint32_t* stage) {
     const int lane = threadIdx.x & 63, r = lane >> 2, x = 16 * (lane & 3);
     const int cols = min(CT, w - x0);
     const bool full = cols == CT;
@@ -286,12 +292,11 @@ __device__ __forceinline__ void tile_words_eq(const uint8_t* __restrict__ img, i
     }
     if (!full) F &= (1ull << cols) - 1ull;
     if (y0 + lane >= h) F = 0;
-    edge[lane] = (uint8_t)c[0];
-    edge[CT + lane] = (uint8_t)(c[15] >> 24);
     const uint64_t Fu = shfl_up64(F);
     const uint64_t jl = F & (F << 1) & ~nl;
     R = RowWords{F & ~jl, F};
     J = joins_to_unite<CONN>(jl, F & Fu & ~nu, F & (Fu << 1) & ~nul, F & (Fu >> 1) & ~nur, shfl_up64(jl));
+    return (c[0] & 255u) | (c[15] >> 24) << 8;
 }
 
 // The same where equal floats join (NaN joins nothing): four waves of 16 rows each, lane = column; each
@@ -351,71 +356,66 @@ __device__ __forceinline__ void tile_words_feq(const Px& P, int w, int h, int x0
 enum { SRC_NONE = 0, SRC_BYTES = 1, SRC_BORDER = 2 };
 
 constexpr int ccl_cap(int mode) { return mode == FG_NEQ ? CT * CT / 2 : CT * CT; }  // most runs of a tile
-constexpr int ccl_tile_threads(int mode) { return mode == FG_FEQ ? 256 : 64; }
+constexpr int kManyRuns = 512;  // runs from which four waves share a tile: eight a row, a mask of noise
+constexpr int kFewRuns = 512;   // codes that the consumers load before they know the run count
+constexpr int ccl_tile_threads(int mode, int waves) { return mode == FG_FEQ ? 256 : 64 * waves; }
 
-// One tile per workgroup (its first wave, once the words are there).  Per tile-local root: P = its own
-// index; area (optional) = the pixels of its tile-local component; flag (optional) = whether that
-// holds a source pixel: a nonzero pixel of src (SRC_BYTES) or a pixel on the image border
-// (SRC_BORDER).  *zero (optional) is cleared for the passes that follow.
-template <int MODE, int CONN, int SRC>
-__global__ __launch_bounds__(ccl_tile_threads(MODE)) void ccl_tile(Px P, CclBufs B, int32_t* __restrict__ forest, int w, int h,
-                                                                   int tiles_x, int32_t* __restrict__ area,
-                                                                   uint8_t* __restrict__ flag,
-                                                                   const uint8_t* __restrict__ src, int* __restrict__ zero) {
-    // the runs' nodes (8 KB of LDS for binary masks: every tile of a 4096^2 image is resident at once)
-    __shared__ uint32_t node[ccl_cap(MODE)];
-    __shared__ union {
-        uint16_t bits[4 * CT];
-        uint32_t bytes[MODE == FG_EQ ? CT * kBytePitch : 1];
-        uint64_t words[MODE == FG_FEQ ? CT : 1][kEqWords];
-    } stage;
-    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x;
-    const int x0 = tx * CT, y0 = ty * CT, lane = threadIdx.x & 63;
-    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
-    RowWords R;
-    JoinWords J;
-    if constexpr (MODE == FG_NEQ) {
-        R.F = tile_bits(P.img, w, h, x0, y0, P.key, stage.bits);
-        const uint64_t jl = R.F & (R.F << 1), Fu = shfl_up64(R.F);
-        R.S = R.F & ~jl;
-        J = joins_to_unite<CONN>(jl, R.F & Fu, R.F & (Fu << 1), R.F & (Fu >> 1), Fu & (Fu << 1));
-    } else if constexpr (MODE == FG_EQ) {
-        tile_words_eq<CONN>(P.img, w, h, x0, y0, R, J, static_cast<uint8_t*>(B.edge) + (size_t)blockIdx.x * 2 * CT,
-                            stage.bytes);
-    } else {
-        tile_words_feq<CONN>(P, w, h, x0, y0, R, J, static_cast<float*>(B.edge) + (size_t)blockIdx.x * 2 * CT, stage.words);
-        if (threadIdx.x >= 64) return;
-        wave_order();  // the words have been read before their LDS holds bits
-    }
-    uint64_t T = 0;  // source pixels of the row
-    if constexpr (SRC == SRC_BYTES) T = tile_bits(src, w, h, x0, y0, 0, stage.bits);
-    if constexpr (SRC == SRC_BORDER) {
-        const int y = y0 + lane;
-        if (y == 0 || y == h - 1) T = ~0ull;
-        if (x0 == 0) T |= 1ull;
-        if (w - 1 - x0 < CT) T |= 1ull << (w - 1 - x0);
-    }
-    // the rows' first run numbers: exclusive scan of the run counts
-    const int nrun = popc64(R.S);
-    int off = nrun;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int q = __shfl_up(off, o);
-        if (lane >= o) off += q;
-    }
-    off -= nrun;
-    B.rows[(size_t)blockIdx.x * CT + lane] = R;
-    B.off[(size_t)blockIdx.x * CT + lane] = (uint16_t)off;
+// global index of the place r of tile (tx, ty)
+__device__ __forceinline__ int place_index(int tx, int ty, int r, int w) {
+    return (int)((size_t)(ty * CT + (r >> 6)) * w + (tx * CT + (r & 63)));
+}
+// whether another tile lies across a side of tile (tx, ty)
+__device__ __forceinline__ bool side_open(int side, int tx, int ty, int tiles_x, int tiles_y) {
+    return side == E_LEFT ? tx > 0 : (side == E_RIGHT ? tx + 1 < tiles_x : (side == E_TOP ? ty > 0 : ty + 1 < tiles_y));
+}
+
+// A tile from its words on, by one wave (solo) or by four, each with the runs that start in 16 columns.
+struct TileWork {
+    CclBufs B;
+    int32_t* forest;
+    int w, tx, ty, tiles_x, tiles_y;
+    int32_t* area;
+    int lo, hi;
+    uint8_t* flag;
+};
+template <int SRC, bool solo>
+__device__ __forceinline__ void ccl_tile_runs(const TileWork& K, uint32_t* node, const RowWords R, JoinWords J, const uint64_t T,
+                                              const int off, const int wv) {
+    const CclBufs& B = K.B;
+    int32_t* const forest = K.forest;
+    int32_t* const area = K.area;
+    uint8_t* const flag = K.flag;
+    const int w = K.w, tx = K.tx, ty = K.ty, tiles_x = K.tiles_x, tiles_y = K.tiles_y, lo = K.lo, hi = K.hi;
+    const int lane = threadIdx.x & 63;
+    const int nrun = popc64(R.S), tid = solo ? lane : (int)threadIdx.x;
+    constexpr int threads = solo ? 64 : 256;
+    // between steps that read in LDS what another lane has written
+    auto order = [&] {
+        if (solo) wave_order();
+        else __syncthreads();
+    };
+    auto any = [&](bool v) { return solo ? __any(v) != 0 : __syncthreads_or(v ? 1 : 0) != 0; };
     const uint64_t Su = shfl_up64(R.S);
     const int offu = dpp_from_left(0, off);
     const int row = lane * CT, runs = __builtin_amdgcn_readlane(off + nrun, 63);
+    // the wave's runs, the number of the first, and their joins
+    uint64_t mine = R.S;
+    int first = off;
+    if (!solo) {
+        const uint64_t before = (1ull << (16 * wv)) - 1ull, in = 0xFFFFull << (16 * wv);
+        mine = R.S & in;
+        first = off + popc64(R.S & before);
+        const uint64_t after = R.S & ~(before | in);  // the next wave's first run ends the last of these
+        const uint64_t px = mine ? (after ? (after & (0ull - after)) - 1ull : ~0ull) & ~((mine & (0ull - mine)) - 1ull) : 0ull;
+        J = JoinWords{J.up & px, J.ul & px, J.ur & px};
+    }
     // A run starts out pointing at the run above of one of its joins, if it has any (a smaller number,
     // so this is a forest without any atomics), and the forest is flattened: along a tall component
     // one union per row at once would build a chain that every later find walks.  The joins that
     // are left, where a run meets a second run above it, unite what is flat already.
     {
-        int k = off;
-        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+        int k = first;
+        for (uint64_t m = mine; m; m &= m - 1, ++k) {
             const int a = __ffsll((long long)m) - 1;
             const uint64_t rb = run_bits(a, run_end(R.S, R.F, a)), up = J.up & rb, ul = J.ul & rb, ur = J.ur & rb;
             const uint64_t f = up ? up : (ul ? ul : ur);
@@ -429,33 +429,33 @@ __global__ __launch_bounds__(ccl_tile_threads(MODE)) void ccl_tile(Px P, CclBufs
             node[k] = (uint32_t)(row + a) << 16 | (uint32_t)par;
         }
     }
-    wave_order();
-    // every run at its root: pointer doubling, lane = run, four runs' reads in one round trip
+    order();
+    // every run at its root: pointer doubling, thread = run, four runs' reads in one round trip
     auto flatten = [&]() {
         for (;;) {
             bool changed = false;
-            for (int k0 = 0; k0 < runs; k0 += 256) {
+            for (int k0 = 0; k0 < runs; k0 += 4 * threads) {
                 uint32_t v[4];
                 int q[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = node_of(node, min(k0 + 64 * j + lane, runs - 1));
+                for (int j = 0; j < 4; ++j) v[j] = node_of(node, min(k0 + threads * j + tid, runs - 1));
 #pragma unroll
                 for (int j = 0; j < 4; ++j) q[j] = parent_of(node, (int)(v[j] & 0xFFFFu));
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const int k = k0 + 64 * j + lane;
+                    const int k = k0 + threads * j + tid;
                     if (k < runs && q[j] != (int)(v[j] & 0xFFFFu)) {
                         node[k] = (v[j] & 0xFFFF0000u) | (uint32_t)q[j];
                         changed = true;
                     }
                 }
             }
-            wave_order();
-            if (!__any(changed)) break;
+            if (solo) wave_order();
+            if (!any(changed)) break;
         }
     };
     flatten();
-    if (__any((J.up | J.ul | J.ur) != 0)) {
+    if (any((J.up | J.ul | J.ur) != 0)) {
         // one union per lane and turn, straight ones first
         while (J.up | J.ul | J.ur) {
             const uint64_t m = J.up ? J.up : (J.ul ? J.ul : J.ur);
@@ -466,19 +466,26 @@ __global__ __launch_bounds__(ccl_tile_threads(MODE)) void ccl_tile(Px P, CclBufs
             else J.ur &= clr;
             lunite(node, off + run_index(R.S, x), offu + run_index(Su, xu));
         }
-        wave_order();
+        order();
         flatten();
     }
-    uint16_t* const roots = B.roots + (size_t)blockIdx.x * B.cap;
+    // edge pixels: left and right of the lane's row, top and bottom of the lane's column.  Roots that they hold
+    // on a side with a tile across it are open.
+    constexpr uint32_t kOpen = 1u << 30;
     uint16_t* const er = B.edge_roots + (size_t)blockIdx.x * 4 * CT;
-    for (int k = lane; k < runs; k += 64) roots[k] = (uint16_t)parent_of(node, k);
-    wave_order();
+    int eroot[4], eplace[4];  // open roots that no pixel before it on the side has: number (else -1), place
     {
-        // edge pixels: left and right of the lane's row, top and bottom of the lane's column
-        auto root_place = [&](bool fg, int k) {
+        auto edge = [&](int side, bool fg, int k) {
+            eroot[side] = -1;
+            eplace[side] = 0;
+            if (!solo && side != wv) return;  // a side a wave
             const int r = fg ? parent_of(node, k) : 0;
-            const uint32_t p = node[r] >> 16;
-            return fg ? (uint16_t)p : kNoRoot;
+            const int p = (int)(node_of(node, r) >> 16 & 0xFFFu);
+            er[side * CT + lane] = fg ? (uint16_t)p : kNoRoot;
+            const int o = fg && side_open(side, tx, ty, tiles_x, tiles_y) ? r : -1;
+            eroot[side] = o != dpp_from_left(-1, o) ? o : -1;
+            eplace[side] = p;
+            if (eroot[side] >= 0) atomicOr(&node[o], kOpen);  // (bits that no reader of a place or parent looks at)
         };
         auto word_of = [](uint64_t v, int l) {
             return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l) |
@@ -486,40 +493,152 @@ __global__ __launch_bounds__(ccl_tile_threads(MODE)) void ccl_tile(Px P, CclBufs
         };
         const uint64_t S0 = word_of(R.S, 0), F0 = word_of(R.F, 0), S3 = word_of(R.S, 63), F3 = word_of(R.F, 63);
         const int off3 = __builtin_amdgcn_readlane(off, 63);
-        er[E_LEFT * CT + lane] = root_place(R.F & 1ull, off);
-        er[E_RIGHT * CT + lane] = root_place(R.F >> 63, off + nrun - 1);
-        er[E_TOP * CT + lane] = root_place((F0 >> lane) & 1ull, run_index(S0, lane));
-        er[E_BOTTOM * CT + lane] = root_place((F3 >> lane) & 1ull, off3 + run_index(S3, lane));
+        edge(E_LEFT, R.F & 1ull, off);
+        edge(E_RIGHT, R.F >> 63, off + nrun - 1);
+        edge(E_TOP, (F0 >> lane) & 1ull, run_index(S0, lane));
+        edge(E_BOTTOM, (F3 >> lane) & 1ull, off3 + run_index(S3, lane));
     }
+    order();
     if (area || SRC != SRC_NONE) {
         // the roots' places are not needed any more: count in bits 16..28, flag in bit 31
-        wave_order();
-        int k = off;
-        for (uint64_t m = R.S; m; m &= m - 1, ++k)
-            if (parent_of(node, k) == k) node[k] = (uint32_t)k;
-        wave_order();
-        k = off;
-        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
+        for (int k = tid; k < runs; k += threads) {
+            const uint32_t v = node_of(node, k);
+            if ((int)(v & 0xFFFFu) == k) node[k] = (v & kOpen) | (uint32_t)k;
+        }
+        order();
+        int k = first;
+        for (uint64_t m = mine; m; m &= m - 1, ++k) {
             const int a = __ffsll((long long)m) - 1, end = run_end(R.S, R.F, a), r = parent_of(node, k);
             if (area) atomicAdd(&node[r], (uint32_t)(end - a) << 16);
             if (SRC != SRC_NONE && (T & run_bits(a, end))) atomicOr(&node[r], 0x80000000u);
         }
-        wave_order();
+        order();
     }
-    int k = off;
-    for (uint64_t m = R.S; m; m &= m - 1, ++k) {
-        const uint32_t v = node_of(node, k);
-        if ((int)(v & 0xFFFFu) != k) continue;
-        const int g = (int)((size_t)(y0 + lane) * w + (x0 + __ffsll((long long)m) - 1));
+    // the runs' codes, four at a time
+    uint16_t* const roots = B.roots + (size_t)blockIdx.x * B.cap;
+    for (int k0 = 4 * tid; k0 < runs; k0 += 4 * threads) {
+        const uint4 q = *reinterpret_cast<const uint4*>(&node[k0]);
+        const uint32_t r[4] = {q.x & kRunRoot, q.y & kRunRoot, q.z & kRunRoot, q.w & kRunRoot};
+        uint32_t code[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t v = node_of(node, k0 + j < runs ? (int)r[j] : 0);
+            const int c = (int)(v >> 16 & 0x1FFFu);
+            const bool sel = SRC != SRC_NONE ? (v >> 31) != 0 : area && c >= lo && c < hi;
+            code[j] = r[j] | (v & kOpen ? 0u : kClosed | (sel ? kSelected : 0u));
+        }
+        *reinterpret_cast<uint2*>(roots + k0) = make_uint2(code[0] | code[1] << 16, code[2] | code[3] << 16);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (eroot[e] < 0) continue;
+        const uint32_t v = node_of(node, eroot[e]);
+        const int g = place_index(tx, ty, eplace[e], w);
         forest[g] = g;
         if (area) area[g] = (int)(v >> 16 & 0x1FFFu);
         if (SRC != SRC_NONE) flag[g] = (uint8_t)(v >> 31);
     }
 }
 
-// global index of the place r of tile (tx, ty)
-__device__ __forceinline__ int place_index(int tx, int ty, int r, int w) {
-    return (int)((size_t)(ty * CT + (r >> 6)) * w + (tx * CT + (r & 63)));
+// One tile per workgroup, by its first wave once the words are there; where the launch has four waves a tile
+// (kFewTiles), a tile of more than kManyRuns runs is shared by all four.  Per open root: P = its own index; area
+// (optional) = the pixels of its tile-local component; flag (optional) = whether that holds a source
+// pixel: a nonzero pixel of src (SRC_BYTES) or a pixel on the image border (SRC_BORDER).  A closed root is
+// selected by its area in [lo, hi), or by its flag.  *zero (optional) is cleared for the passes that follow.
+template <int MODE, int CONN, int SRC, int WAVES>
+__global__ __launch_bounds__(ccl_tile_threads(MODE, WAVES)) void ccl_tile(Px P, CclBufs B, int32_t* __restrict__ forest, int w, int h,
+                                                                   int tiles_x, int32_t* __restrict__ area, int lo,
+                                                                   int hi, uint8_t* __restrict__ flag,
+                                                                   const uint8_t* __restrict__ src, int* __restrict__ zero) {
+    // the runs' nodes (8 KB of LDS for binary masks: every tile of a 4096^2 image is resident at once)
+    __shared__ alignas(16) uint32_t node[ccl_cap(MODE)];
+    __shared__ union {
+        uint16_t bits[4 * CT];
+        uint32_t bytes[MODE == FG_EQ ? CT * kBytePitch : 1];
+        uint64_t words[MODE == FG_FEQ ? CT : 1][kEqWords];
+    } stage;
+    __shared__ uint64_t shared_words[WAVES > 1 ? CT : 1][6];
+    __shared__ int shared_runs;
+    const int tx = blockIdx.x % tiles_x, ty = blockIdx.x / tiles_x, tiles_y = gridDim.x / tiles_x;
+    const int x0 = tx * CT, y0 = ty * CT, lane = threadIdx.x & 63;
+    const int wv = ccl_tile_threads(MODE, WAVES) == 64 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
+    RowWords R{};
+    JoinWords J{};
+    uint64_t T = 0;  // source pixels of the row
+    uint32_t ends = 0;
+    if constexpr (MODE == FG_FEQ) {
+        tile_words_feq<CONN>(P, w, h, x0, y0, R, J, static_cast<float*>(B.edge) + (size_t)blockIdx.x * 2 * CT, stage.words);
+        if (WAVES == 1 && wv) return;
+        if (WAVES > 1) __syncthreads();
+        else wave_order();  // the words have been read before their LDS holds bits
+    }
+    if (wv == 0) {
+        if constexpr (MODE == FG_NEQ) {
+            R.F = tile_bits(P.img, w, h, x0, y0, P.key, stage.bits);
+            const uint64_t jl = R.F & (R.F << 1), Fu = shfl_up64(R.F);
+            R.S = R.F & ~jl;
+            J = joins_to_unite<CONN>(jl, R.F & Fu, R.F & (Fu << 1), R.F & (Fu >> 1), Fu & (Fu << 1));
+        } else if constexpr (MODE == FG_EQ) {
+            ends = tile_words_eq<CONN>(P.img, w, h, x0, y0, R, J, stage.bytes);
+        }
+        if constexpr (SRC == SRC_BYTES) T = tile_bits(src, w, h, x0, y0, 0, stage.bits);
+        if constexpr (SRC == SRC_BORDER) {
+            const int y = y0 + lane;
+            if (y == 0 || y == h - 1) T = ~0ull;
+            if (x0 == 0) T |= 1ull;
+            if (w - 1 - x0 < CT) T |= 1ull << (w - 1 - x0);
+        }
+    }
+    // the rows' first run numbers: exclusive scan of the run counts
+    auto first_runs = [&] {
+        int o = popc64(R.S);
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int q = __shfl_up(o, d);
+            if (lane >= d) o += q;
+        }
+        return o - popc64(R.S);
+    };
+    int off = first_runs();
+    bool solo = true;
+    if constexpr (WAVES > 1) {
+        if (wv == 0) {
+            const uint64_t v[6] = {R.S, R.F, J.up, J.ul, J.ur, T};
+            const int n = __builtin_amdgcn_readlane(off + popc64(R.S), 63);
+            if (lane == 0) shared_runs = n;
+            if (n > kManyRuns)
+#pragma unroll
+                for (int k = 0; k < 6; ++k) shared_words[lane][k] = v[k];
+        }
+        __syncthreads();
+        solo = __builtin_amdgcn_readfirstlane(shared_runs) <= kManyRuns;  // (wave-uniform)
+        if (solo && wv) return;
+        if (!solo && wv) {
+            const uint64_t* v = shared_words[lane];
+            R = RowWords{v[0], v[1]};
+            J = JoinWords{v[2], v[3], v[4]};
+            T = v[5];
+            off = first_runs();
+        }
+    }
+    if (wv == 0) {  // (stores after the barrier, which would wait for them)
+        B.rows[(size_t)blockIdx.x * CT + lane] = R;
+        B.off[(size_t)blockIdx.x * CT + lane] = (uint16_t)off;
+        if constexpr (MODE == FG_EQ) {
+            uint8_t* const edge = static_cast<uint8_t*>(B.edge) + (size_t)blockIdx.x * 2 * CT;
+            edge[lane] = (uint8_t)ends;
+            edge[CT + lane] = (uint8_t)(ends >> 8);
+        }
+    }
+    const TileWork K{B, forest, w, tx, ty, tiles_x, tiles_y, area, lo, hi, flag};
+    if constexpr (WAVES > 1) {
+        if (__builtin_expect(!solo, 0)) {
+            ccl_tile_runs<SRC, false>(K, node, R, J, T, off, wv);
+            return;
+        }
+    }
+    ccl_tile_runs<SRC, true>(K, node, R, J, T, off, wv);
 }
 
 // Unions across tile edges: the tile's first wave takes the pixels of its first column with their left
@@ -606,23 +725,40 @@ __device__ __forceinline__ int final_root(const int32_t* forest, int g) {
     return r;
 }
 
-// Every tile-local root that is not final hands its count or flag to the final root and points at it.
+// A lane's four pixels of a tile's 256 edge pixels (16 lanes a side) and their roots' places; those that are
+// open, and not the pixel's before it, are visited.
+__device__ __forceinline__ uint2 edge_places(const CclBufs& B, int t) {
+    return *reinterpret_cast<const uint2*>(B.edge_roots + ((size_t)t * 4 * CT + 4 * (threadIdx.x & 63)));
+}
+template <class Visit>
+__device__ __forceinline__ void open_edge_roots(uint2 q, int tx, int ty, int tiles_x, int tiles_y, Visit visit) {
+    const int lane = threadIdx.x & 63;
+    const bool open = side_open(lane >> 4, tx, ty, tiles_x, tiles_y);
+    const uint32_t p[4] = {q.x & 0xFFFFu, q.x >> 16, q.y & 0xFFFFu, q.y >> 16};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) visit((int)p[j], open && p[j] != kNoRoot && (j == 0 || p[j] != p[j ? j - 1 : 0]));
+}
+
+// Every open root that is not final hands its count or flag to the final root and points at it.
 __global__ __launch_bounds__(256) void ccl_roots(CclBufs B, int32_t* forest, int w, int tiles_x, int ntiles, int32_t* area,
                                                  uint8_t* flag) {
+    __shared__ uint32_t seen_s[4][CT * CT / 32];  // by place
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (t >= ntiles) return;
-    const uint64_t S = B.rows[(size_t)t * CT + lane].S;
-    int k = B.off[(size_t)t * CT + lane];
-    const uint16_t* roots = B.roots + (size_t)t * B.cap;
-    for (uint64_t m = S; m; m &= m - 1, ++k) {
-        if (roots[k] != k) continue;
-        const int g = place_index(t % tiles_x, t / tiles_x, lane * CT + __ffsll((long long)m) - 1, w);
-        const int r = final_root(forest, g);
-        if (r == g) continue;
+    uint32_t* const seen = seen_s[threadIdx.x >> 6];
+    const uint2 places = edge_places(B, t);
+    seen[lane] = 0;
+    seen[64 + lane] = 0;
+    wave_order();
+    const int tx = t % tiles_x, ty = t / tiles_x;
+    open_edge_roots(places, tx, ty, tiles_x, ntiles / tiles_x, [&](int p, bool take) {
+        if (!take || (atomicOr(&seen[p >> 5], 1u << (p & 31)) >> (p & 31) & 1u)) return;
+        const int g = place_index(tx, ty, p, w), r = final_root(forest, g);
+        if (r == g) return;
         forest[g] = r;
         if (area) atomicAdd(&area[r], area[g]);
         if (flag && flag[g]) flag[r] = 1;
-    }
+    });
 }
 
 // What a selection writes per pixel, sel = the pixel's component is selected (by its area in [lo, hi),
@@ -647,8 +783,9 @@ __device__ __forceinline__ uint32_t select_word(uint32_t sel, uint32_t a, uint32
     return sel;
 }
 
-// One tile per wave: the selected tile-local roots become bits in LDS, the selected runs bits of the
-// rows' words (lane = row), the words bytes (a lane writes four 16-byte pieces, a row is four lanes).
+// One tile per wave: the selected open roots become bits in LDS (by run number), the selected runs bits of the
+// rows' words (lane = row; the codes staged in LDS, cap of them a wave), the words bytes (a lane writes four
+// 16-byte pieces, a row is four lanes).
 // *count (optional) = number of selected components, counted at their final roots; one atomic per
 // workgroup, and the grid is at most kSelectBlocks (atomics on one address cost about 10 ns each: one
 // per tile of a 4096^2 image took 40 us).
@@ -660,7 +797,10 @@ __global__ __launch_bounds__(256) void ccl_select(CclBufs B, const int32_t* __re
                                                   uint8_t* out, int* count) {
     __shared__ uint32_t keep_s[4][CT * CT / 32];
     __shared__ uint64_t words_s[4][CT];
+    extern __shared__ uint4 codes_s[];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    uint4* const codes8 = codes_s + (size_t)wv * (B.cap / 8);
+    const uint16_t* const codes = reinterpret_cast<const uint16_t*>(codes8);
     uint32_t* const keep = keep_s[wv];
     uint64_t* const words = words_s[wv];
     int n = 0;
@@ -668,30 +808,43 @@ __global__ __launch_bounds__(256) void ccl_select(CclBufs B, const int32_t* __re
         const int tx = t % tiles_x, ty = t / tiles_x;
         const RowWords R = B.rows[(size_t)t * CT + lane];
         const int off = B.off[(size_t)t * CT + lane];
-        const uint16_t* roots = B.roots + (size_t)t * B.cap;
+        const uint2 places = edge_places(B, t);
+        const uint4* roots = reinterpret_cast<const uint4*>(B.roots + (size_t)t * B.cap);
+        codes8[lane] = roots[lane];  // a usual tile's codes, without waiting for its run count
+        const int runs = __builtin_amdgcn_readlane(off + popc64(R.S), 63);
+        for (int k = 64 + lane; 8 * k < runs; k += 64) codes8[k] = roots[k];
         keep[lane] = 0;
         keep[64 + lane] = 0;
         wave_order();
-        int k = off;
-        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
-            if (roots[k] != k) continue;
-            const int g = place_index(tx, ty, lane * CT + __ffsll((long long)m) - 1, w), r = forest[g];  // final: ccl_roots has run
+        open_edge_roots(places, tx, ty, tiles_x, ntiles / tiles_x, [&](int p, bool take) {
+            // the run that starts there, from its row's words (every lane takes part)
+            const int row = take ? p >> 6 : 0;
+            const uint64_t S = (uint64_t)(uint32_t)__shfl((int)(uint32_t)R.S, row) |
+                               (uint64_t)(uint32_t)__shfl((int)(uint32_t)(R.S >> 32), row) << 32;
+            const int k = __shfl(off, row) + run_index(S, p & 63);
+            if (!take) return;
+            const int g = place_index(tx, ty, p, w), r = forest[g];  // final: ccl_roots has run
             bool s;
             if (OUT == OUT_MASK) {
                 const int ar = area[r];
                 s = ar >= lo && ar < hi;
-                n += (s && r == g) ? 1 : 0;
             } else {
                 s = flag[r] != 0;
             }
-            if (s) atomicOr(&keep[k >> 5], 1u << (k & 31));
-        }
+            if (!s) return;
+            const bool first = !(atomicOr(&keep[k >> 5], 1u << (k & 31)) >> (k & 31) & 1u);
+            if (OUT == OUT_MASK) n += (first && r == g) ? 1 : 0;
+        });
         wave_order();
         uint64_t sel = 0;
-        k = off;
+        int k = off;
         for (uint64_t m = R.S; m; m &= m - 1, ++k) {
-            const int x = __ffsll((long long)m) - 1, r = roots[k];
-            if ((keep[r >> 5] >> (r & 31)) & 1u) sel |= run_bits(x, run_end(R.S, R.F, x));
+            const uint32_t c = codes[k], r = c & kRunRoot;
+            const bool s = c & kClosed ? (c & kSelected) != 0 : ((keep[r >> 5] >> (r & 31)) & 1u) != 0;
+            if (!s) continue;
+            const int x = __ffsll((long long)m) - 1;
+            sel |= run_bits(x, run_end(R.S, R.F, x));
+            if (OUT == OUT_MASK) n += ((c & kClosed) && (int)r == k) ? 1 : 0;
         }
         words[lane] = OUT == OUT_UNSEL ? R.F & ~sel : sel;
         wave_order();
@@ -722,9 +875,10 @@ __global__ __launch_bounds__(256) void ccl_select(CclBufs B, const int32_t* __re
     if (count) block_count_add(n, count);  // `count` is the same for every thread
 }
 
-// Labels of a tile: the final root of each tile-local root, then of each run, in LDS; then lane = column
-// and a row a step.  forest may be the label image itself: a root's entry is overwritten with its
-// final root, which any walk may meet instead of the entry it replaces, and no other entry is read.
+// Labels of a tile by run, in LDS: every run's own first pixel (a closed root's label), the open roots' final
+// roots (thread = edge pixel), then each run's root's label; then lane = column and a row a step.  forest
+// may be the label image itself: an open root's entry is overwritten with its final root, which any walk may
+// meet instead of the entry it replaces, and no other entry is read.
 __global__ __launch_bounds__(256) void ccl_label(CclBufs B, int32_t* forest, int32_t* L, int w, int h, int tiles_x,
                                                  int32_t bgval) {
     __shared__ int lab[CT * CT];  // by run number
@@ -733,7 +887,18 @@ __global__ __launch_bounds__(256) void ccl_label(CclBufs B, int32_t* forest, int
     const int t = blockIdx.x, tx = t % tiles_x, ty = t / tiles_x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const RowWords R = B.rows[(size_t)t * CT + lane];
     const int off = B.off[(size_t)t * CT + lane];
-    const uint16_t* roots = B.roots + (size_t)t * B.cap;
+    const int p = B.edge_roots[(size_t)t * 4 * CT + threadIdx.x];
+    // eight codes at a time, all of a thread's before their use; a usual tile's without waiting for its run count
+    const uint4* roots = reinterpret_cast<const uint4*>(B.roots + (size_t)t * B.cap);
+    constexpr int kPer = CT * CT / (8 * 256);
+    uint4 codes[kPer];
+    if (threadIdx.x < kFewRuns / 8) codes[0] = roots[threadIdx.x];
+    const int runs = __builtin_amdgcn_readlane(off + popc64(R.S), 63);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const int k = threadIdx.x + 256 * j;
+        if (k >= kFewRuns / 8 && 8 * k < runs) codes[j] = roots[k];
+    }
     if (wv == 0) {
         words[lane] = R;
         offs[lane] = off;
@@ -741,18 +906,21 @@ __global__ __launch_bounds__(256) void ccl_label(CclBufs B, int32_t* forest, int
     // the four waves take a row's runs in turn
     {
         int k = off;
-        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
-            if (((k - off) & 3) != wv) continue;
-            if (roots[k] == k) lab[k] = final_root(forest, place_index(tx, ty, lane * CT + __ffsll((long long)m) - 1, w));
-        }
+        for (uint64_t m = R.S; m; m &= m - 1, ++k)
+            if (((k - off) & 3) == wv) lab[k] = place_index(tx, ty, lane * CT + __ffsll((long long)m) - 1, w);
     }
     __syncthreads();
-    {
-        int k = off;
-        for (uint64_t m = R.S; m; m &= m - 1, ++k) {
-            if (((k - off) & 3) != wv) continue;
-            const int r = roots[k];
-            if (r != k) lab[k] = lab[r];
+    if (side_open(wv, tx, ty, tiles_x, (int)gridDim.x / tiles_x) && p != kNoRoot && p != dpp_from_left(-1, p))
+        lab[offs[p >> 6] + run_index(words[p >> 6].S, p & 63)] = final_root(forest, place_index(tx, ty, p, w));
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        if (8 * ((int)threadIdx.x + 256 * j) >= runs) break;
+        const uint32_t c[4] = {codes[j].x, codes[j].y, codes[j].z, codes[j].w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int k = 8 * ((int)threadIdx.x + 256 * j) + i, r = (int)(c[i >> 1] >> (16 * (i & 1)) & kRunRoot);
+            if (k < runs && r != k) lab[k] = lab[r];  // (roots' entries are only read)
         }
     }
     __syncthreads();
@@ -789,24 +957,38 @@ CclBufs ccl_carve(Carver& c, int nt, int mode) {
     return B;
 }
 
+// LDS of a ccl_select workgroup beside its fixed part: the codes of four tiles
+size_t select_lds(const CclBufs& B) { return 4 * sizeof(uint16_t) * (size_t)B.cap; }
+
 struct CclWork {  // a labelling in progress
     Scratch sc;
     CclBufs B;
     CclGrid g;
 };
 
+// Launches of at most kFewTiles tiles (two a CU, 1448 x 1448) give a tile four waves: there a tile of many runs lasts
+// as long as its own loops over them.  Kernel time at 600 x 600, one wave a tile and four: 50 % noise 24.6 and
+// 17.3 us, discs 7.4 and 7.7 (three of the four leave at once).  More tiles fill the chip by themselves, and the
+// idle waves take room: hole filling of 4096 x 4096 discs 56 us a call with one wave, 62 with four.
+constexpr int kFewTiles = 512;
+
 // the tile and seam passes; flag / src: see ccl_tile
 template <int MODE, int CONN, int SRC>
-int ccl_forest_t(const Px& P, CclWork& W, int32_t* forest, int w, int h, int32_t* area, uint8_t* flag, const uint8_t* src,
-                 int* zero, hipStream_t s) {
+int ccl_forest_t(const Px& P, CclWork& W, int32_t* forest, int w, int h, int32_t* area, int lo, int hi, uint8_t* flag,
+                 const uint8_t* src, int* zero, hipStream_t s) {
     W.g = ccl_grid(w, h);
     Carver m(nullptr);
     (void)ccl_carve(m, W.g.nt, MODE);
     NSC_CHECK(W.sc.alloc(m.size(), s));
     Carver c(W.sc.p);
     W.B = ccl_carve(c, W.g.nt, MODE);
-    hipLaunchKernelGGL((ccl_tile<MODE, CONN, SRC>), dim3(W.g.nt), dim3(ccl_tile_threads(MODE)), 0, s, P, W.B, forest, w, h, W.g.tiles_x, area,
-                       flag, src, zero);
+    auto tiles = [&](auto waves) {
+        constexpr int WAVES = decltype(waves)::value;
+        hipLaunchKernelGGL((ccl_tile<MODE, CONN, SRC, WAVES>), dim3(W.g.nt), dim3(ccl_tile_threads(MODE, WAVES)), 0, s, P, W.B,
+                           forest, w, h, W.g.tiles_x, area, lo, hi, flag, src, zero);
+    };
+    if (W.g.nt <= kFewTiles) tiles(std::integral_constant<int, 4>{});
+    else tiles(std::integral_constant<int, 1>{});
     hipLaunchKernelGGL((ccl_seams<MODE, CONN>), dim3(W.g.nt), dim3(128), 0, s, P, W.B, forest, w, h, W.g.tiles_x);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
@@ -815,8 +997,8 @@ int ccl_forest_t(const Px& P, CclWork& W, int32_t* forest, int w, int h, int32_t
 template <int MODE>
 int ccl_labels(const Px& P, int32_t* L, int w, int h, int conn, int32_t bgval, hipStream_t s) {
     CclWork W;
-    if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_NONE>(P, W, L, w, h, nullptr, nullptr, nullptr, nullptr, s)));
-    else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_NONE>(P, W, L, w, h, nullptr, nullptr, nullptr, nullptr, s)));
+    if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_NONE>(P, W, L, w, h, nullptr, 0, 0, nullptr, nullptr, nullptr, s)));
+    else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_NONE>(P, W, L, w, h, nullptr, 0, 0, nullptr, nullptr, nullptr, s)));
     hipLaunchKernelGGL(ccl_label, dim3(W.g.nt), dim3(256), 0, s, W.B, L, L, w, h, W.g.tiles_x, bgval);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
@@ -828,15 +1010,15 @@ int ccl_select_flag(const Px& P, const uint8_t* src, const uint8_t* a, const uin
                     int32_t* forest, uint8_t* flag, hipStream_t s) {
     CclWork W;
     if (src) {
-        if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_BYTES>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
-        else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_BYTES>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
+        if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_BYTES>(P, W, forest, w, h, nullptr, 0, 0, flag, src, nullptr, s)));
+        else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_BYTES>(P, W, forest, w, h, nullptr, 0, 0, flag, src, nullptr, s)));
     } else {
-        if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_BORDER>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
-        else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_BORDER>(P, W, forest, w, h, nullptr, flag, src, nullptr, s)));
+        if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_BORDER>(P, W, forest, w, h, nullptr, 0, 0, flag, src, nullptr, s)));
+        else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_BORDER>(P, W, forest, w, h, nullptr, 0, 0, flag, src, nullptr, s)));
     }
     hipLaunchKernelGGL(ccl_roots, dim3(cdiv(W.g.nt, 4)), dim3(256), 0, s, W.B, forest, w, W.g.tiles_x, W.g.nt,
                        (int32_t*)nullptr, flag);
-    hipLaunchKernelGGL((ccl_select<OUT>), dim3(cdiv(W.g.nt, 4)), dim3(256), 0, s, W.B, forest, w, h, W.g.tiles_x, W.g.nt,
+    hipLaunchKernelGGL((ccl_select<OUT>), dim3(cdiv(W.g.nt, 4)), dim3(256), select_lds(W.B), s, W.B, forest, w, h, W.g.tiles_x, W.g.nt,
                        (const int32_t*)nullptr, 0, 0, flag, a, b, out, (int*)nullptr);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
@@ -846,12 +1028,12 @@ template <int MODE>
 int ccl_select_area(const Px& P, uint8_t* out, int w, int h, int lo, int hi, int conn, int* dcount, int32_t* forest,
                     int32_t* area, hipStream_t s) {
     CclWork W;
-    if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_NONE>(P, W, forest, w, h, area, nullptr, nullptr, dcount, s)));
-    else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_NONE>(P, W, forest, w, h, area, nullptr, nullptr, dcount, s)));
+    if (conn == 8) NSC_CHECK((ccl_forest_t<MODE, 8, SRC_NONE>(P, W, forest, w, h, area, lo, hi, nullptr, nullptr, dcount, s)));
+    else NSC_CHECK((ccl_forest_t<MODE, 4, SRC_NONE>(P, W, forest, w, h, area, lo, hi, nullptr, nullptr, dcount, s)));
     hipLaunchKernelGGL(ccl_roots, dim3(cdiv(W.g.nt, 4)), dim3(256), 0, s, W.B, forest, w, W.g.tiles_x, W.g.nt, area,
                        (uint8_t*)nullptr);
     const unsigned nb = dcount ? std::min<unsigned>(cdiv(W.g.nt, 4), kSelectBlocks) : cdiv(W.g.nt, 4);
-    hipLaunchKernelGGL((ccl_select<OUT_MASK>), dim3(nb), dim3(256), 0, s, W.B, forest, w, h, W.g.tiles_x, W.g.nt, area, lo, hi,
+    hipLaunchKernelGGL((ccl_select<OUT_MASK>), dim3(nb), dim3(256), select_lds(W.B), s, W.B, forest, w, h, W.g.tiles_x, W.g.nt, area, lo, hi,
                        (const uint8_t*)nullptr, (const uint8_t*)nullptr, (const uint8_t*)nullptr, out, dcount);
     NSC_HIP(hipGetLastError());
     return NSC_OK;
