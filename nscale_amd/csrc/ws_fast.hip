@@ -288,6 +288,8 @@ __global__ __launch_bounds__(1024) void k_sum_partials(const int* __restrict__ p
 
 // ---- phase 1: the flood of one run ----
 // in global memory, by one lane, for runs whose frame exceeds the LDS tiers
+// (MANY: with the plane of pop indexes beyond the records'; the kernel of the others is 4 % slower with its code)
+template <bool MANY>
 __device__ void flood_global(const Dev& D, const int32_t* __restrict__ box5, int nrun, int r, int* __restrict__ qh,
                              int* __restrict__ qt) {
     const int W = D.W;
@@ -329,8 +331,8 @@ __device__ void flood_global(const Dev& D, const int32_t* __restrict__ box5, int
         const int nx = D.qnext[x];
         head[active] = nx;
         if (nx < 0) tail[active] = -1;
-        D.wr[x].z |= min(popc, D.popcap);
-        if (D.popx && popc >= D.popcap) D.popx[x] = popc;
+        D.wr[x].z |= MANY ? min(popc, D.popcap) : popc;
+        if (MANY && popc >= D.popcap) D.popx[x] = popc;
         ++popc;
         if (x >= D.N) continue;  // a leaf: when it pops, nothing else
         const int p = x;
@@ -750,6 +752,7 @@ struct LdsPool {
     }
 };
 
+template <bool MANY>
 __global__ __launch_bounds__(64 * P1_WAVES) void k_phase1(Dev D, const int32_t* __restrict__ box5, int nrun,
                                                           const int* __restrict__ lists, const int* __restrict__ counts,
                                                           int* __restrict__ next_run, int* __restrict__ qh, int* __restrict__ qt) {
@@ -777,7 +780,7 @@ __global__ __launch_bounds__(64 * P1_WAVES) void k_phase1(Dev D, const int32_t* 
         }
         if (r < 0) break;
         if (tier == kRunTiers - 1) {
-            if (lane == 0) flood_global(D, box5, nrun, r, qh, qt);
+            if (lane == 0) flood_global<MANY>(D, box5, nrun, r, qh, qt);
         } else {
             const int L = uni(run_frame(box5, nrun, r));
             const int n = 1 + (L + 63) / 64;  // 102 at most: the pool holds it once the floods in flight are done
@@ -1993,7 +1996,10 @@ int cvws_fast(const uint8_t* img, const int32_t* m0, int32_t* m, int W, int H, i
         }
         // four runs a workgroup (one per SIMD) before a further CU is taken whole
         const int g = std::max(1, std::min((int)cdiv(nrun, 4), device_cus()));
-        hipLaunchKernelGGL(k_phase1, dim3(g), dim3(64 * P1_WAVES), 0, s, D, box5, nrun, lists, bcount, &small[40], qh2, qt);
+        if (D.popx)
+            hipLaunchKernelGGL(k_phase1<true>, dim3(g), dim3(64 * P1_WAVES), 0, s, D, box5, nrun, lists, bcount, &small[40], qh2, qt);
+        else
+            hipLaunchKernelGGL(k_phase1<false>, dim3(g), dim3(64 * P1_WAVES), 0, s, D, box5, nrun, lists, bcount, &small[40], qh2, qt);
     }
     // B pixels with a queue entry: initially queued ones, then those with leaves (the phase-1
     // queue links are dead from here on and hold the list)
