@@ -66,6 +66,7 @@ __global__ __launch_bounds__(E_THREADS) void k_edt_tiles(const uint64_t* __restr
                                                       uint16_t* __restrict__ above, uint16_t* __restrict__ below) {
     __shared__ uint16_t G[SEG][E_WIDE];
     const int sg = blockIdx.y, y0 = sg * SEG, x0 = blockIdx.x * E_COLS;
+    int row = -1;
     if (threadIdx.x < E_WIDE) {
         const int x = x0 - E_HALO + (int)threadIdx.x;
         // all three words from clamped (always valid) addresses; what lies outside the image holds no zero
@@ -94,7 +95,6 @@ __global__ __launch_bounds__(E_THREADS) void k_edt_tiles(const uint64_t* __restr
         const bool up = threadIdx.x < 192;  // wave-uniform
         const int x = x0 + (int)(threadIdx.x & 63), step = up ? -1 : 1, n = up ? sg : nseg - 1 - sg;
         const uint64_t* const col = zm + min(x, w - 1);
-        int row = -1;
         // the next segment's word, which nearly always holds one, then eight words' loads at a time
         auto hit = [&](uint64_t q, int s) { return s * SEG + (up ? 63 - (int)__clzll((long long)q) : (int)__ffsll((long long)q) - 1); };
         if (n > 0)
@@ -107,9 +107,10 @@ __global__ __launch_bounds__(E_THREADS) void k_edt_tiles(const uint64_t* __restr
             for (int j = 0; j < 8; ++j)
                 if (row < 0 && q[j]) row = hit(q[j], sg + step * min(k0 + j, n));
         }
-        if (x < w) (up ? above : below)[(size_t)sg * w + x] = row < 0 ? NONE : (uint16_t)row;
     }
     __syncthreads();
+    if (threadIdx.x >= E_WIDE && x0 + (int)(threadIdx.x & 63) < w)  // (a store the barrier need not wait for)
+        (threadIdx.x < 192 ? above : below)[(size_t)sg * w + x0 + (threadIdx.x & 63)] = row < 0 ? NONE : (uint16_t)row;
     constexpr int NP = E_COLS / 2, STEP = E_THREADS / NP, K = 4;  // pairs per row, rows per step
     const int c = 2 * ((int)threadIdx.x % NP), x = x0 + c;
     for (int yb = (int)threadIdx.x / NP; yb < SEG; yb += K * STEP) {
