@@ -154,7 +154,7 @@ struct CclBufs {
     uint16_t *off, *roots;
     uint16_t* edge_roots;  // [tile][4][64]
     void* edge;            // uint8_t or float, [tile][2][64]
-    int cap;               // run slots of a tile
+    int cap;               // run slots of a tile (a multiple of 8)
 };
 
 __device__ __forceinline__ int popc64(uint64_t v) { return (int)__popcll(v); }
@@ -944,11 +944,13 @@ CclGrid ccl_grid(int w, int h) {
     return CclGrid{tx, tx * (int)cdiv(h, CT)};
 }
 
-// scratch of a labelling: run slots for the most runs a tile can hold (every second pixel of a row, or
-// every pixel where equal values join)
-CclBufs ccl_carve(Carver& c, int nt, int mode) {
+// scratch of a labelling: run slots for the most runs that a tile of the image can hold (every second pixel of a
+// row, or every pixel where equal values join; kFewRuns at least, which the consumers load).  A tile of a
+// 64 x 64 image takes 5.8 KB or 10, of an image of one column 2.7.
+CclBufs ccl_carve(Carver& c, int nt, int mode, int w, int h) {
     CclBufs B;
-    B.cap = ccl_cap(mode);
+    const int cols = std::min(w, CT), most = std::min(h, CT) * (mode == FG_NEQ ? (cols + 1) / 2 : cols);
+    B.cap = std::max(kFewRuns, (most + 7) / 8 * 8);
     B.rows = c.take<RowWords>((size_t)nt * CT);
     B.off = c.take<uint16_t>((size_t)nt * CT);
     B.roots = c.take<uint16_t>((size_t)nt * B.cap);
@@ -978,10 +980,10 @@ int ccl_forest_t(const Px& P, CclWork& W, int32_t* forest, int w, int h, int32_t
                  const uint8_t* src, int* zero, hipStream_t s) {
     W.g = ccl_grid(w, h);
     Carver m(nullptr);
-    (void)ccl_carve(m, W.g.nt, MODE);
+    (void)ccl_carve(m, W.g.nt, MODE, w, h);
     NSC_CHECK(W.sc.alloc(m.size(), s));
     Carver c(W.sc.p);
-    W.B = ccl_carve(c, W.g.nt, MODE);
+    W.B = ccl_carve(c, W.g.nt, MODE, w, h);
     auto tiles = [&](auto waves) {
         constexpr int WAVES = decltype(waves)::value;
         hipLaunchKernelGGL((ccl_tile<MODE, CONN, SRC, WAVES>), dim3(W.g.nt), dim3(ccl_tile_threads(MODE, WAVES)), 0, s, P, W.B,
