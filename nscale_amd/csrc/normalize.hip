@@ -38,7 +38,9 @@ constexpr int kNormChunk = 4 * kNormThreads;  // pixels per work item (at most)
 // statistics partials (8 doubles each): two workgroups per CU, few enough that every workgroup of
 // k_norm_apply can sum them itself
 constexpr int kNormMaxBlocks = 512;
-constexpr int kApplyMaxBlocks = 1024;         // four workgroups of 15 KB of LDS per CU
+// three workgroups per CU, which its registers allow (20 KB of LDS each would allow eight); a fourth per CU ran
+// after them: 4096^2 white 66 us with 1024, 64 with 768, 512 x 3900 crop 36 and 35, H&E and noise alike
+constexpr int kApplyMaxBlocks = 768;
 
 struct NormConsts {
     float k3, k6, k2;  // 1/sqrtf(3), 1/sqrtf(6), 1/sqrtf(2) (Normalization.cpp:112-114, 172-174)
