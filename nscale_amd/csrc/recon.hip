@@ -185,10 +185,8 @@ struct WinMask {
 #pragma unroll
         for (int x = 0; x < TW; ++x) mr[x] = lm[lane][x];
     }
-    __device__ void opaque() {}
     __device__ __forceinline__ R clamp_col(R v, R n, int y) const { return clamp_up(v, n, mc[y]); }
     __device__ __forceinline__ R clamp_row(R v, R n, int x) const { return clamp_up(v, n, mr[x]); }
-    static __device__ __forceinline__ void fence(int) {}
 };
 // one round of the four direction sweeps over a window held in v (column state on entry and exit).
 // The down and up sweeps run as two interleaved chains, each updating v in place: step k moves the
@@ -201,7 +199,6 @@ template <typename T, int CONN>
 __device__ __forceinline__ void sweep_round(int32_t (&v)[TH], WinMask<T>& M, int32_t (*tr)[TW + 1],
                                             int lane) {
     using R = int32_t;
-    M.opaque();
     {
         R pd = v[0], pu = v[TH - 1];
 #pragma unroll
@@ -213,7 +210,6 @@ __device__ __forceinline__ void sweep_round(int32_t (&v)[TH], WinMask<T>& M, int
             const R nu = M.clamp_col(v[yu], (CONN == 8) ? nbr3(pu) : pu, yu);
             v[yu] = nu;
             pu = nu;
-            M.fence(yd);
         }
     }
     // ---- transpose to row state (lane = row) ----
@@ -222,7 +218,6 @@ __device__ __forceinline__ void sweep_round(int32_t (&v)[TH], WinMask<T>& M, int
     __syncthreads();
 #pragma unroll
     for (int x = 0; x < TW; ++x) v[x] = tr[lane][x];
-    M.opaque();
     {
         // with 8-connectivity the row sweeps take the diagonal neighbours too (the rows above and
         // below are the adjacent lanes), so a path that wanders by one row at a time while it runs
@@ -237,7 +232,6 @@ __device__ __forceinline__ void sweep_round(int32_t (&v)[TH], WinMask<T>& M, int
             const R nr = M.clamp_row(v[xr], (CONN == 8) ? nbr3(pr) : pr, xr);
             v[xr] = nr;
             pr = nr;
-            M.fence(xl);
         }
     }
 #pragma unroll

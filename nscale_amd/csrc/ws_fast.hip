@@ -8,8 +8,9 @@
 // Facts the decomposition rests on (each B-B colour difference is 0, every B-F difference is >0):
 //  1. Runs = 4-connected components of F.  Until the first pop of a B pixel that receives a
 //     positive label (call it b1, at time T1), runs do not interact: a B pixel popped as -1 changes
-//     nothing any other pixel reads.  Each run is flooded on its own lane ("phase 1"); B
-//     neighbours are recorded as leaf items (when, at what level and by whom they are queued).
+//     nothing any other pixel reads.  Each run is flooded by itself ("phase 1": by a wave in LDS, or by a
+//     lane in global memory where its frame is too large); B neighbours are recorded as leaf items (when,
+//     at what level and by whom they are queued).
 //  2. The global pop order of the merged runs is a total order computable from per-run data: for
 //     items x, y of different runs, x pops first iff the largest (level, push time) key on x's
 //     push chain is smaller than y's, comparing push times recursively through the pushers
@@ -19,7 +20,7 @@
 //     pixel not yet queued that it reaches (label Y1: such a pixel has no labelled F neighbour,
 //     which would have queued it) before anything else pops.
 //  4. After that, the unresolved pixels fall into 4-connected components that are again
-//     independent ("phase 2"), each flooded on its own lane from the queue state at T1.  The only
+//     independent ("phase 2"), each flooded by a lane, a larger one by a wave, from the queue state at T1.  The only
 //     order not known locally is the FIFO order among F pixels queued by the flood from b1 at the
 //     same level; for those the lane checks that every permutation gives the same labels.
 // Anything outside these assumptions (a capacity, a comparison that does not terminate, a tie
